@@ -1,6 +1,7 @@
 // Context, error reporting, device memory helpers and RNS NTT plans.
 #include <cstring>
 
+#include "fused.hpp"
 #include "host_math.hpp"
 #include "internal.hpp"
 
@@ -88,6 +89,7 @@ int ckks_context_destroy(ckks_context *ctx) {
         hipFree(kv.second.inv);
         if (kv.second.rowf) hipFree(kv.second.rowf);
         if (kv.second.rowf_inv) hipFree(kv.second.rowf_inv);
+        if (kv.second.zf) hipFree(kv.second.zf);
     }
     for (void *p : ctx->owned) hipFree(p);
     for (int i = 0; i < 2 * ckks_context::kSlots; ++i)
@@ -330,6 +332,16 @@ int ckks_rns_plan_create(ckks_context *ctx, const uint64_t *moduli, size_t n_lim
                 CK_HIP(hipMemcpy(tt.rowf, rf.data(), rb, hipMemcpyHostToDevice));
                 CK_HIP(hipMemcpy(tt.rowf_inv, rfi.data(), rb, hipMemcpyHostToDevice));
             }
+            if (logn > 12) {
+                // row products of both directions, gathered from the tables
+                const bool fp = q < host::kFpModulusBound;
+                const size_t zb = degree * (fp ? sizeof(double) : sizeof(Tw));
+                CK_HIP(hipMalloc(&tt.zf, 2 * zb));
+                tt.zi = (char *)tt.zf + zb;
+                int rc = build_row_products(ctx->stream, tt.fwd, q, fp, logn, tt.zf);
+                if (!rc) rc = build_row_products(ctx->stream, tt.inv, q, fp, logn, tt.zi);
+                if (rc) return rc;
+            }
             it = ctx->tables.emplace(key, tt).first;
         }
         DevPrime p{};
@@ -338,6 +350,8 @@ int ckks_rns_plan_create(ckks_context *ctx, const uint64_t *moduli, size_t n_lim
         p.inv = it->second.inv;
         p.rowf = it->second.rowf;
         p.rowf_inv = it->second.rowf_inv;
+        p.zf = it->second.zf;
+        p.zi = it->second.zi;
         p.ninv = host::invmod(degree % q, q);
         p.ninv_q = host::shoup_quotient(p.ninv, q);
         host::barrett(q, p.br_hi, p.br_lo);

@@ -1,0 +1,571 @@
+// Fused NTT passes (gfx950): column passes that read a key switch's digits in
+// the form it has them, and row passes that do its pointwise work between the
+// forward and the inverse transform of one tile, so NTT-domain data never
+// reaches HBM.  The tiles are in col_tile.hpp and row_tile.hpp.
+#include "host_math.hpp"
+#include "fused.hpp"
+#include "ntt_pass.hpp"
+#include "col_tile.hpp"
+
+namespace ck {
+
+// ---- row products -------------------------------------------------------------
+
+// psi^e for e < N is T[bitrev(e)], psi^(N + e) = -psi^e; the Shoup quotient of
+// q - w is 2^64 - 1 - floor(w 2^64 / q) (w 2^64 / q is no integer).
+__global__ __launch_bounds__(256) void k_row_products(const Tw *table, u64 q, u32 fp, u32 logn, void *out) {
+    const u32 x = blockIdx.x * 256 + threadIdx.x, N = 1u << logn;
+    if (x >= N) return;
+    const u32 n2 = ntt_n2(logn), n1 = logn - n2;
+    const u32 u = bitrev(x >> n2, n1), t = x & ((1u << n2) - 1);
+    const u32 e = ((2 * u + 1) * t) & (2 * N - 1);
+    const Tw w = table[bitrev(e & (N - 1), logn)];
+    if (fp) {
+        const double d = u64_as_f64(w.w);
+        ((double *)out)[x] = e >= N ? (double)q - d : d;
+    } else {
+        ((Tw *)out)[x] = e >= N ? Tw{q - w.w, ~w.wq} : w;
+    }
+}
+
+int build_row_products(hipStream_t s, const Tw *table, u64 q, bool fp, u32 logn, void *out) {
+    const u32 N = 1u << logn;
+    hipLaunchKernelGGL(k_row_products, dim3(N / 256), dim3(256), 0, s, table, q, fp ? 1u : 0u, logn, out);
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
+}
+
+bool fused_rows_apply(const ckks_rns_plan *plan) {
+    if (plan->logn < 13 || plan->logn > 17) return false;
+    for (u64 q : plan->moduli)
+        if (q >= kLazyModulusBound) return false;
+    return true;
+}
+
+// Loads at a uniform pointer plus a 32-bit byte offset per lane: one register
+// of address per lane instead of a 64-bit pointer per load.
+__device__ __forceinline__ u64 load_at(const u64 *base, u32 byte_off) {
+    return *(const u64 *)((const char *)base + byte_off);
+}
+__device__ __forceinline__ u64 load_once_at(const u64 *base, u32 byte_off) {
+    return ld_stream((const u64 *)((const char *)base + byte_off));
+}
+__device__ __forceinline__ void store_once_at(u64 *base, u32 byte_off, u64 v) {
+    st_stream((u64 *)((char *)base + byte_off), v);
+}
+__device__ __forceinline__ double load_z(const double *base, u32 off) {
+    return *(const double *)((const char *)base + off * 8);
+}
+__device__ __forceinline__ Tw load_z(const Tw *base, u32 off) { return *(const Tw *)((const char *)base + off * 16); }
+typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u64x2 load2_at(const u64 *base, u32 byte_off) {
+    return *(const u64x2 *)((const char *)base + byte_off);
+}
+
+// ---- column passes --------------------------------------------------------------
+
+// One entry of a launch.  The inter-pass side is limb-major: limb transform
+// limb * n_polys + poly.
+struct ColEntry {
+    const u64 *src;
+    u64 *dst;
+    const DevPrime *primes;
+    u64 stride;       // elements between polynomials on the coefficient side
+    u32 n_polys, n_limbs, logn, block_start;
+    u32 kind, digits;  // ColKind; polynomials per ciphertext (lifts)
+    u64 limit;         // digits: 2^(w-1)
+};
+
+constexpr int kMaxColEntries = 16;
+
+struct ColLaunch {
+    ColEntry e[kMaxColEntries];
+    u32 n;
+};
+
+// Input of limb prime P, largest bounds after it (see RowFp, RowInt):
+//   plain: canonical residues;
+//   residue: canonical modulo another prime of the plan (`limit`);
+//   digit: a balanced digit, |d| <= limit <= 2^62.
+// FP64 limbs take values up to 2^44 whole (with eight stages of 0.52 q they
+// stay below 2^45) and cut larger ones at bit 30; integer limbs take residues
+// up to 4q whole, add q to negative digits when limit < q, and reduce the rest
+// (below 2^64) into 3q.  Which of them is the same for a whole block.
+constexpr int kColFpIn = 16, kColIntIn = 4;
+constexpr u64 kColFpWhole = 1ull << 44;
+
+template <int K1>
+__device__ __forceinline__ void col_read(u64 (&v)[16], const u64 *src, u32 n2, u32 tile, u32 tid, u32 kind) {
+    typedef ColTile<K1> C;
+    const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
+    if (kind == kColPlain) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = load_once_at(src + C::template step<0>(n2, i), o0);
+    } else {
+        // read once per target limb: not streamed
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = load_at(src + C::template step<0>(n2, i), o0);
+    }
+}
+
+// 2^52 + 2^51 + d in the mantissa: exact for |d| < 2^51
+__device__ __forceinline__ double signed_to_f64(u64 d) {
+    return u64_as_f64(d + 0x4338000000000000ull) - 6755399441055744.0;
+}
+
+__device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, const RowFp &ar, const CK_CONST_AS DevPrime &) {
+    if (kind == kColPlain || limit <= kColFpWhole) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = f64_as_u64(signed_to_f64(v[i]));
+        return;
+    }
+    const double k30 = fp_reduce(1073741824.0, ar.q, ar.qinv);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const double hi = signed_to_f64((u64)((int64_t)v[i] >> 30)), lo = (double)(u32)(v[i] & 0x3fffffffu);
+        v[i] = f64_as_u64(lo + fp_mulmod_q(hi, k30, ar.q, ar.qinv));
+        if ((i & 3) == 3) sched_fence();
+    }
+}
+__device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, const RowInt &ar, const CK_CONST_AS DevPrime &P) {
+    if (kind == kColDigit && limit < ar.q) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] += (int64_t)v[i] < 0 ? ar.q : 0;
+    } else if (kind == kColDigit || (kind == kColResidue && limit > 4 * ar.q)) {
+        // a multiple of q from limit to limit + 2q makes every digit positive
+        const u64 up = kind == kColDigit ? (mulhi64(limit, P.br_hi) + 2) * ar.q : 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            v[i] = shoup_lazy3(v[i] + up, 1, P.br_hi, ar.q);
+            if ((i & 3) == 3) sched_fence();
+        }
+    }
+}
+
+template <int K1, class Ar>
+__device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS DevPrime &P, const Ar &ar, u32 limb,
+                                            u32 poly, u32 tile, u64 *lds) {
+    typedef ColTile<K1> C;
+    const u32 tid = threadIdx.x, n2 = e.logn - K1;
+    const u64 N = (u64)1 << e.logn;
+    const u64 *src;
+    u64 limit = 0;
+    if (e.kind == kColPlain) {
+        src = e.src + poly * e.stride + limb * N;
+    } else {
+        // digit j of ciphertext ct, shared by every limb
+        const u32 ct = poly / e.digits, j = poly % e.digits;
+        src = e.src + ct * e.stride + j * N;
+        limit = e.kind == kColResidue ? const_table(e.primes)[j].q : e.limit;
+    }
+    u64 v[16];
+    int b[16];
+    col_read<K1>(v, src, n2, tile, tid, e.kind);
+    col_lift(v, e.kind, limit, ar, P);
+    C::set(b, Ar::kFp ? kColFpIn : kColIntIn);
+    C::template fwd<0>(v, b, tid, P.fwd, ar);
+    C::template put<0>(v, tid, lds);
+    __syncthreads();
+    C::template get<1>(v, tid, lds);
+    C::level(b);
+    C::template fwd<1>(v, b, tid, P.fwd, ar);
+    // on to the row pass: times psi^((2u+1) t)
+    u64 *dst = e.dst + ((u64)limb * e.n_polys + poly) * N;
+    const typename Ar::Z *z = (const typename Ar::Z *)P.zf;
+    const u32 o1 = C::template offset<1>(tile, n2, tid, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const u32 st = C::template step<1>(n2, i);
+        store_once_at(dst + st, o1 * 8, ar.times(v[i], load_z(z + st, o1)));
+        // a few row products in flight at a time
+        if ((i & 3) == 3) sched_fence();
+    }
+}
+
+template <int K1, class Ar>
+__device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS DevPrime &P, const Ar &ar, u32 limb,
+                                            u32 poly, u32 tile, u64 *lds) {
+    typedef ColTile<K1> C;
+    const u32 tid = threadIdx.x, n2 = e.logn - K1;
+    const u64 N = (u64)1 << e.logn;
+    const u64 *src = e.src + ((u64)limb * e.n_polys + poly) * N;
+    u64 *dst = e.dst + poly * e.stride + limb * N;
+    u64 v[16];
+    int b[16];
+    const typename Ar::Z *z = (const typename Ar::Z *)P.zi;
+    const u32 o1 = C::template offset<1>(tile, n2, tid, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const u32 st = C::template step<1>(n2, i);
+        v[i] = load_once_at(src + st, o1 * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        v[i] = ar.times(v[i], load_z(z + C::template step<1>(n2, i), o1));
+        if (!Ar::kFp && (i & 3) == 3) sched_fence();
+    }
+    C::set(b, Ar::kZ);
+    C::template inv<1>(v, b, tid, P.inv, ar);
+    C::template put<1>(v, tid, lds);
+    __syncthreads();
+    C::template get<0>(v, tid, lds);
+    C::level(b);
+    C::template inv<0>(v, b, tid, P.inv, ar);
+    const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        u64 r;
+        if constexpr (Ar::kFp) {
+            r = fp_residue(fp_mulmod(u64_as_f64(v[i]), P.ninv_d, P.ninv_p, ar.q), ar.q, ar.qinv);
+        } else {
+            r = shoup(v[i], P.ninv, P.ninv_q, ar.q);
+        }
+        store_once_at(dst + C::template step<0>(n2, i), o0, r);
+        if (!Ar::kFp && (i & 3) == 3) sched_fence();
+    }
+}
+
+// Blocks of an entry.  Lifts: the limbs of one (polynomial, tile) follow each
+// other on one XCD, which reads the shared input once into its L2.  Plain and
+// inverse passes share nothing but the small twiddle tables: limb-major.
+template <bool FWD>
+__global__ __launch_bounds__(256, 5) void k_columns(ColLaunch l) {
+    __shared__ u64 lds[4096];
+    u32 di = 0;
+    while (di + 1 < l.n && blockIdx.x >= l.e[di + 1].block_start) ++di;
+    const ColEntry &e = l.e[di];
+    const u32 b = blockIdx.x - e.block_start, lt = e.logn - 12, tiles = 1u << lt;
+    u32 limb, poly, tile;
+    if (FWD && e.kind != kColPlain) {
+        const u32 k = b >> 3, group = k / e.n_limbs * 8 + (b & 7);
+        if (group >= e.n_polys * tiles) return;
+        limb = k % e.n_limbs;
+        poly = group >> lt;
+        tile = group & (tiles - 1);
+    } else {
+        tile = b & (tiles - 1);
+        poly = (b >> lt) % e.n_polys;
+        limb = (b >> lt) / e.n_polys;
+    }
+    const CK_CONST_AS DevPrime &P = const_table(e.primes)[limb];
+    const RowFp fp{P.qd, P.qinv};
+    const RowInt in{P.q};
+    switch (e.logn - ntt_n2(e.logn)) {
+#define CK_COL(K1)                                                            \
+    case K1:                                                                  \
+        if (FWD) {                                                            \
+            if (P.fp) col_forward<K1>(e, P, fp, limb, poly, tile, lds);       \
+            else col_forward<K1>(e, P, in, limb, poly, tile, lds);            \
+        } else {                                                              \
+            if (P.fp) col_inverse<K1>(e, P, fp, limb, poly, tile, lds);       \
+            else col_inverse<K1>(e, P, in, limb, poly, tile, lds);            \
+        }                                                                     \
+        break;
+        CK_COL(6)
+        CK_COL(7)
+        CK_COL(8)
+#undef CK_COL
+    }
+}
+
+int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward) {
+    if (count > (size_t)kMaxColEntries) return fail(CKKS_ERR_INVALID, "NTT batch holds at most 16 entries");
+    ColLaunch l{};
+    size_t blocks = 0;
+    for (size_t i = 0; i < count; ++i) {
+        const ColCall &c = calls[i];
+        if (c.n_polys == 0) continue;
+        if (!fused_rows_apply(c.plan)) return fail(CKKS_ERR_UNSUPPORTED, "column passes: two-pass degrees, primes below 2^60");
+        ColEntry e{};
+        e.src = c.in;
+        e.dst = c.out;
+        e.primes = c.plan->d_primes;
+        e.stride = c.stride;
+        e.n_polys = (u32)c.n_polys;
+        e.n_limbs = (u32)c.n_limbs;
+        e.logn = c.plan->logn;
+        e.block_start = (u32)blocks;
+        e.kind = (u32)c.kind;
+        e.digits = (u32)c.digits;
+        e.limit = c.limit;
+        l.e[l.n++] = e;
+        const size_t groups = c.n_polys << (e.logn - 12);
+        blocks += (forward && c.kind != kColPlain ? (groups + 7) / 8 * 8 : groups) * c.n_limbs;
+        if (blocks >= (1ull << 31)) return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
+        ckks_execution_profile &pc = ctx->counts();
+        (forward ? pc.ntt_forwards : pc.ntt_inverses) += c.n_polys;
+        pc.ntt_limb_transforms += c.n_polys * c.n_limbs;
+    }
+    if (!blocks) return CKKS_OK;
+    if (forward) hipLaunchKernelGGL(k_columns<true>, dim3((u32)blocks), dim3(256), 0, ctx->stream, l);
+    else hipLaunchKernelGGL(k_columns<false>, dim3((u32)blocks), dim3(256), 0, ctx->stream, l);
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
+}
+
+// ---- block order ----------------------------------------------------------------
+
+// Workgroups (limb, tile, ciphertext).  Integer limbs cost two to three times
+// an FP64 limb, so they are dealt first; blocks reach the 8 XCDs round-robin,
+// and group (limb, tile) g runs on XCD g mod 8 with its ciphertexts one after
+// another, so its key tile is read into one L2 and every XCD gets the same
+// share of heavy limbs.
+constexpr u32 kMaxOrder = 64;
+
+struct RowGrid {
+    u32 n_cts, limbs, logn, groups;
+    u32 xcd;  // 0: ciphertexts of a group on consecutive blocks
+    unsigned char order[kMaxOrder];
+};
+
+static RowGrid row_grid(const ckks_rns_plan *plan, size_t limbs, size_t n_cts, bool xcd) {
+    RowGrid g{};
+    g.n_cts = (u32)n_cts;
+    g.limbs = (u32)limbs;
+    g.logn = plan->logn;
+    g.groups = (u32)(limbs << (plan->logn - 12));
+    g.xcd = xcd ? 1u : 0u;
+    if (limbs <= kMaxOrder) {
+        u32 n = 0;
+        for (int heavy = 1; heavy >= 0; --heavy)
+            for (size_t i = 0; i < limbs; ++i)
+                if ((plan->h_primes[i].fp == 0) == (heavy == 1)) g.order[n++] = (unsigned char)i;
+    }
+    return g;
+}
+
+static u32 row_blocks(const RowGrid &g) { return g.xcd ? (g.groups + 7) / 8 * 8 * g.n_cts : g.groups * g.n_cts; }
+
+struct RowBlock {
+    u32 ct, limb, tile;
+    bool idle;
+};
+
+__device__ __forceinline__ RowBlock row_block(const RowGrid &g, u32 b) {
+    RowBlock r;
+    u32 group;
+    if (g.xcd) {
+        const u32 l = b >> 3;
+        group = l / g.n_cts * 8 + (b & 7);
+        r.ct = l % g.n_cts;
+    } else {
+        group = b / g.n_cts;
+        r.ct = b % g.n_cts;
+    }
+    r.idle = group >= g.groups;
+    const u32 lt = g.logn - 12, pos = group >> lt;
+    r.tile = group & ((1u << lt) - 1);
+    r.limb = r.idle ? 0 : g.limbs <= kMaxOrder ? g.order[pos] : pos;
+    return r;
+}
+
+// ---- key inner product ------------------------------------------------------------
+
+struct RowMacArgs {
+    const u64 *digits;   // [limb][ct][j][N], forward column pass output
+    const u64 *kb, *ka;  // [dnum][limbs][N]
+    u64 *out;            // [limb][ct][2][N], input of the inverse column pass
+    const DevPrime *primes;
+    RowGrid grid;
+    u32 dnum;
+};
+
+// A value the compiler cannot see through: index math that depends on it
+// stays inside the digit loop instead of being kept in registers across it.
+__device__ __forceinline__ u32 opaque(u32 x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x));
+#endif
+    return x;
+}
+
+// Two sums per residue, 64 bits each.
+//   FP64: products within 0.52 q, summed as doubles and reduced every 8 digits
+//     (below 2^45 throughout);
+//   integer: Montgomery products.  With T = d k for a digit d < 16 q < 2^64 and
+//     a canonical key entry k, m = T q^-1 mod 2^64 makes T - m q a multiple of
+//     2^64, so T_hi - (m q)_hi = T / 2^64 (mod q), in (-q, q).  Four of them and
+//     a reduced sum stay in (-4q, 7q), inside 63 bits; the factor 2^64 comes
+//     back with the last reduction, one product by 2^64 mod q.  (128-bit sums
+//     need no reduction per product but twice the registers.)
+struct SumFp {
+    static constexpr int kIn = 1;  // bound of total()
+    double q, qinv;
+    typedef double S;
+    __device__ __forceinline__ void mac(S &s, u64 y, u64 w) const {
+        s += fp_mulmod_q(u64_as_f64(y), small_to_f64(w), q, qinv);
+    }
+    __device__ __forceinline__ static bool full(u32 j) { return (j & 7) == 7; }
+    __device__ __forceinline__ S reduced(S s) const { return fp_reduce(s, q, qinv); }
+    __device__ __forceinline__ u64 total(S s) const { return f64_as_u64(fp_reduce(s, q, qinv)); }
+};
+struct SumInt {
+    static constexpr int kIn = 3;
+    u64 q, qi, r_hi, r_lo;  // modulus, q^-1 mod 2^64, floor(2^128 / q)
+    typedef u64 S;          // two's complement
+    __device__ __forceinline__ SumInt(const CK_CONST_AS DevPrime &P) : q(P.q), r_hi(P.br_hi), r_lo(P.br_lo) {
+        qi = q;  // q q == 1 mod 8; each step doubles the correct bits
+#pragma unroll
+        for (int it = 0; it < 5; ++it) qi *= 2 - q * qi;
+    }
+    __device__ __forceinline__ void mac(S &s, u64 y, u64 w) const {
+        const unsigned __int128 T = (unsigned __int128)y * w;
+        s += (u64)(T >> 64) - mulhi64((u64)T * qi, q);
+    }
+    __device__ __forceinline__ static bool full(u32 j) { return (j & 3) == 3; }
+    __device__ __forceinline__ S reduced(S s) const { return shoup_lazy3(s + 4 * q, 1, r_hi, q); }
+    __device__ __forceinline__ u64 total(S s) const { return shoup_lazy3(s + 4 * q, 0 - r_hi * q, r_lo, q); }
+};
+
+template <int L, class Ar, class Sum>
+struct RowMacBody {
+    typedef RowTile<L> R;
+    const RowMacArgs &a;
+    const CK_CONST_AS DevPrime &P;
+    const Ar ar;
+    const Sum sum;
+    u64 (*lds)[4096];
+    u32 tid;
+
+    // An exchange writes one of two LDS buffers and reads it after the barrier;
+    // the buffer's previous readers passed the other exchange's barrier in
+    // between, so one barrier per exchange is enough.
+    __device__ __forceinline__ void run(const RowBlock &blk) {
+        const u32 logn = a.grid.logn, n1 = logn - L;
+        const u64 N = (u64)1 << logn;
+        const u32 off0 = R::internal_off(blk.tile, n1, tid, 0) * 8;
+        const u32 nat0 = R::natural_off(blk.tile, n1, tid, 0) * 8;
+        const u32 D = a.dnum;
+        const u64 *src = a.digits + ((u64)blk.limb * a.grid.n_cts + blk.ct) * D * N;
+        const u64 *kb = a.kb + (u64)blk.limb * N, *ka = a.ka + (u64)blk.limb * N;
+        const u64 kstride = (u64)a.grid.limbs * N;
+        typename Sum::S sb[8], sa[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sb[i] = sa[i] = 0;
+        typename R::LowTw low;
+        u64 v[8], nx[8], wb[8], wa[8];
+        int b[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) nx[i] = load_at(src + (i << (L - 3)), off0);
+#pragma unroll 1
+        for (u32 j = 0;; ++j) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = nx[i];
+            R::set(b, Ar::kZ);
+            tid = opaque(tid);
+            // the key entries and the next digit are on their way while the
+            // stages run, each requested as late as registers allow
+            // (natural position of register i: rows bitrev(t) apart, the 2^EX
+            // columns of a thread adjacent and 16-byte aligned)
+            auto key = [&](u64 (&w)[8], const u64 *k) {
+#pragma unroll
+                for (int i = 0; i < 8; i += R::EX ? 2 : 1) {
+                    const u64 *at = k + (bitrev((u32)i >> R::EX, L) << n1) + (i & ((1 << R::EX) - 1));
+                    if constexpr (R::EX > 0) {
+                        const u64x2 p = load2_at(at, nat0);
+                        w[i] = p.x;
+                        w[i + 1] = p.y;
+                    } else {
+                        w[i] = load_at(at, nat0);
+                    }
+                }
+            };
+            key(wb, kb);
+            R::template fwd<0>(v, b, tid, P.fwd, low, ar);
+            R::template put<0>(v, tid, lds[0]);
+            src += N;
+            if (j + 1 < D) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) nx[i] = load_at(src + (i << (L - 3)), off0);
+            }
+            __syncthreads();
+            R::template get<1>(v, tid, lds[0]);
+            R::level(b);
+            R::template fwd<1>(v, b, tid, P.fwd, low, ar);
+            R::template put<1>(v, tid, lds[1]);
+            key(wa, ka);
+            low = R::low_twiddles(P.fwd, tid);
+            __syncthreads();
+            R::template get<2>(v, tid, lds[1]);
+            R::level(b);
+#pragma unroll
+            for (int x = 0; x < (1 << R::EX); ++x) {
+                R::fwd_group(v, b, x, low, ar);
+#pragma unroll
+                for (int i = x; i < 8; i += 1 << R::EX) {
+                    sum.mac(sb[i], v[i], wb[i]);
+                    sum.mac(sa[i], v[i], wa[i]);
+                }
+                sched_fence();
+            }
+            kb += kstride;
+            ka += kstride;
+            if (j + 1 == D) break;
+            if (Sum::full(j)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    sb[i] = sum.reduced(sb[i]);
+                    sa[i] = sum.reduced(sa[i]);
+                }
+            }
+        }
+        tid = opaque(tid);
+        low = R::low_twiddles(P.inv, tid);
+        u64 *out = a.out + ((u64)blk.limb * a.grid.n_cts + blk.ct) * 2 * N;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = sum.total(c ? sa[i] : sb[i]);
+            R::set(b, Sum::kIn);
+            R::template inv<2>(v, b, tid, P.inv, low, ar);
+            R::template put<2>(v, tid, lds[0]);
+            __syncthreads();
+            R::template get<1>(v, tid, lds[0]);
+            R::level(b);
+            R::template inv<1>(v, b, tid, P.inv, low, ar);
+            R::template put<1>(v, tid, lds[1]);
+            __syncthreads();
+            R::template get<0>(v, tid, lds[1]);
+            R::level(b);
+            R::template inv<0>(v, b, tid, P.inv, low, ar);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) *(u64 *)((char *)(out + c * N + (i << (L - 3))) + off0) = v[i];
+        }
+    }
+};
+
+template <int L>
+__global__ __launch_bounds__(512, 4) void k_row_mac(RowMacArgs a) {
+    __shared__ u64 lds[2][4096];
+    const RowBlock blk = row_block(a.grid, blockIdx.x);
+    if (blk.idle) return;
+    const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
+    if (P.fp)
+        RowMacBody<L, RowFp, SumFp>{a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, threadIdx.x}.run(blk);
+    else
+        RowMacBody<L, RowInt, SumInt>{a, P, RowInt{P.q}, SumInt(P), lds, threadIdx.x}.run(blk);
+}
+
+int launch_row_mac(ckks_context *ctx, const RowMac &m) {
+    if (!fused_rows_apply(m.plan)) return fail(CKKS_ERR_UNSUPPORTED, "fused row passes: 2^13 <= N <= 2^17, primes below 2^60");
+    RowMacArgs a{};
+    a.digits = m.digits;
+    a.kb = m.kb;
+    a.ka = m.ka;
+    a.out = m.out;
+    a.primes = m.plan->d_primes;
+    a.grid = row_grid(m.plan, m.limbs, m.n_cts, m.xcd_order);
+    a.dnum = (u32)m.dnum;
+    if ((u64)m.limbs * m.n_cts << (m.plan->logn - 12) >= (1ull << 30))
+        return fail(CKKS_ERR_INVALID, "key-switch batch too large for one launch");
+    const dim3 g(row_blocks(a.grid)), t(512);
+    switch (ntt_n2(m.plan->logn)) {
+        case 7: hipLaunchKernelGGL(k_row_mac<7>, g, t, 0, ctx->stream, a); break;
+        case 8: hipLaunchKernelGGL(k_row_mac<8>, g, t, 0, ctx->stream, a); break;
+        default: hipLaunchKernelGGL(k_row_mac<9>, g, t, 0, ctx->stream, a); break;
+    }
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
+}
+
+}  // namespace ck

@@ -1,0 +1,51 @@
+// Interface of the fused NTT passes (fused.hip).
+#pragma once
+#include "internal.hpp"
+
+namespace ck {
+
+// The passes serve two-pass degrees with primes below 2^60 (RowInt's lazy range): column passes
+// that read a key switch's digits in the form it has them, and row passes
+// that do the pointwise work between the forward and the inverse transform.
+bool fused_rows_apply(const ckks_rns_plan *plan);
+// Row products psi^((2u+1) t) of one prime's table into out (FP64 primes:
+// doubles, others: Tw), queued on s.
+int build_row_products(hipStream_t s, const Tw *table, u64 q, bool fp, u32 logn, void *out);
+
+// Input of a forward column pass.
+enum ColKind {
+    kColPlain = 0,    // polynomials [p][limb][N], canonical residues
+    kColResidue = 1,  // digit j of a ciphertext is its limb j ([ct][digits][N]), lifted to every limb
+    kColDigit = 2,    // balanced digits, int64 [ct][digits][N], |d| <= limit, lifted to every limb
+};
+// Forward: `in` (as kind says, `stride` elements between polynomials, lifts:
+// between ciphertexts) to inter-pass data in `out`.  Inverse: inter-pass data
+// `in` to polynomials in `out`, `stride` apart.  Inter-pass data is limb-major
+// ([limb][poly][N]), already multiplied (forward), not yet multiplied
+// (inverse) by the row products.
+struct ColCall {
+    const ckks_rns_plan *plan;
+    const u64 *in;
+    u64 *out;
+    size_t n_polys, n_limbs, stride;
+    int kind = kColPlain;
+    size_t digits = 1;  // polynomials per ciphertext (lifts)
+    u64 limit = 0;      // kColDigit
+};
+int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward);
+
+// Key inner product between the column passes of a key switch: the forward
+// row pass of the digits, the products with the key and the inverse row pass
+// of both sums.  digits: inter-pass, polynomials [ct][j]; out: inter-pass,
+// polynomials [ct][2].
+struct RowMac {
+    const ckks_rns_plan *plan;
+    const u64 *digits;
+    const u64 *kb, *ka;  // [dnum][limbs][N], NTT domain, natural order
+    u64 *out;
+    size_t n_cts, dnum, limbs;
+    bool xcd_order;  // ciphertexts of one key tile on one XCD
+};
+int launch_row_mac(ckks_context *ctx, const RowMac &m);
+
+}  // namespace ck

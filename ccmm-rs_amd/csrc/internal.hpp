@@ -22,6 +22,9 @@ struct DevPrime {
     // FP64 primes of a two-pass degree: row factors (row_factor_table_fp)
     // of the forward and inverse tables, null otherwise
     const Tw *rowf, *rowf_inv;
+    // two-pass degrees: psi^((2u+1) t) and its inverse at inter-pass position
+    // bitrev(u) N2 + t (row_tile.hpp); doubles for FP64 primes, Tw otherwise
+    const void *zf, *zi;
     u64 ninv, ninv_q;
     u64 br_hi, br_lo;  // floor(2^128 / q)
     double qd, qinv;      // FP64 path: q and 1/q
@@ -68,6 +71,7 @@ struct TwiddleTables {
     u32 logn;
     Tw *fwd = nullptr, *inv = nullptr;  // device
     Tw *rowf = nullptr, *rowf_inv = nullptr;
+    void *zf = nullptr, *zi = nullptr;  // one allocation, at zf
 };
 
 }  // namespace ck
@@ -189,12 +193,6 @@ int launch_ntt(ckks_context *ctx, const NttCall *calls, size_t count, bool forwa
 // device (looked up once per device, at context creation).
 int ntt_scratch_lookup(int device, u64 **out);
 int ntt_variant_for(const ckks_context *ctx, u32 logn);
-// Forward NTT of key-switch digits [ct][dnum][limbs][N] fused with the key
-// inner product into acc [ct][2][limbs][N] (two-pass degrees only).
-int launch_ntt_mac(ckks_context *ctx, const ckks_rns_plan *plan, const u64 *digits, size_t n_cts,
-                   size_t dnum, size_t limbs, const u64 *kb, const u64 *ka, u64 *acc,
-                   bool xcd_order);
-
 int check_plan_limbs(const ckks_rns_plan *plan, size_t n_limbs, const char *what);
 
 }  // namespace ck

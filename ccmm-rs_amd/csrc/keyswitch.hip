@@ -22,6 +22,7 @@
 
 #include "baseconv.hpp"
 #include "crt.hpp"
+#include "fused.hpp"
 #include "host_math.hpp"
 #include "internal.hpp"
 
@@ -101,7 +102,7 @@ struct ckks_ksk {
     unsigned base_log = 0, bounded_words = 0;
     ck::u64 *d_bounded = nullptr;  // table blob (BoundedTable points into it)
     int tuned_engine = CKKS_BASECONV_VALU;  // engine of CKKS_BASECONV_AUTO for this key
-    int tuned_fusion = CKKS_KS_FUSION_OFF;  // mode of CKKS_KS_FUSION_AUTO for this key
+    int tuned_fusion = CKKS_KS_FUSION_XCD;  // mode of CKKS_KS_FUSION_AUTO for this key (see ks_fused)
     int tuned_split = CKKS_KS_SPLIT_OFF;    // mode of CKKS_KS_SPLIT_AUTO for this key
     // hoisted rotations: key entries [2][D][B][N] permuted by k^-1, per k,
     // at most kHoistKeyCacheMax of them; hoist_lru lists the exponents most
@@ -477,6 +478,27 @@ static int launch_hoist(hipStream_t s, const HoistArgs &a) {
                        s, a);
     CK_HIP(hipGetLastError());
     return CKKS_OK;
+}
+
+// sigma_k of a component, limb by limb: out[ct][i][n] = +-in[i][g] (Gather),
+// the digits of single-limb blocks before their lift.
+struct RotateArgs {
+    const u64 *in;
+    u64 in_stride;
+    u64 *out;  // [ct][limbs][N]
+    const DevPrime *primes;
+    u64 kinv;
+    u32 limbs, logn;
+};
+
+__global__ __launch_bounds__(kKsThreads) void k_rotate(RotateArgs a) {
+    const u32 chunks = (1u << a.logn) / kKsThreads;
+    const u32 b = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const u32 row = b / chunks, i = row % a.limbs, ct = row / a.limbs;
+    const u64 N = (u64)1 << a.logn, n = (u64)(b % chunks) * kKsThreads + threadIdx.x;
+    const Gather g = galois_gather(n, a.kinv, a.logn);
+    const u64 v = a.in[ct * a.in_stride + i * N + g.idx];
+    a.out[(u64)row * N + n] = g.neg ? neg_mod(v, const_table(a.primes)[i].q) : v;
 }
 
 struct MacArgs {
@@ -1749,6 +1771,7 @@ struct KsJob {
     const HoistedMac *hm;
     u64 *digits, *acc, *mac_out;  // [ct][D][B][N] (or the hoisted digits), [ct][2][B][N], MAC output
     bool mfma;
+    bool raw;  // bounded digits: write the balanced digits [ct][D][N] themselves
 };
 
 static bool ks_uses_mfma(const ckks_ksk *k) {
@@ -1793,10 +1816,13 @@ static int ks_decompose(const KsJob &j, hipStream_t s) {
         ba.base_log = k->base_log;
         ba.small = digits_below_primes(plan, B, k->base_log);
         ba.total = (u64)j.n_cts * N;
+        // the fused column pass lifts the digits itself
+        if (j.raw) ba.raw = (int64_t *)j.digits;
         if (j.hoisted) {
             HoistArgs ha{};
             ha.digits = j.hoisted;
             ha.lifted = j.digits;
+            ha.raw = ba.raw;
             ha.primes = plan->d_primes;
             ha.kinv = j.galois_kinv;
             ha.limbs = (u32)B;
@@ -1967,6 +1993,85 @@ static bool hoisted_mac_fused(const ckks_context *ctx, u32 logn, size_t dnum) {
     return logn > 12 && logn <= 17 && dnum <= 8 && ctx->ks_fusion == CKKS_KS_FUSION_INVERSE;
 }
 
+// CKKS_KS_FUSION_XCD / LINEAR (XCD for an untuned key): the digits' forward
+// row pass, the key MAC and the inverse row pass of both sums run in one
+// kernel per tile (launch_row_mac), between the two column passes; neither
+// the NTT-domain digits nor the sums reach HBM.  Other degrees and primes
+// from 2^60 up take the separate kernels.
+static int ks_fusion(const ckks_ksk *k) {
+    const ckks_context *ctx = k->ctx;
+    return ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;
+}
+static bool ks_fused(const ckks_ksk *k) {
+    const int f = ks_fusion(k);
+    return (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && fused_rows_apply(k->plan);
+}
+
+// What a fused key switch hands its forward column pass: the digits of
+// single-limb blocks are the (rotated) input limbs themselves and bounded
+// digits one balanced integer per coefficient, both lifted to every limb as
+// the pass loads them; only larger blocks need their lift (ModUp) in HBM.
+static ColKind ks_lift(const ckks_ksk *k) {
+    if (k->bounded) return kColDigit;
+    for (size_t s : k->block_size)
+        if (s != 1) return kColPlain;
+    return kColResidue;
+}
+
+// Residues of the digit buffer per ciphertext.  Fused: the column pass's input
+// (see ks_lift), reused for the two sums the row passes write.
+static size_t ks_digit_residues(const ckks_ksk *k) {
+    const size_t full = k->dnum * k->limbs;
+    if (!ks_fused(k)) return full * k->degree;
+    return std::max(ks_lift(k) == kColPlain ? full : k->dnum, 2 * k->limbs) * k->degree;
+}
+
+// Steps 1 to 4 of the fused jobs: the digits in the form ks_lift names, their
+// column pass into `cols` (jobs one after another), fused row passes back into
+// the digit buffer, inverse column pass into the accumulators.
+static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t count, u64 *cols) {
+    std::vector<ColCall> fwd(count), inv(count);
+    u64 *c = cols;
+    int rc = CKKS_OK;
+    for (size_t i = 0; i < count && !rc; ++i) {
+        const KsJob &j = *jobs[i];
+        const ckks_ksk *k = j.k;
+        const size_t B = k->limbs, N = k->degree, D = k->dnum;
+        ColCall &f = fwd[i];
+        f = ColCall{k->plan, j.digits, c, j.n_cts * D, B, B * N, ks_lift(k)};
+        if (f.kind == kColResidue) {
+            f.digits = D;
+            if (j.galois_kinv) {
+                const RotateArgs ra{j.x, j.x_stride, j.digits, k->plan->d_primes, j.galois_kinv, (u32)D, k->plan->logn};
+                hipLaunchKernelGGL(k_rotate, dim3((u32)(j.n_cts * D * (N / kKsThreads))), dim3(kKsThreads), 0,
+                                   ctx->stream, ra);
+                CK_HIP(hipGetLastError());
+                f.stride = D * N;
+            } else {
+                f.in = j.x;
+                f.stride = j.x_stride;
+            }
+        } else {
+            if (f.kind == kColDigit) {
+                f.digits = D;
+                f.stride = D * N;
+                f.limit = (u64)1 << (k->base_log - 1);
+            }
+            rc = ks_decompose(j, ctx->stream);
+        }
+        inv[i] = ColCall{k->plan, j.digits, j.acc, j.n_cts * 2, B, B * N};
+        c += j.n_cts * D * B * N;
+    }
+    if (!rc) rc = launch_columns(ctx, fwd.data(), count, true);
+    for (size_t i = 0; i < count && !rc; ++i) {
+        const KsJob &j = *jobs[i];
+        const RowMac m{j.k->plan, fwd[i].out, j.k->d_kb, j.k->d_ka, j.digits, j.n_cts, j.k->dnum, j.k->limbs,
+                       ks_fusion(j.k) == CKKS_KS_FUSION_XCD};
+        rc = launch_row_mac(ctx, m);
+    }
+    return rc ? rc : launch_columns(ctx, inv.data(), count, false);
+}
+
 static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const u64 *add0,
                            const u64 *add1, u64 add_stride, u64 *out, u64 out_stride, size_t n_cts,
                            u64 galois_kinv, const int64_t *hoisted, const HoistedMac *hm) {
@@ -1982,7 +2087,7 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
     const bool two_pass = logn > 12 && logn <= 17;
     const bool hoist_fused = hm && !hm->bhat && hoisted_mac_fused(ctx, logn, D);
     // hoisted: slot 4 holds the unpermuted MAC output instead of the digits
-    const size_t slot4 = hm ? n_cts * 2 * B * N : n_cts * D * B * N;
+    const size_t slot4 = hm ? n_cts * 2 * B * N : n_cts * ks_digit_residues(k);
     if (!hoist_fused && (rc = ctx->workspace(4, slot4 * sizeof(u64), &wd))) return rc;
     if ((rc = ctx->workspace(5, n_cts * 2 * B * N * sizeof(u64), &wa))) return rc;
     KsJob j{k, x, x_stride, add0, add1, add_stride, out, out_stride, n_cts, galois_kinv, hoisted, hm};
@@ -1990,22 +2095,23 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
     j.acc = (u64 *)wa;
     j.mac_out = hm ? (u64 *)wd : j.acc;
     j.mfma = ks_uses_mfma(k);
+    j.raw = !hm && ks_fused(k);
+    if (!hm && ks_fused(k)) {
+        void *wc;
+        if ((rc = ctx->workspace(0, n_cts * D * B * N * sizeof(u64), &wc))) return rc;
+        const KsJob *jp = &j;
+        if ((rc = ks_fused_middle(ctx, &jp, 1, (u64 *)wc))) return rc;
+        return ks_moddown(j, s);
+    }
     // 1. ModUp
     if ((rc = ks_decompose(j, s))) return rc;
     // 2+3. forward NTT of every digit limb, key MAC
-    const int fusion = ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;
     // CKKS_KS_FUSION_INVERSE: the MAC is computed inside the first inverse
     // NTT pass (step 4) and the accumulators never reach HBM in the NTT domain
-    const bool mac_in_inverse = fusion == CKKS_KS_FUSION_INVERSE && two_pass && D <= 8 && !hm;
-    if ((fusion == CKKS_KS_FUSION_XCD || fusion == CKKS_KS_FUSION_LINEAR) && two_pass && !hm) {
-        if ((rc = launch_ntt_mac(ctx, plan, j.digits, n_cts, D, B, k->d_kb, k->d_ka, j.acc,
-                                 fusion == CKKS_KS_FUSION_XCD)))
-            return rc;
-    } else {
-        NttCall f{plan, j.digits, j.digits, n_cts * D, B, B * N, B * N};
-        if (!hm && (rc = launch_ntt(ctx, &f, 1, true))) return rc;
-        if (!mac_in_inverse && !hoist_fused && (rc = ks_mac(j, s))) return rc;
-    }
+    const bool mac_in_inverse = ks_fusion(k) == CKKS_KS_FUSION_INVERSE && two_pass && D <= 8 && !hm;
+    NttCall f{plan, j.digits, j.digits, n_cts * D, B, B * N, B * N};
+    if (!hm && (rc = launch_ntt(ctx, &f, 1, true))) return rc;
+    if (!mac_in_inverse && !hoist_fused && (rc = ks_mac(j, s))) return rc;
     // 4. inverse NTT of both accumulators.  Hoisted: the MAC runs over
     // sigma_k^-1-permuted keys; the inverse NTT reads its output permuted by
     // k, which is sum_j NTT(sigma_k(d_j)) * key_j
@@ -2022,9 +2128,9 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
 // of different ring degrees, levels and kinds may mix): every phase runs for
 // all entries before the next, and the forward and inverse NTTs of all
 // entries go out as one launch per pass (mixed degrees share the descriptor
-// table), so small batches ride in the big batches' launches.  Forward
-// row-pass fusion of the key MAC applies per entry (its key's mode); no
-// inverse-pass fusion, hoisting or stream split; at most 16 entries.
+// table), so small batches ride in the big batches' launches.  The fused
+// row passes apply per entry (ks_fused); no inverse-pass fusion, hoisting or
+// stream split; at most 16 entries.
 struct KsMultiEntry {
     const ckks_ksk *k;
     const u64 *x, *add0, *add1;
@@ -2039,7 +2145,7 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
     if (count > 16) return fail(CKKS_ERR_INVALID, "a key-switch batch holds at most 16 entries");
     size_t dig = 0, acc = 0;
     for (size_t i = 0; i < count; ++i) {
-        dig += e[i].n_cts * e[i].k->dnum * e[i].k->limbs * e[i].k->degree;
+        dig += e[i].n_cts * ks_digit_residues(e[i].k);
         acc += e[i].n_cts * 2 * e[i].k->limbs * e[i].k->degree;
         ckks_execution_profile &pc = ctx->counts();
         pc.key_switches += e[i].n_cts;
@@ -2063,37 +2169,36 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
         j.digits = pd;
         j.acc = j.mac_out = pa;
         j.mfma = ks_uses_mfma(k);
-        pd += e[i].n_cts * k->dnum * B * N;
+        j.raw = ks_fused(k);
+        pd += e[i].n_cts * ks_digit_residues(k);
         pa += e[i].n_cts * 2 * B * N;
         fwd[i] = NttCall{k->plan, j.digits, j.digits, e[i].n_cts * k->dnum, B, B * N, B * N};
         inv[i] = NttCall{k->plan, j.acc, j.acc, e[i].n_cts * 2, B, B * N, B * N};
-        if ((rc = ks_decompose(j, s))) return rc;
+        if (!ks_fused(k) && (rc = ks_decompose(j, s))) return rc;
     }
-    // entries whose key runs the MAC fused into the digits' forward row pass
-    // (tuned, or set on the context) take launch_ntt_mac; the others share
-    // one forward launch per pass
-    std::vector<char> fused(count, 0);
-    std::vector<NttCall> plain;
+    // fused entries (ks_fused) share one launch per column pass, the others
+    // one launch per pass of the whole transforms
+    std::vector<const KsJob *> fused;
+    std::vector<NttCall> plain, back;
+    size_t cols = 0;
     for (size_t i = 0; i < count; ++i) {
-        const ckks_ksk *k = e[i].k;
-        const int f = ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;
-        const u32 logn = k->plan->logn;
-        fused[i] = (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && logn > 12 && logn <= 17;
-        if (!fused[i]) plain.push_back(fwd[i]);
+        if (ks_fused(e[i].k)) {
+            fused.push_back(&jobs[i]);
+            cols += e[i].n_cts * e[i].k->dnum * e[i].k->limbs * e[i].k->degree;
+        } else {
+            plain.push_back(fwd[i]);
+            back.push_back(inv[i]);
+        }
+    }
+    if (!fused.empty()) {
+        void *wc;
+        if ((rc = ctx->workspace(0, cols * sizeof(u64), &wc))) return rc;
+        if ((rc = ks_fused_middle(ctx, fused.data(), fused.size(), (u64 *)wc))) return rc;
     }
     if ((rc = launch_ntt(ctx, plain.data(), plain.size(), true))) return rc;
-    for (size_t i = 0; i < count; ++i) {
-        const ckks_ksk *k = e[i].k;
-        if (!fused[i]) {
-            if ((rc = ks_mac(jobs[i], s))) return rc;
-            continue;
-        }
-        const int f = ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;
-        if ((rc = launch_ntt_mac(ctx, k->plan, jobs[i].digits, e[i].n_cts, k->dnum, k->limbs, k->d_kb, k->d_ka,
-                                 jobs[i].acc, f == CKKS_KS_FUSION_XCD)))
-            return rc;
-    }
-    if ((rc = launch_ntt(ctx, inv.data(), count, false))) return rc;
+    for (size_t i = 0; i < count; ++i)
+        if (!ks_fused(e[i].k) && (rc = ks_mac(jobs[i], s))) return rc;
+    if ((rc = launch_ntt(ctx, back.data(), back.size(), false))) return rc;
     for (size_t i = 0; i < count; ++i)
         if ((rc = ks_moddown(jobs[i], s))) return rc;
     return CKKS_OK;

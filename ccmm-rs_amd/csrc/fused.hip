@@ -64,6 +64,22 @@ __device__ __forceinline__ u64x2 load2_at(const u64 *base, u32 byte_off) {
 
 // ---- column passes --------------------------------------------------------------
 
+// Integer limbs cost two to three times an FP64 limb: they are spread evenly
+// among the others, one first, so that heavy and light blocks run side by
+// side.  Plans of more limbs run them in order.
+constexpr u32 kMaxOrder = 64;
+
+static void limb_order(const ckks_rns_plan *plan, size_t limbs, unsigned char *order) {
+    if (limbs > kMaxOrder) return;
+    std::vector<unsigned char> heavy, light;
+    for (size_t i = 0; i < limbs; ++i) (plan->h_primes[i].fp ? light : heavy).push_back((unsigned char)i);
+    size_t h = 0, l = 0;
+    for (size_t n = 0; n < limbs; ++n) {
+        const bool take = h < heavy.size() && (l >= light.size() || h * light.size() <= l * heavy.size());
+        order[n] = take ? heavy[h++] : light[l++];
+    }
+}
+
 // One entry of a launch.  The inter-pass side is limb-major: limb transform
 // limb * n_polys + poly.
 struct ColEntry {
@@ -74,6 +90,7 @@ struct ColEntry {
     u32 n_polys, n_limbs, logn, block_start;
     u32 kind, digits;  // ColKind; polynomials per ciphertext (lifts)
     u64 limit;         // digits: 2^(w-1)
+    unsigned char order[kMaxOrder];  // limb_order
 };
 
 constexpr int kMaxColEntries = 16;
@@ -165,20 +182,26 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
     C::set(b, Ar::kFp ? kColFpIn : kColIntIn);
     C::template fwd<0>(v, b, tid, P.fwd, ar);
     C::template put<0>(v, tid, lds);
-    __syncthreads();
-    C::template get<1>(v, tid, lds);
-    C::level(b);
-    C::template fwd<1>(v, b, tid, P.fwd, ar);
     // on to the row pass: times psi^((2u+1) t)
     u64 *dst = e.dst + ((u64)limb * e.n_polys + poly) * N;
     const typename Ar::Z *z = (const typename Ar::Z *)P.zf;
     const u32 o1 = C::template offset<1>(tile, n2, tid, 0);
+    typename Ar::Z zv[16];
+    if (Ar::kFp) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) zv[i] = load_z(z + C::template step<1>(n2, i), o1);
+    }
+    __syncthreads();
+    C::template get<1>(v, tid, lds);
+    C::level(b);
+    C::template fwd<1>(v, b, tid, P.fwd, ar);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const u32 st = C::template step<1>(n2, i);
-        store_once_at(dst + st, o1 * 8, ar.times(v[i], load_z(z + st, o1)));
-        // a few row products in flight at a time
-        if ((i & 3) == 3) sched_fence();
+        // 16-byte row products: a few in flight at a time
+        if (!Ar::kFp) zv[i] = load_z(z + st, o1);
+        store_once_at(dst + st, o1 * 8, ar.times(v[i], zv[i]));
+        if (!Ar::kFp && (i & 3) == 3) sched_fence();
     }
 }
 
@@ -227,7 +250,11 @@ __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS
 
 // Blocks of an entry.  Lifts: the limbs of one (polynomial, tile) follow each
 // other on one XCD, which reads the shared input once into its L2.  Plain and
-// inverse passes share nothing but the small twiddle tables: limb-major.
+// inverse passes take four limbs of every polynomial at a time: the four
+// limbs' row products stay in the XCDs' L2s over the batch (all limbs' do
+// not), and heavy limbs still run beside light ones.
+constexpr u32 kColGroup = 4;
+
 template <bool FWD>
 __global__ __launch_bounds__(256, 5) void k_columns(ColLaunch l) {
     __shared__ u64 lds[4096];
@@ -244,9 +271,13 @@ __global__ __launch_bounds__(256, 5) void k_columns(ColLaunch l) {
         tile = group & (tiles - 1);
     } else {
         tile = b & (tiles - 1);
-        poly = (b >> lt) % e.n_polys;
-        limb = (b >> lt) / e.n_polys;
+        const u32 x = b >> lt, per = kColGroup * e.n_polys, whole = e.n_limbs / kColGroup;
+        const u32 grp = x / per < whole ? x / per : whole;
+        const u32 width = grp < whole ? kColGroup : e.n_limbs % kColGroup, y = x - grp * per;
+        poly = y / width;
+        limb = grp * kColGroup + y % width;
     }
+    if (e.n_limbs <= kMaxOrder) limb = e.order[limb];
     const CK_CONST_AS DevPrime &P = const_table(e.primes)[limb];
     const RowFp fp{P.qd, P.qinv};
     const RowInt in{P.q};
@@ -288,6 +319,7 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
         e.kind = (u32)c.kind;
         e.digits = (u32)c.digits;
         e.limit = c.limit;
+        limb_order(c.plan, c.n_limbs, e.order);
         l.e[l.n++] = e;
         const size_t groups = c.n_polys << (e.logn - 12);
         blocks += (forward && c.kind != kColPlain ? (groups + 7) / 8 * 8 : groups) * c.n_limbs;
@@ -310,8 +342,6 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
 // and group (limb, tile) g runs on XCD g mod 8 with its ciphertexts one after
 // another, so its key tile is read into one L2 and every XCD gets the same
 // share of heavy limbs.
-constexpr u32 kMaxOrder = 64;
-
 struct RowGrid {
     u32 n_cts, limbs, logn, groups;
     u32 xcd;  // 0: ciphertexts of a group on consecutive blocks
@@ -325,12 +355,7 @@ static RowGrid row_grid(const ckks_rns_plan *plan, size_t limbs, size_t n_cts, b
     g.logn = plan->logn;
     g.groups = (u32)(limbs << (plan->logn - 12));
     g.xcd = xcd ? 1u : 0u;
-    if (limbs <= kMaxOrder) {
-        u32 n = 0;
-        for (int heavy = 1; heavy >= 0; --heavy)
-            for (size_t i = 0; i < limbs; ++i)
-                if ((plan->h_primes[i].fp == 0) == (heavy == 1)) g.order[n++] = (unsigned char)i;
-    }
+    limb_order(plan, limbs, g.order);
     return g;
 }
 
@@ -382,12 +407,13 @@ __device__ __forceinline__ u32 opaque(u32 x) {
 // Two sums per residue, 64 bits each.
 //   FP64: products within 0.52 q, summed as doubles and reduced every 8 digits
 //     (below 2^45 throughout);
-//   integer: Montgomery products.  With T = d k for a digit d < 16 q < 2^64 and
-//     a canonical key entry k, m = T q^-1 mod 2^64 makes T - m q a multiple of
-//     2^64, so T_hi - (m q)_hi = T / 2^64 (mod q), in (-q, q).  Four of them and
-//     a reduced sum stay in (-4q, 7q), inside 63 bits; the factor 2^64 comes
-//     back with the last reduction, one product by 2^64 mod q.  (128-bit sums
-//     need no reduction per product but twice the registers.)
+//   integer: Montgomery products, two 32-bit steps.  With T = d k for a digit
+//     d < 16 q < 2^64 and a canonical key entry k, T < 2^124, each step adds
+//     the multiple m q that clears the lowest word and drops it: T / 2^64
+//     (mod q) below 2q.  Four of them and a reduced sum stay below 11 q; the
+//     factor 2^64 comes back with the last reduction, one product by 2^64 mod
+//     q.  (128-bit sums need no reduction per product but twice the registers,
+//     which then spill.)
 struct SumFp {
     static constexpr int kIn = 1;  // bound of total()
     double q, qinv;
@@ -401,20 +427,28 @@ struct SumFp {
 };
 struct SumInt {
     static constexpr int kIn = 3;
-    u64 q, qi, r_hi, r_lo;  // modulus, q^-1 mod 2^64, floor(2^128 / q)
-    typedef u64 S;          // two's complement
+    u64 q, r_hi, r_lo;  // modulus, floor(2^128 / q)
+    u32 qi;             // -q^-1 mod 2^32
+    typedef u64 S;
     __device__ __forceinline__ SumInt(const CK_CONST_AS DevPrime &P) : q(P.q), r_hi(P.br_hi), r_lo(P.br_lo) {
-        qi = q;  // q q == 1 mod 8; each step doubles the correct bits
+        u32 x = (u32)q;  // q q == 1 mod 8; each step doubles the correct bits
 #pragma unroll
-        for (int it = 0; it < 5; ++it) qi *= 2 - q * qi;
+        for (int it = 0; it < 4; ++it) x *= 2u - (u32)q * x;
+        qi = 0u - x;
     }
     __device__ __forceinline__ void mac(S &s, u64 y, u64 w) const {
+        const u32 q0 = (u32)q, q1 = (u32)(q >> 32);
         const unsigned __int128 T = (unsigned __int128)y * w;
-        s += (u64)(T >> 64) - mulhi64((u64)T * qi, q);
+        const u32 m0 = (u32)T * qi;
+        const u64 c0 = (u64)m0 * q1 + (((u64)m0 * q0 + (u32)T) >> 32);
+        const unsigned __int128 U = (T >> 32) + c0;  // three words
+        const u32 m1 = (u32)U * qi;
+        const u64 c1 = (u64)m1 * q1 + (((u64)m1 * q0 + (u32)U) >> 32);
+        s += (u64)(U >> 32) + c1;
     }
     __device__ __forceinline__ static bool full(u32 j) { return (j & 3) == 3; }
-    __device__ __forceinline__ S reduced(S s) const { return shoup_lazy3(s + 4 * q, 1, r_hi, q); }
-    __device__ __forceinline__ u64 total(S s) const { return shoup_lazy3(s + 4 * q, 0 - r_hi * q, r_lo, q); }
+    __device__ __forceinline__ S reduced(S s) const { return shoup_lazy3(s, 1, r_hi, q); }
+    __device__ __forceinline__ u64 total(S s) const { return shoup_lazy3(s, 0 - r_hi * q, r_lo, q); }
 };
 
 template <int L, class Ar, class Sum>
@@ -424,7 +458,7 @@ struct RowMacBody {
     const CK_CONST_AS DevPrime &P;
     const Ar ar;
     const Sum sum;
-    u64 (*lds)[4096];
+    u64 (*lds)[RowTile<L>::LDS];
     u32 tid;
 
     // An exchange writes one of two LDS buffers and reads it after the barrier;
@@ -453,8 +487,6 @@ struct RowMacBody {
             for (int i = 0; i < 8; ++i) v[i] = nx[i];
             R::set(b, Ar::kZ);
             tid = opaque(tid);
-            // the key entries and the next digit are on their way while the
-            // stages run, each requested as late as registers allow
             // (natural position of register i: rows bitrev(t) apart, the 2^EX
             // columns of a thread adjacent and 16-byte aligned)
             auto key = [&](u64 (&w)[8], const u64 *k) {
@@ -470,14 +502,19 @@ struct RowMacBody {
                     }
                 }
             };
+            auto next = [&]() {
+                src += N;
+                if (j + 1 < D) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) nx[i] = load_at(src + (i << (L - 3)), off0);
+                }
+            };
+            // the key entries and the next digit are on their way while the
+            // stages run, each requested as late as registers allow
             key(wb, kb);
             R::template fwd<0>(v, b, tid, P.fwd, low, ar);
             R::template put<0>(v, tid, lds[0]);
-            src += N;
-            if (j + 1 < D) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) nx[i] = load_at(src + (i << (L - 3)), off0);
-            }
+            next();
             __syncthreads();
             R::template get<1>(v, tid, lds[0]);
             R::level(b);
@@ -495,6 +532,7 @@ struct RowMacBody {
                 for (int i = x; i < 8; i += 1 << R::EX) {
                     sum.mac(sb[i], v[i], wb[i]);
                     sum.mac(sa[i], v[i], wa[i]);
+                    if (!Ar::kFp) sched_fence();
                 }
                 sched_fence();
             }
@@ -536,7 +574,7 @@ struct RowMacBody {
 
 template <int L>
 __global__ __launch_bounds__(512, 4) void k_row_mac(RowMacArgs a) {
-    __shared__ u64 lds[2][4096];
+    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
     const RowBlock blk = row_block(a.grid, blockIdx.x);
     if (blk.idle) return;
     const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];

@@ -110,6 +110,15 @@ struct RowInt {
     static constexpr bool kFp = false;
     static constexpr int kMax = 16;  // bounds in units of q < 2^60
     u64 q;
+    // k q kept out of the compiler's sight: it would fold k q + x into two
+    // 64-bit multiply-adds where a uniform k q takes one addition
+    CK_HD u64 times_q(int k) const {
+        u64 m = q * (u64)k;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm("" : "+s"(m));
+#endif
+        return m;
+    }
     CK_HD static V from_bits(u64 x) { return x; }
     CK_HD static u64 to_bits(V x) { return x; }
     CK_HD V mul(V y, const Tw &w) const { return shoup_lazy3(y, w.w, w.wq, q); }
@@ -118,7 +127,7 @@ struct RowInt {
 #pragma unroll
         for (int s = 8; s >= 1; s >>= 1)
             if (b > target && b > s) {
-                const u64 sq = q * (u64)s;
+                const u64 sq = times_q(s);
                 x = x >= sq ? x - sq : x;
                 b = b - s > s ? b - s : s;
             }
@@ -135,21 +144,21 @@ struct RowInt {
         if (bx + 3 > kMax) reduce_to(x, bx, 8);
         const V a = x, t = mul(y, w);
         x = a + t;
-        y = a + 3 * q - t;
+        y = a + times_q(3) - t;
         bx = by = bx + 3;
     }
     CK_HD void ct1(V &x, V &y, int &bx, int &by) const {
         fit(x, y, bx, by);
         const V a = x, b = y;
         x = a + b;
-        y = a + (u64)by * q - b;
+        y = a + times_q(by) - b;
         bx = by = bx + by;
     }
     CK_HD void gs(V &x, V &y, const Tw &w, int &bx, int &by) const {
         fit(x, y, bx, by);
         const V a = x, b = y;
         x = a + b;
-        y = mul(a + (u64)by * q - b, w);
+        y = mul(a + times_q(by) - b, w);
         bx += by;
         by = 3;
     }
@@ -164,11 +173,11 @@ CK_HD void sched_fence() {
 #endif
 }
 
-// LDS placement: linear address (t << CL) | col with bits 0..4 XORed by
-// kRowSwizzle[k] for every set bit 5 + k.  The seven columns were searched so
-// that for L = 7, 8, 9 and each of the three geometries the six lane bits of a
-// wave, and its first five, map onto five independent low bits: 64 lanes of
-// 8 bytes touch each 8-byte bank slot exactly twice.
+// LDS placement of the column tile: linear address (t << CL) | col with bits
+// 0..4 XORed by kRowSwizzle[k] for every set bit 5 + k: no padding, so five
+// 32 KiB tiles fit a CU.  The seven columns were searched so that in every
+// geometry the six lane bits of a wave, and its first five, map onto five
+// independent low bits: 64 lanes of 8 bytes touch each 8-byte slot twice.
 constexpr u32 kRowSwizzle[7] = {31, 17, 26, 22, 5, 21, 30};
 
 CK_HD u32 row_swizzle(u32 a) {
@@ -185,6 +194,11 @@ CK_HD u32 row_swizzle(u32 a) {
 // of t, so the twiddles of stages 3..5 are wave-uniform), C the low L - 6
 // bits of t and the low 9 - L columns (lanes walk columns, so the natural
 // positions bitrev(t) N1 + u of a wave are whole 128-byte runs).
+// two adjacent residues, 16-byte aligned in LDS
+struct alignas(16) Pair {
+    u64 x, y;
+};
+
 template <int L>
 struct RowTile {
     static constexpr int CL = 12 - L, KC = L - 6, EX = 3 - KC;
@@ -201,22 +215,45 @@ struct RowTile {
         if (geo == 1) return (tid & 63u) >> KC;
         return ((tid & ((1u << (CL - EX)) - 1)) << EX) | ((u32)i & ((1u << EX) - 1));
     }
-    // the swizzle is linear over disjoint bits: thread part ^ register part
+    // LDS placement: slot a + 2 (a >> 4) of linear address a = (t << CL) | col.
+    // Additive over disjoint bits, so register i is the thread's address plus
+    // a constant the instruction carries as its offset; 64 lanes of 8 bytes
+    // touch an 8-byte slot two to four times (two is the least), geometry C's
+    // 16-byte accesses each slot four times (the least).
+    static constexpr int LDS = 4096 + 2 * 256;
+    CK_HD static u32 slot(u32 a) { return a + 2 * (a >> 4); }
     CK_HD static u32 lds_at(int geo, u32 tid, int i) {
-        const u32 a = row_swizzle((t_of(geo, tid, 0) << CL) | col_of(geo, tid, 0)) ^
-                      row_swizzle((t_of(geo, 0, i) << CL) | col_of(geo, 0, i));
-        CK_BOUNDS(a, 4096u);
+        const u32 a = slot((t_of(geo, tid, 0) << CL) | col_of(geo, tid, 0)) +
+                      slot((t_of(geo, 0, i) << CL) | col_of(geo, 0, i));
+        CK_BOUNDS(a, (u32)LDS);
         return a;
     }
     template <int GEO>
     CK_HD static void put(const u64 (&v)[8], u32 tid, u64 *lds) {
+        if constexpr (GEO == 2 && EX > 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) lds[lds_at(GEO, tid, i)] = v[i];
+            for (int i = 0; i < 8; i += 2) {
+                Pair p = {v[i], v[i + 1]};
+                *(Pair *)(lds + lds_at(GEO, tid, i)) = p;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) lds[lds_at(GEO, tid, i)] = v[i];
+        }
     }
     template <int GEO>
     CK_HD static void get(u64 (&v)[8], u32 tid, const u64 *lds) {
+        if constexpr (GEO == 2 && EX > 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = lds[lds_at(GEO, tid, i)];
+            for (int i = 0; i < 8; i += 2) {
+                const Pair p = *(const Pair *)(lds + lds_at(GEO, tid, i));
+                v[i] = p.x;
+                v[i + 1] = p.y;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = lds[lds_at(GEO, tid, i)];
+        }
     }
 
     // inter-pass offset of register i (geometry A): row m of column u
@@ -272,11 +309,13 @@ struct RowTile {
             const int bit = 1 << (lo + K - 1 - k);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (i & bit) continue;
-                if (GEO == 0 && (i >> (3 - k)) == 0)
-                    ar.ct1(v[i], v[i | bit], b[i], b[i | bit]);
-                else
-                    ar.ct(v[i], v[i | bit], twiddle<GEO>(tw, low, tid, i, k), b[i], b[i | bit]);
+                if (!(i & bit)) {
+                    if (GEO == 0 && (i >> (3 - k)) == 0)
+                        ar.ct1(v[i], v[i | bit], b[i], b[i | bit]);
+                    else
+                        ar.ct(v[i], v[i | bit], twiddle<GEO>(tw, low, tid, i, k), b[i], b[i | bit]);
+                }
+                if (!Ar::kFp && (i & 3) == 3) sched_fence();
             }
         }
 #pragma unroll
@@ -293,11 +332,13 @@ struct RowTile {
             const int bit = 1 << (lo + K - 1 - k);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (i & bit) continue;
-                if (GEO == 0 && (i >> (3 - k)) == 0)
-                    ar.gs1(v[i], v[i | bit], b[i], b[i | bit]);
-                else
-                    ar.gs(v[i], v[i | bit], twiddle<GEO>(tw, low, tid, i, k), b[i], b[i | bit]);
+                if (!(i & bit)) {
+                    if (GEO == 0 && (i >> (3 - k)) == 0)
+                        ar.gs1(v[i], v[i | bit], b[i], b[i | bit]);
+                    else
+                        ar.gs(v[i], v[i | bit], twiddle<GEO>(tw, low, tid, i, k), b[i], b[i | bit]);
+                }
+                if (!Ar::kFp && (i & 3) == 3) sched_fence();
             }
         }
         if (GEO != 0) {

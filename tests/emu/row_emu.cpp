@@ -55,7 +55,7 @@ void row_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward
     typedef RowTile<L> R;
     const u32 n1 = p.logn - L;
     static u64 v[512][8];
-    static u64 lds[4096];
+    alignas(16) static u64 lds[RowTile<L>::LDS];
     for (u32 tile = 0; tile < (1u << (p.logn - 12)); ++tile) {
         int b[8], bx[8];
         auto each = [&](auto &&f) {

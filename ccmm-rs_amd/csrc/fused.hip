@@ -4,6 +4,7 @@
 // reaches HBM.  The tiles are in col_tile.hpp and row_tile.hpp.
 #include "host_math.hpp"
 #include "fused.hpp"
+#include "fused_dev.hpp"
 #include "ntt_pass.hpp"
 #include "col_tile.hpp"
 
@@ -42,43 +43,7 @@ bool fused_rows_apply(const ckks_rns_plan *plan) {
     return true;
 }
 
-// Loads at a uniform pointer plus a 32-bit byte offset per lane: one register
-// of address per lane instead of a 64-bit pointer per load.
-__device__ __forceinline__ u64 load_at(const u64 *base, u32 byte_off) {
-    return *(const u64 *)((const char *)base + byte_off);
-}
-__device__ __forceinline__ u64 load_once_at(const u64 *base, u32 byte_off) {
-    return ld_stream((const u64 *)((const char *)base + byte_off));
-}
-__device__ __forceinline__ void store_once_at(u64 *base, u32 byte_off, u64 v) {
-    st_stream((u64 *)((char *)base + byte_off), v);
-}
-__device__ __forceinline__ double load_z(const double *base, u32 off) {
-    return *(const double *)((const char *)base + off * 8);
-}
-__device__ __forceinline__ Tw load_z(const Tw *base, u32 off) { return *(const Tw *)((const char *)base + off * 16); }
-typedef u64 u64x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ u64x2 load2_at(const u64 *base, u32 byte_off) {
-    return *(const u64x2 *)((const char *)base + byte_off);
-}
-
 // ---- column passes --------------------------------------------------------------
-
-// Integer limbs cost two to three times an FP64 limb: they are spread evenly
-// among the others, one first, so that heavy and light blocks run side by
-// side.  Plans of more limbs run them in order.
-constexpr u32 kMaxOrder = 64;
-
-static void limb_order(const ckks_rns_plan *plan, size_t limbs, unsigned char *order) {
-    if (limbs > kMaxOrder) return;
-    std::vector<unsigned char> heavy, light;
-    for (size_t i = 0; i < limbs; ++i) (plan->h_primes[i].fp ? light : heavy).push_back((unsigned char)i);
-    size_t h = 0, l = 0;
-    for (size_t n = 0; n < limbs; ++n) {
-        const bool take = h < heavy.size() && (l >= light.size() || h * light.size() <= l * heavy.size());
-        order[n] = take ? heavy[h++] : light[l++];
-    }
-}
 
 // One entry of a launch.  The inter-pass side is limb-major: limb transform
 // limb * n_polys + poly.
@@ -90,6 +55,7 @@ struct ColEntry {
     u32 n_polys, n_limbs, logn, block_start;
     u32 kind, digits;  // ColKind; polynomials per ciphertext (lifts)
     u64 limit;         // digits: 2^(w-1)
+    const ColBlock *blocks;
     unsigned char order[kMaxOrder];  // limb_order
 };
 
@@ -97,7 +63,7 @@ constexpr int kMaxColEntries = 16;
 
 struct ColLaunch {
     ColEntry e[kMaxColEntries];
-    u32 n;
+    u32 n, blocks;
 };
 
 // Input of limb prime P, largest bounds after it (see RowFp, RowInt):
@@ -108,6 +74,7 @@ struct ColLaunch {
 // stay below 2^45) and cut larger ones at bit 30; integer limbs take residues
 // up to 4q whole, add q to negative digits when limit < q, and reduce the rest
 // (below 2^64) into 3q.  Which of them is the same for a whole block.
+//   block: a mixed-radix value, see col_blocks; within 0.54 q or below 2q.
 constexpr int kColFpIn = 16, kColIntIn = 4;
 constexpr u64 kColFpWhole = 1ull << 44;
 
@@ -123,11 +90,6 @@ __device__ __forceinline__ void col_read(u64 (&v)[16], const u64 *src, u32 n2, u
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = load_at(src + C::template step<0>(n2, i), o0);
     }
-}
-
-// 2^52 + 2^51 + d in the mantissa: exact for |d| < 2^51
-__device__ __forceinline__ double signed_to_f64(u64 d) {
-    return u64_as_f64(d + 0x4338000000000000ull) - 6755399441055744.0;
 }
 
 __device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, const RowFp &ar, const CK_CONST_AS DevPrime &) {
@@ -160,14 +122,67 @@ __device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, cons
 }
 
 template <int K1, class Ar>
+__device__ __forceinline__ void col_blocks(u64 (&v)[16], const u64 *src, u64 N, const CK_CONST_AS ColBlock &blk,
+                                           u32 limb, u32 n2, u32 tile, u32 tid, const CK_CONST_AS DevPrime &P) {
+    typedef ColTile<K1> C;
+    typedef BlockSum<Ar::kFp> Sum;
+    constexpr int W = 8;  // residues summed at a time: what their partial sums leave room for
+    const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
+    const CK_CONST_AS u64 *row0 = const_table(blk.rows) + (u64)limb * kColTerms * 2;
+    const u32 first = blk.first, terms = blk.terms, split = blk.split;
+#pragma unroll
+    for (int g = 0; g < 16; g += W) {
+        Sum s[W];
+        u64 x[W];
+        const CK_CONST_AS u64 *row = row0;
+        const u64 *d = src + (u64)first * N;
+#pragma unroll
+        for (int i = 0; i < W; ++i) x[i] = load_at(d + C::template step<0>(n2, g + i), o0);
+        u32 t = 0;
+        if (split) {
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                s[i].add((x[i] & 0x3fffffffu) | kDigitBias, row[0], u64_as_f64(row[1]));
+                s[i].add((x[i] >> 30) | kDigitBias, row[2], u64_as_f64(row[3]));
+                if (i & 1) sched_fence();
+            }
+            t = 2;
+        } else {
+#pragma unroll
+            for (int i = 0; i < W; ++i) s[i].add(x[i] | kDigitBias, row[0], u64_as_f64(row[1]));
+            t = 1;
+        }
+#pragma unroll 1
+        for (row += 2 * t; t < terms; ++t, row += 2) {
+            d += N;
+#pragma unroll
+            for (int i = 0; i < W; ++i) x[i] = load_at(d + C::template step<0>(n2, g + i), o0);
+            const u64 w = row[0];
+            const double wp = u64_as_f64(row[1]);
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                s[i].add(x[i] | kDigitBias, w, wp);
+                if ((i & 3) == 3) sched_fence();
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            v[g + i] = s[i].value(P.q);
+            if (i & 1) sched_fence();
+        }
+    }
+}
+
+template <int K1, bool BLOCK, class Ar>
 __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS DevPrime &P, const Ar &ar, u32 limb,
                                             u32 poly, u32 tile, u64 *lds) {
     typedef ColTile<K1> C;
     const u32 tid = threadIdx.x, n2 = e.logn - K1;
     const u64 N = (u64)1 << e.logn;
-    const u64 *src;
+    const u64 *src = nullptr;
     u64 limit = 0;
-    if (e.kind == kColPlain) {
+    if (BLOCK) {
+    } else if (e.kind == kColPlain) {
         src = e.src + poly * e.stride + limb * N;
     } else {
         // digit j of ciphertext ct, shared by every limb
@@ -177,8 +192,13 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
     }
     u64 v[16];
     int b[16];
-    col_read<K1>(v, src, n2, tile, tid, e.kind);
-    col_lift(v, e.kind, limit, ar, P);
+    if (BLOCK) {
+        const u32 ct = poly / e.digits, j = poly % e.digits;
+        col_blocks<K1, Ar>(v, e.src + ct * e.stride, N, const_table(e.blocks)[j], limb, n2, tile, tid, P);
+    } else {
+        col_read<K1>(v, src, n2, tile, tid, e.kind);
+        col_lift(v, e.kind, limit, ar, P);
+    }
     C::set(b, Ar::kFp ? kColFpIn : kColIntIn);
     C::template fwd<0>(v, b, tid, P.fwd, ar);
     C::template put<0>(v, tid, lds);
@@ -255,15 +275,15 @@ __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS
 // not), and heavy limbs still run beside light ones.
 constexpr u32 kColGroup = 4;
 
-template <bool FWD>
-__global__ __launch_bounds__(256, 5) void k_columns(ColLaunch l) {
+template <bool FWD, bool BLOCK>
+__global__ __launch_bounds__(256, BLOCK ? 4 : 5) void k_columns(ColLaunch l) {
     __shared__ u64 lds[4096];
     u32 di = 0;
     while (di + 1 < l.n && blockIdx.x >= l.e[di + 1].block_start) ++di;
     const ColEntry &e = l.e[di];
     const u32 b = blockIdx.x - e.block_start, lt = e.logn - 12, tiles = 1u << lt;
     u32 limb, poly, tile;
-    if (FWD && e.kind != kColPlain) {
+    if (BLOCK || (FWD && e.kind != kColPlain)) {
         const u32 k = b >> 3, group = k / e.n_limbs * 8 + (b & 7);
         if (group >= e.n_polys * tiles) return;
         limb = k % e.n_limbs;
@@ -285,8 +305,8 @@ __global__ __launch_bounds__(256, 5) void k_columns(ColLaunch l) {
 #define CK_COL(K1)                                                            \
     case K1:                                                                  \
         if (FWD) {                                                            \
-            if (P.fp) col_forward<K1>(e, P, fp, limb, poly, tile, lds);       \
-            else col_forward<K1>(e, P, in, limb, poly, tile, lds);            \
+            if (P.fp) col_forward<K1, BLOCK>(e, P, fp, limb, poly, tile, lds);       \
+            else col_forward<K1, BLOCK>(e, P, in, limb, poly, tile, lds);            \
         } else {                                                              \
             if (P.fp) col_inverse<K1>(e, P, fp, limb, poly, tile, lds);       \
             else col_inverse<K1>(e, P, in, limb, poly, tile, lds);            \
@@ -301,10 +321,10 @@ __global__ __launch_bounds__(256, 5) void k_columns(ColLaunch l) {
 
 int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward) {
     if (count > (size_t)kMaxColEntries) return fail(CKKS_ERR_INVALID, "NTT batch holds at most 16 entries");
-    ColLaunch l{};
-    size_t blocks = 0;
+    ColLaunch l{}, lb{};  // lb: kColBlock entries
     for (size_t i = 0; i < count; ++i) {
         const ColCall &c = calls[i];
+        ColLaunch &to = forward && c.kind == kColBlock ? lb : l;
         if (c.n_polys == 0) continue;
         if (!fused_rows_apply(c.plan)) return fail(CKKS_ERR_UNSUPPORTED, "column passes: two-pass degrees, primes below 2^60");
         ColEntry e{};
@@ -315,22 +335,28 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
         e.n_polys = (u32)c.n_polys;
         e.n_limbs = (u32)c.n_limbs;
         e.logn = c.plan->logn;
-        e.block_start = (u32)blocks;
+        e.block_start = to.blocks;
         e.kind = (u32)c.kind;
         e.digits = (u32)c.digits;
         e.limit = c.limit;
+        e.blocks = c.blocks;
         limb_order(c.plan, c.n_limbs, e.order);
-        l.e[l.n++] = e;
+        to.e[to.n++] = e;
         const size_t groups = c.n_polys << (e.logn - 12);
-        blocks += (forward && c.kind != kColPlain ? (groups + 7) / 8 * 8 : groups) * c.n_limbs;
+        const size_t blocks = to.blocks + (forward && c.kind != kColPlain ? (groups + 7) / 8 * 8 : groups) * c.n_limbs;
+        to.blocks = (u32)blocks;
         if (blocks >= (1ull << 31)) return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
         ckks_execution_profile &pc = ctx->counts();
         (forward ? pc.ntt_forwards : pc.ntt_inverses) += c.n_polys;
         pc.ntt_limb_transforms += c.n_polys * c.n_limbs;
     }
-    if (!blocks) return CKKS_OK;
-    if (forward) hipLaunchKernelGGL(k_columns<true>, dim3((u32)blocks), dim3(256), 0, ctx->stream, l);
-    else hipLaunchKernelGGL(k_columns<false>, dim3((u32)blocks), dim3(256), 0, ctx->stream, l);
+    // blocks of both kinds (forward): one launch each
+    if (!forward) {
+        if (l.blocks) hipLaunchKernelGGL((k_columns<false, false>), dim3(l.blocks), dim3(256), 0, ctx->stream, l);
+    } else {
+        if (l.blocks) hipLaunchKernelGGL((k_columns<true, false>), dim3(l.blocks), dim3(256), 0, ctx->stream, l);
+        if (lb.blocks) hipLaunchKernelGGL((k_columns<true, true>), dim3(lb.blocks), dim3(256), 0, ctx->stream, lb);
+    }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
 }
@@ -394,15 +420,6 @@ struct RowMacArgs {
     RowGrid grid;
     u32 dnum;
 };
-
-// A value the compiler cannot see through: index math that depends on it
-// stays inside the digit loop instead of being kept in registers across it.
-__device__ __forceinline__ u32 opaque(u32 x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(x));
-#endif
-    return x;
-}
 
 // Two sums per residue, 64 bits each.
 //   FP64: products within 0.52 q, summed as doubles and reduced every 8 digits

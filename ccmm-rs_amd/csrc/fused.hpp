@@ -17,6 +17,17 @@ enum ColKind {
     kColPlain = 0,    // polynomials [p][limb][N], canonical residues
     kColResidue = 1,  // digit j of a ciphertext is its limb j ([ct][digits][N]), lifted to every limb
     kColDigit = 2,    // balanced digits, int64 [ct][digits][N], |d| <= limit, lifted to every limb
+    kColBlock = 3,    // digit j is given by its mixed-radix digits ([ct][.][N], see ColBlock)
+};
+// A gadget block as kColBlock evaluates it: the block's value is sum_t c_t W_t,
+// c_t < 2^41 the mixed-radix digits (limbs first .. of the ciphertext's data);
+// split: digit 0 is below 2^60 and enters as its low 30 bits (t = 0) and the
+// rest (t = 1, weight 2^30 W_0).  Row i of `rows` holds, per term, W_t mod q_i
+// and fl(that / q_i) as double bits.
+constexpr int kColTerms = 13;
+struct ColBlock {
+    u32 first, terms, split;
+    const u64 *rows;  // [limb][kColTerms][2]
 };
 // Forward: `in` (as kind says, `stride` elements between polynomials, lifts:
 // between ciphertexts) to inter-pass data in `out`.  Inverse: inter-pass data
@@ -31,6 +42,7 @@ struct ColCall {
     int kind = kColPlain;
     size_t digits = 1;  // polynomials per ciphertext (lifts)
     u64 limit = 0;      // kColDigit
+    const ColBlock *blocks = nullptr;  // kColBlock: one per digit, device memory
 };
 int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward);
 

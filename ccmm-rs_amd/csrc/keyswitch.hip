@@ -23,6 +23,7 @@
 #include "baseconv.hpp"
 #include "crt.hpp"
 #include "fused.hpp"
+#include "fused_dev.hpp"
 #include "host_math.hpp"
 #include "internal.hpp"
 
@@ -53,11 +54,10 @@ struct ModUpBlock {
     // other digit is below 2^41.
     // Garner row gf[k] (k >= 1, q_k < 2^41): q_k, 1/q_k, inv[k], fl(inv[k] / q_k),
     // pm[k][0] 2^30 mod q_k, its quotient, then (pm[k][m], fl(pm[k][m] / q_k))
-    // for m < k.  Target row tf + i * kFpRow (q_i < 2^41): q_i, 1/q_i,
-    // w_i0 2^30 mod q_i, its quotient, then (w_im, fl(w_im / q_i)) for m < size.
+    // for m < k.  Target weights: ColBlock's rows.
     u32 fp_mode;
     double gf[kMaxAlpha][kFpRow];
-    const double *tf;
+    const u64 *rows;
 };
 
 struct ModDownTable {
@@ -111,6 +111,9 @@ struct ckks_ksk {
     mutable std::vector<ck::u64> hoist_lru;
     ck::BcPlan *d_bc = nullptr;
     signed char *d_bt = nullptr;
+    // every block in an FP64 mode: the blocks as the fused column pass
+    // evaluates them (one per digit), null otherwise
+    ck::ColBlock *d_col = nullptr;
 };
 
 // Digits of a ciphertext batch's a components for hoisted bounded rotations:
@@ -187,12 +190,14 @@ __device__ __forceinline__ Barrett barrett_at(const CK_CONST_AS DevPrime *p, u32
 // Integer mode: Garner digits and every target by 128-bit accumulation and
 // Barrett reduction.
 //
-// FP64 modes (MODE = blk->fp_mode = 1 or 2): Garner digits c_k (k >= 1) and
-// the targets whose bit is set in a.fp_targets (q_i < 2^41) as sums of
-// fp_mulmod terms, each |term| <= 0.51 q, at most kMaxAlpha + 1 of them, so
-// every sum stays below 2^45 and is exact; fp_canon / fp_residue make it
-// canonical.  Digit 0 is x_0 itself: whole in mode 1 (first block prime below
-// 2^41), split at bit 30 in mode 2; the other digits are below 2^41.
+// FP64 modes (MODE = blk->fp_mode = 1 or 2): Garner digits c_k (k >= 1) as sums
+// of fp_mulmod terms, each |term| <= 0.51 q, at most kMaxAlpha + 1 of them, so
+// every sum stays below 2^45 and is exact; fp_canon makes it canonical.  Digit 0
+// is x_0 itself: whole in mode 1 (first block prime below 2^41), split at bit
+// 30 in mode 2; the other digits are below 2^41.  The targets are BlockSum's
+// sums: an FP64 quotient and the low bits of the remainder by integer products
+// (64 ciphertexts at N = 2^16, blocks of 9 and 8 limbs: 406 + 712 us with a
+// fp_mulmod per term).
 template <int A, int MODE>
 __device__ void modup_thread(const ModUpArgs &a, const CK_CONST_AS ModUpBlock *blk, u32 ct, u32 j, u64 n) {
     const u64 N = (u64)1 << a.logn;
@@ -258,28 +263,36 @@ __device__ void modup_thread(const ModUpArgs &a, const CK_CONST_AS ModUpBlock *b
         for (int m = 1; m < k; ++m) t -= fp_mulmod(cl[m], g[6 + 2 * m], g[7 + 2 * m], q);
         cl[k] = fp_canon(fp_mulmod(t, g[2], g[3], q), q, g[1]);
     }
-    const CK_CONST_AS double *tf = const_table(blk->tf);
+    // the digits as biased doubles (BlockSum)
+    u64 d[A];
+    const u64 d0 = (x[0] & 0x3fffffffull) | kDigitBias, d1 = (x[0] >> 30) | kDigitBias;
+#pragma unroll
+    for (int m = 0; m < A; ++m) d[m] = m == 0 ? x[0] | kDigitBias : f64_as_u64(cl[m] + 4503599627370496.0);
     const u64 fpm = a.fp_targets;
-    for (u32 i = 0; i < a.limbs; ++i) {
+    const CK_CONST_AS u64 *row = const_table(blk->rows);
+    for (u32 i = 0; i < a.limbs; ++i, row += 2 * kColTerms) {
         if (i - start < (u32)A) continue;  // block limbs are stored above
+        const u64 q = primes[i].q;
+        auto sum = [&](auto s) {
+            const CK_CONST_AS u64 *r = row;
+            if (SPLIT0) {
+                s.add(d0, r[0], u64_as_f64(r[1]));
+                s.add(d1, r[2], u64_as_f64(r[3]));
+                r += 2;
+            } else {
+                s.add(d[0], r[0], u64_as_f64(r[1]));
+            }
+#pragma unroll
+            for (int m = 1; m < A; ++m) s.add(d[m], r[2 * m], u64_as_f64(r[2 * m + 1]));
+            return s.value(q);
+        };
         u64 v;
         if (i < 64 && ((fpm >> i) & 1)) {  // the mask is empty for bases over 64 limbs
-            const CK_CONST_AS double *r = tf + (u64)i * kFpRow;
-            const double q = r[0];
-            double acc = fp_mulmod(cl[0], r[4], r[5], q);
-            if (SPLIT0) acc += fp_mulmod(ch0, r[2], r[3], q);
-#pragma unroll
-            for (int m = 1; m < A; ++m) acc += fp_mulmod(cl[m], r[4 + 2 * m], r[5 + 2 * m], q);
-            v = fp_residue(acc, q, r[1]);
+            const double r = u64_as_f64(sum(BlockSum<true>{}));  // |r| < 0.54 q
+            v = f64_to_small(r < 0.0 ? r + primes[i].qd : r);
         } else {
-            const Barrett bi = barrett_at(primes, i);
-            const CK_CONST_AS u64 *w = wt + (u64)i * kMaxAlpha;
-            Acc128 t;
-            t.zero();
-            t.mac(x[0], w[0]);
-#pragma unroll
-            for (int m = 1; m < A; ++m) t.mac(f64_to_small(cl[m]), w[m]);
-            v = t.reduce(bi);
+            v = sum(BlockSum<false>{});  // below 1.6 q
+            v = v >= q ? v - q : v;
         }
         st_stream(dst + (u64)i * N, v);
     }
@@ -296,6 +309,65 @@ __global__ __launch_bounds__(kKsThreads) void k_modup(ModUpArgs a, u32 j_first, 
     const u32 j = j_first + cj % n_j, ct = cj / n_j;
     const u64 n = (u64)chunk * kKsThreads + threadIdx.x;
     modup_thread<A, MODE>(a, const_table(a.blocks) + j, ct, j, n);
+}
+
+// The mixed-radix digits alone, [ct][q_limbs][N] in the block's limb order: what
+// the fused column pass evaluates at every limb (kColBlock).  Same digits as
+// modup_thread's FP64 modes; one launch for blocks of every size up to AMAX.
+struct GarnerArgs {
+    const u64 *in;  // as ModUpArgs
+    u64 in_stride, kinv;
+    u64 *out;       // [ct][q_limbs][N]
+    const ModUpBlock *blocks;
+    const DevPrime *primes;
+    u32 dnum, q_limbs, logn, chunks;
+};
+
+template <int A>
+__device__ __forceinline__ void garner_thread(const GarnerArgs &a, const CK_CONST_AS ModUpBlock *blk, u32 ct, u64 n) {
+    const u64 N = (u64)1 << a.logn;
+    const CK_CONST_AS DevPrime *primes = const_table(a.primes);
+    const u32 start = blk->start;
+    const Gather gi = galois_gather(n, a.kinv, a.logn);
+    const u64 *src = a.in + ct * a.in_stride + (u64)start * N + gi.idx;
+    u64 *dst = a.out + ((u64)ct * a.q_limbs + start) * N + n;
+    u64 x[A];
+#pragma unroll
+    for (int m = 0; m < A; ++m) {
+        const u64 v = src[(u64)m * N];
+        x[m] = gi.neg ? neg_mod(v, primes[start + m].q) : v;
+    }
+    dst[0] = x[0];
+    if (A == 1) return;
+    // digit 0 cut at bit 30 whether or not its prime needs it (mode 2)
+    const double ch0 = small_to_f64(x[0] >> 30);
+    double cl[A];
+    cl[0] = small_to_f64(x[0] & 0x3fffffffull);
+#pragma unroll
+    for (int k = 1; k < A; ++k) {
+        const CK_CONST_AS double *g = blk->gf[k];
+        const double q = g[0];
+        double t = small_to_f64(x[k]) - fp_mulmod(cl[0], g[6], g[7], q) - fp_mulmod(ch0, g[4], g[5], q);
+#pragma unroll
+        for (int m = 1; m < k; ++m) t -= fp_mulmod(cl[m], g[6 + 2 * m], g[7 + 2 * m], q);
+        cl[k] = fp_canon(fp_mulmod(t, g[2], g[3], q), q, g[1]);
+        dst[(u64)k * N] = f64_to_small(cl[k]);
+    }
+}
+
+template <int AMAX>
+__global__ __launch_bounds__(kKsThreads) void k_garner(GarnerArgs a) {
+    const u32 b = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const u32 chunk = b % a.chunks, cj = b / a.chunks, j = cj % a.dnum, ct = cj / a.dnum;
+    const u64 n = (u64)chunk * kKsThreads + threadIdx.x;
+    const CK_CONST_AS ModUpBlock *blk = const_table(a.blocks) + j;
+    switch (blk->size) {
+#define CK_GA(A) \
+    case A: if constexpr (A <= AMAX) garner_thread<A>(a, blk, ct, n); break;
+        CK_GA(1) CK_GA(2) CK_GA(3) CK_GA(4) CK_GA(5) CK_GA(6)
+        CK_GA(7) CK_GA(8) CK_GA(9) CK_GA(10) CK_GA(11) CK_GA(12)
+#undef CK_GA
+    }
 }
 
 // sizes / fp: per digit, its block size and its mode (0 integer, 1 / 2 FP64).
@@ -1505,20 +1577,32 @@ static int create_key(const ckks_rns_plan *plan, size_t q_limbs, const size_t *b
     size_t md_w_off = consts.size();
     ModDownTable md{};
     if (hybrid) build_moddown(mods, q_limbs, consts, md);
-    // FP64 ModUp target rows of every block (ModUpBlock::tf)
-    const size_t tf_off = consts.size();
+    // the weights of FP64-mode blocks at every limb (ColBlock): integers with
+    // their quotients, digit 0 of a prime from 2^41 up in two terms (cut at
+    // bit 30)
+    bool col_ok = true;
+    std::vector<ColBlock> cols;
+    const size_t col_off = consts.size();
     for (size_t j = 0; j < n_blocks; ++j) {
+        ColBlock cb{};
+        cb.first = (u32)k->block_start[j];
+        cb.split = k->block_fp[j] == 2 ? 1 : 0;
+        cb.terms = (u32)block_sizes[j] + cb.split;
+        cols.push_back(cb);
+        col_ok = col_ok && k->block_fp[j] != 0;
         for (size_t i = 0; i < B; ++i) {
             const size_t row0 = consts.size();
             const u64 q = mods[i];
-            if (k->block_fp[j] && fp_prime(q)) {
-                const u64 w0 = consts[(j * B + i) * kMaxAlpha];
-                consts.push_back(double_bits((double)q));
-                consts.push_back(double_bits(1.0 / (double)q));
-                push_fp_pair(consts, host::mulmod(w0, (1ull << 30) % q, q), q);
-                for (size_t m = 0; m < block_sizes[j]; ++m) push_fp_pair(consts, consts[(j * B + i) * kMaxAlpha + m], q);
+            auto term = [&](u64 w) {
+                consts.push_back(w);
+                consts.push_back(double_bits((double)w / (double)q));
+            };
+            for (size_t m = 0; m < block_sizes[j] && k->block_fp[j]; ++m) {
+                const u64 w = consts[(j * B + i) * kMaxAlpha + m];
+                term(w);
+                if (m == 0 && cb.split) term(host::mulmod(w, (1ull << 30) % q, q));
             }
-            consts.resize(row0 + kFpRow, 0);
+            consts.resize(row0 + 2 * kColTerms, 0);
         }
     }
     k->fp_targets = fp_target_mask(mods, B);
@@ -1527,7 +1611,12 @@ static int create_key(const ckks_rns_plan *plan, size_t q_limbs, const size_t *b
     CK_HIP(hipMemcpy(k->d_consts, consts.data(), consts.size() * sizeof(u64), hipMemcpyHostToDevice));
     for (size_t j = 0; j < n_blocks; ++j) {
         k->h_modup[j].w = k->d_consts + j * B * kMaxAlpha;
-        k->h_modup[j].tf = (const double *)(k->d_consts + tf_off) + j * B * kFpRow;
+        k->h_modup[j].rows = k->d_consts + col_off + j * B * 2 * kColTerms;
+    }
+    if (col_ok) {
+        for (size_t j = 0; j < n_blocks; ++j) cols[j].rows = k->h_modup[j].rows;
+        CK_HIP(hipMalloc(&k->d_col, n_blocks * sizeof(ColBlock)));
+        CK_HIP(hipMemcpy(k->d_col, cols.data(), n_blocks * sizeof(ColBlock), hipMemcpyHostToDevice));
     }
     CK_HIP(hipMalloc(&k->d_modup, n_blocks * sizeof(ModUpBlock)));
     CK_HIP(hipMemcpy(k->d_modup, k->h_modup.data(), n_blocks * sizeof(ModUpBlock), hipMemcpyHostToDevice));
@@ -2007,23 +2096,57 @@ static bool ks_fused(const ckks_ksk *k) {
     return (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && fused_rows_apply(k->plan);
 }
 
-// What a fused key switch hands its forward column pass: the digits of
-// single-limb blocks are the (rotated) input limbs themselves and bounded
-// digits one balanced integer per coefficient, both lifted to every limb as
-// the pass loads them; only larger blocks need their lift (ModUp) in HBM.
-static ColKind ks_lift(const ckks_ksk *k) {
+// What a fused key switch of n_cts ciphertexts hands its forward column pass:
+// the digits of single-limb blocks are the (rotated) input limbs themselves,
+// bounded digits one balanced integer per coefficient, larger blocks their
+// mixed-radix digits (as many as the block has limbs); the pass lifts each of
+// them to every limb as it loads.
+//
+// Lifting in HBM (ModUp) remains for blocks with integer Garner digits (a
+// second prime from 2^41 up), for the matrix-core engine, and where it is
+// faster: evaluating a block costs the column pass as many L2 reads per
+// residue as the block has limbs, against one write and one read of the lifted
+// residue.  Blocks of 9 and 8 limbs at N = 2^16: 174 against 194 us for one
+// ciphertext, 889 / 887 us for 8 (402 MB lifted), 7213 / 6227 us for 64.
+// Blocks of 5 and 4 at N = 2^15: 77 / 92 us for one, 1528 / 1611 us for 64; of 4
+// at N = 2^14 the same order throughout.  Around the line, 64 ciphertexts at
+// N = 2^16: blocks of 6 and 6 limbs 2887 / 2779 us; 32 ciphertexts with five
+// blocks of 5 limbs 3721 / 3764 us.
+constexpr size_t kLiftInHbmBlock = 6;             // limbs of the largest block ..
+constexpr size_t kLiftInHbmBytes = 256ull << 20;  // .. and lifted bytes from which ModUp wins
+static ColKind ks_lift(const ckks_ksk *k, size_t n_cts) {
     if (k->bounded) return kColDigit;
-    for (size_t s : k->block_size)
-        if (s != 1) return kColPlain;
-    return kColResidue;
+    size_t most = 0;
+    for (size_t s : k->block_size) most = std::max(most, s);
+    if (most == 1) return kColResidue;
+    if (!k->d_col || ks_uses_mfma(k)) return kColPlain;
+    const size_t lifted = n_cts * k->dnum * k->limbs * k->degree * sizeof(u64);
+    return most >= kLiftInHbmBlock && lifted > kLiftInHbmBytes ? kColPlain : kColBlock;
+}
+
+static int launch_garner(const ckks_ksk *k, const u64 *in, u64 in_stride, u64 kinv, u64 *out, size_t n_cts,
+                         hipStream_t s) {
+    const u32 chunks = (u32)(k->degree / kKsThreads);
+    const GarnerArgs a{in, in_stride, kinv, out, k->d_modup, k->plan->d_primes, (u32)k->dnum, (u32)k->q_limbs,
+                       k->plan->logn, chunks};
+    size_t most = 0;
+    for (size_t z : k->block_size) most = std::max(most, z);
+    const dim3 g((u32)(n_cts * k->dnum * chunks)), t(kKsThreads);
+    if (most <= 4) hipLaunchKernelGGL(k_garner<4>, g, t, 0, s, a);
+    else if (most <= 9) hipLaunchKernelGGL(k_garner<9>, g, t, 0, s, a);
+    else hipLaunchKernelGGL(k_garner<12>, g, t, 0, s, a);
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
 }
 
 // Residues of the digit buffer per ciphertext.  Fused: the column pass's input
 // (see ks_lift), reused for the two sums the row passes write.
-static size_t ks_digit_residues(const ckks_ksk *k) {
+static size_t ks_digit_residues(const ckks_ksk *k, size_t n_cts) {
     const size_t full = k->dnum * k->limbs;
     if (!ks_fused(k)) return full * k->degree;
-    return std::max(ks_lift(k) == kColPlain ? full : k->dnum, 2 * k->limbs) * k->degree;
+    const ColKind lift = ks_lift(k, n_cts);
+    const size_t in = lift == kColPlain ? full : lift == kColBlock ? k->q_limbs : k->dnum;
+    return std::max(in, 2 * k->limbs) * k->degree;
 }
 
 // Steps 1 to 4 of the fused jobs: the digits in the form ks_lift names, their
@@ -2038,7 +2161,7 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
         const ckks_ksk *k = j.k;
         const size_t B = k->limbs, N = k->degree, D = k->dnum;
         ColCall &f = fwd[i];
-        f = ColCall{k->plan, j.digits, c, j.n_cts * D, B, B * N, ks_lift(k)};
+        f = ColCall{k->plan, j.digits, c, j.n_cts * D, B, B * N, ks_lift(k, j.n_cts)};
         if (f.kind == kColResidue) {
             f.digits = D;
             if (j.galois_kinv) {
@@ -2051,6 +2174,11 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
                 f.in = j.x;
                 f.stride = j.x_stride;
             }
+        } else if (f.kind == kColBlock) {
+            f.digits = D;
+            f.stride = k->q_limbs * N;
+            f.blocks = k->d_col;
+            rc = launch_garner(k, j.x, j.x_stride, j.galois_kinv, j.digits, j.n_cts, ctx->stream);
         } else {
             if (f.kind == kColDigit) {
                 f.digits = D;
@@ -2087,7 +2215,7 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
     const bool two_pass = logn > 12 && logn <= 17;
     const bool hoist_fused = hm && !hm->bhat && hoisted_mac_fused(ctx, logn, D);
     // hoisted: slot 4 holds the unpermuted MAC output instead of the digits
-    const size_t slot4 = hm ? n_cts * 2 * B * N : n_cts * ks_digit_residues(k);
+    const size_t slot4 = hm ? n_cts * 2 * B * N : n_cts * ks_digit_residues(k, n_cts);
     if (!hoist_fused && (rc = ctx->workspace(4, slot4 * sizeof(u64), &wd))) return rc;
     if ((rc = ctx->workspace(5, n_cts * 2 * B * N * sizeof(u64), &wa))) return rc;
     KsJob j{k, x, x_stride, add0, add1, add_stride, out, out_stride, n_cts, galois_kinv, hoisted, hm};
@@ -2145,7 +2273,7 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
     if (count > 16) return fail(CKKS_ERR_INVALID, "a key-switch batch holds at most 16 entries");
     size_t dig = 0, acc = 0;
     for (size_t i = 0; i < count; ++i) {
-        dig += e[i].n_cts * ks_digit_residues(e[i].k);
+        dig += e[i].n_cts * ks_digit_residues(e[i].k, e[i].n_cts);
         acc += e[i].n_cts * 2 * e[i].k->limbs * e[i].k->degree;
         ckks_execution_profile &pc = ctx->counts();
         pc.key_switches += e[i].n_cts;
@@ -2170,7 +2298,7 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
         j.acc = j.mac_out = pa;
         j.mfma = ks_uses_mfma(k);
         j.raw = ks_fused(k);
-        pd += e[i].n_cts * ks_digit_residues(k);
+        pd += e[i].n_cts * ks_digit_residues(k, e[i].n_cts);
         pa += e[i].n_cts * 2 * B * N;
         fwd[i] = NttCall{k->plan, j.digits, j.digits, e[i].n_cts * k->dnum, B, B * N, B * N};
         inv[i] = NttCall{k->plan, j.acc, j.acc, e[i].n_cts * 2, B, B * N, B * N};
@@ -2420,6 +2548,7 @@ int ckks_ksk_destroy(ckks_ksk *k) {
     hipFree(k->d_bc);
     hipFree(k->d_bt);
     hipFree(k->d_bounded);
+    hipFree(k->d_col);
     delete k;
     return CKKS_OK;
 }

@@ -37,16 +37,13 @@ __global__ __launch_bounds__(256) void k_encode_round(EncodeArgs a) {
         r = 0;
     }
     const int64_t v = (int64_t)r;
+    const u64 mag = v < 0 ? 0 - (u64)v : (u64)v;
     u64 *o = a.out + p * (u64)a.n_limbs * N + n;
     for (u32 i = 0; i < a.n_limbs; ++i) {
-        const u64 q = a.primes[i].q;
-        u64 res;
-        if (v >= 0) {
-            res = (u64)v % q;
-        } else {
-            const u64 mag = ((u64)(-(v + 1)) + 1) % q;
-            res = mag ? q - mag : 0;
-        }
+        const DevPrime &P = a.primes[i];
+        u64 res = mag;  // a 64-bit division is a software loop of its own per limb
+        if (mag >= P.q) res = barrett_reduce128(0, mag, Barrett{P.q, P.br_hi, P.br_lo});
+        if (v < 0) res = neg_mod(res, P.q);
         o[(u64)i * N] = res;
     }
 }

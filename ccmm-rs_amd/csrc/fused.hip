@@ -56,6 +56,10 @@ struct ColEntry {
     u32 kind, digits;  // ColKind; polynomials per ciphertext (lifts)
     u64 limit;         // digits: 2^(w-1)
     const ColBlock *blocks;
+    const u64 *m;      // inverse: ColAdd operands
+    const int64_t *err;
+    u64 m_stride;
+    u32 add;
     unsigned char order[kMaxOrder];  // limb_order
 };
 
@@ -74,6 +78,7 @@ struct ColLaunch {
 // stay below 2^45) and cut larger ones at bit 30; integer limbs take residues
 // up to 4q whole, add q to negative digits when limit < q, and reduce the rest
 // (below 2^64) into 3q.  Which of them is the same for a whole block.
+//   bytes: |d| <= 128, below every prime of a two-pass degree;
 //   block: a mixed-radix value, see col_blocks; within 0.54 q or below 2q.
 constexpr int kColFpIn = 16, kColIntIn = 4;
 constexpr u64 kColFpWhole = 1ull << 44;
@@ -82,7 +87,11 @@ template <int K1>
 __device__ __forceinline__ void col_read(u64 (&v)[16], const u64 *src, u32 n2, u32 tile, u32 tid, u32 kind) {
     typedef ColTile<K1> C;
     const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
-    if (kind == kColPlain) {
+    if (kind == kColInt8) {
+        const int8_t *b = (const int8_t *)src;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = (u64)(int64_t)(b + C::template step<0>(n2, i))[o0 / 8];
+    } else if (kind == kColPlain) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = load_once_at(src + C::template step<0>(n2, i), o0);
     } else {
@@ -93,7 +102,7 @@ __device__ __forceinline__ void col_read(u64 (&v)[16], const u64 *src, u32 n2, u
 }
 
 __device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, const RowFp &ar, const CK_CONST_AS DevPrime &) {
-    if (kind == kColPlain || limit <= kColFpWhole) {
+    if (kind == kColPlain || limit <= kColFpWhole) {  // limit 0 for bytes
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = f64_as_u64(signed_to_f64(v[i]));
         return;
@@ -107,7 +116,7 @@ __device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, cons
     }
 }
 __device__ __forceinline__ void col_lift(u64 (&v)[16], u32 kind, u64 limit, const RowInt &ar, const CK_CONST_AS DevPrime &P) {
-    if (kind == kColDigit && limit < ar.q) {
+    if (kind == kColInt8 || (kind == kColDigit && limit < ar.q)) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] += (int64_t)v[i] < 0 ? ar.q : 0;
     } else if (kind == kColDigit || (kind == kColResidue && limit > 4 * ar.q)) {
@@ -184,6 +193,8 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
     if (BLOCK) {
     } else if (e.kind == kColPlain) {
         src = e.src + poly * e.stride + limb * N;
+    } else if (e.kind == kColInt8) {
+        src = (const u64 *)((const int8_t *)e.src + poly * N);
     } else {
         // digit j of ciphertext ct, shared by every limb
         const u32 ct = poly / e.digits, j = poly % e.digits;
@@ -225,7 +236,7 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
     }
 }
 
-template <int K1, class Ar>
+template <int K1, bool ADD, class Ar>
 __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS DevPrime &P, const Ar &ar, u32 limb,
                                             u32 poly, u32 tile, u64 *lds) {
     typedef ColTile<K1> C;
@@ -263,6 +274,20 @@ __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS
         } else {
             r = shoup(v[i], P.ninv, P.ninv_q, ar.q);
         }
+        if constexpr (ADD) {
+            const u32 st = C::template step<0>(n2, i);
+            const u64 m = load_once_at(e.m + poly * e.m_stride + limb * N + st, o0);
+            if (e.add == kAddBody) {
+                r = add_mod(m, r, P.q);
+            } else {
+                const int64_t x = (int64_t)load_at((const u64 *)e.err + poly * N + st, o0);
+                const u64 mag = x < 0 ? 0 - (u64)x : (u64)x;
+                u64 er = mag;
+                if (mag >= P.q) er = barrett_reduce128(0, mag, Barrett{P.q, P.br_hi, P.br_lo});
+                if (x < 0) er = neg_mod(er, P.q);
+                r = sub_mod(add_mod(m, er, P.q), r, P.q);
+            }
+        }
         store_once_at(dst + C::template step<0>(n2, i), o0, r);
         if (!Ar::kFp && (i & 3) == 3) sched_fence();
     }
@@ -275,15 +300,16 @@ __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS
 // not), and heavy limbs still run beside light ones.
 constexpr u32 kColGroup = 4;
 
-template <bool FWD, bool BLOCK>
-__global__ __launch_bounds__(256, BLOCK ? 4 : 5) void k_columns(ColLaunch l) {
+// OTHER: kColBlock digits (forward) or ColAdd (inverse), which take more registers
+template <bool FWD, bool OTHER>
+__global__ __launch_bounds__(256, OTHER ? 4 : 5) void k_columns(ColLaunch l) {
     __shared__ u64 lds[4096];
     u32 di = 0;
     while (di + 1 < l.n && blockIdx.x >= l.e[di + 1].block_start) ++di;
     const ColEntry &e = l.e[di];
     const u32 b = blockIdx.x - e.block_start, lt = e.logn - 12, tiles = 1u << lt;
     u32 limb, poly, tile;
-    if (BLOCK || (FWD && e.kind != kColPlain)) {
+    if (FWD && e.kind != kColPlain && e.kind != kColInt8) {
         const u32 k = b >> 3, group = k / e.n_limbs * 8 + (b & 7);
         if (group >= e.n_polys * tiles) return;
         limb = k % e.n_limbs;
@@ -305,11 +331,11 @@ __global__ __launch_bounds__(256, BLOCK ? 4 : 5) void k_columns(ColLaunch l) {
 #define CK_COL(K1)                                                            \
     case K1:                                                                  \
         if (FWD) {                                                            \
-            if (P.fp) col_forward<K1, BLOCK>(e, P, fp, limb, poly, tile, lds);       \
-            else col_forward<K1, BLOCK>(e, P, in, limb, poly, tile, lds);            \
+            if (P.fp) col_forward<K1, OTHER>(e, P, fp, limb, poly, tile, lds);      \
+            else col_forward<K1, OTHER>(e, P, in, limb, poly, tile, lds);           \
         } else {                                                              \
-            if (P.fp) col_inverse<K1>(e, P, fp, limb, poly, tile, lds);       \
-            else col_inverse<K1>(e, P, in, limb, poly, tile, lds);            \
+            if (P.fp) col_inverse<K1, OTHER>(e, P, fp, limb, poly, tile, lds);      \
+            else col_inverse<K1, OTHER>(e, P, in, limb, poly, tile, lds);           \
         }                                                                     \
         break;
         CK_COL(6)
@@ -321,10 +347,10 @@ __global__ __launch_bounds__(256, BLOCK ? 4 : 5) void k_columns(ColLaunch l) {
 
 int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward) {
     if (count > (size_t)kMaxColEntries) return fail(CKKS_ERR_INVALID, "NTT batch holds at most 16 entries");
-    ColLaunch l{}, lb{};  // lb: kColBlock entries
+    ColLaunch l{}, lo{};  // lo: OTHER entries of k_columns
     for (size_t i = 0; i < count; ++i) {
         const ColCall &c = calls[i];
-        ColLaunch &to = forward && c.kind == kColBlock ? lb : l;
+        ColLaunch &to = (forward ? c.kind == kColBlock : c.add != kAddNone) ? lo : l;
         if (c.n_polys == 0) continue;
         if (!fused_rows_apply(c.plan)) return fail(CKKS_ERR_UNSUPPORTED, "column passes: two-pass degrees, primes below 2^60");
         ColEntry e{};
@@ -340,22 +366,27 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
         e.digits = (u32)c.digits;
         e.limit = c.limit;
         e.blocks = c.blocks;
+        e.m = c.m;
+        e.err = c.e;
+        e.m_stride = c.m_stride;
+        e.add = (u32)c.add;
         limb_order(c.plan, c.n_limbs, e.order);
         to.e[to.n++] = e;
         const size_t groups = c.n_polys << (e.logn - 12);
-        const size_t blocks = to.blocks + (forward && c.kind != kColPlain ? (groups + 7) / 8 * 8 : groups) * c.n_limbs;
+        const size_t blocks = to.blocks + (forward && c.kind != kColPlain && c.kind != kColInt8 ? (groups + 7) / 8 * 8 : groups) * c.n_limbs;
         to.blocks = (u32)blocks;
         if (blocks >= (1ull << 31)) return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
         ckks_execution_profile &pc = ctx->counts();
         (forward ? pc.ntt_forwards : pc.ntt_inverses) += c.n_polys;
         pc.ntt_limb_transforms += c.n_polys * c.n_limbs;
     }
-    // blocks of both kinds (forward): one launch each
-    if (!forward) {
-        if (l.blocks) hipLaunchKernelGGL((k_columns<false, false>), dim3(l.blocks), dim3(256), 0, ctx->stream, l);
+    const dim3 g(l.blocks), go(lo.blocks), t(256);
+    if (forward) {
+        if (l.blocks) hipLaunchKernelGGL((k_columns<true, false>), g, t, 0, ctx->stream, l);
+        if (lo.blocks) hipLaunchKernelGGL((k_columns<true, true>), go, t, 0, ctx->stream, lo);
     } else {
-        if (l.blocks) hipLaunchKernelGGL((k_columns<true, false>), dim3(l.blocks), dim3(256), 0, ctx->stream, l);
-        if (lb.blocks) hipLaunchKernelGGL((k_columns<true, true>), dim3(lb.blocks), dim3(256), 0, ctx->stream, lb);
+        if (l.blocks) hipLaunchKernelGGL((k_columns<false, false>), g, t, 0, ctx->stream, l);
+        if (lo.blocks) hipLaunchKernelGGL((k_columns<false, true>), go, t, 0, ctx->stream, lo);
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
@@ -364,7 +395,7 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
 // ---- block order ----------------------------------------------------------------
 
 // Workgroups (limb, tile, ciphertext).  Integer limbs cost two to three times
-// an FP64 limb, so they are dealt first; blocks reach the 8 XCDs round-robin,
+// an FP64 limb and are spread evenly (limb_order); blocks reach the 8 XCDs round-robin,
 // and group (limb, tile) g runs on XCD g mod 8 with its ciphertexts one after
 // another, so its key tile is read into one L2 and every XCD gets the same
 // share of heavy limbs.
@@ -468,6 +499,69 @@ struct SumInt {
     __device__ __forceinline__ u64 total(S s) const { return shoup_lazy3(s, 0 - r_hi * q, r_lo, q); }
 };
 
+// An exchange writes one of two LDS buffers and reads it after the barrier; the
+// buffer's previous readers passed the other exchange's barrier in between, so
+// one barrier per exchange is enough, also from one transform to the next.
+template <int L>
+using RowLds = u64[RowTile<L>::LDS];
+
+// geometry A (inter-pass) -> C (natural), bounds in b
+template <int L, class Ar>
+__device__ __forceinline__ void row_forward(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, RowLds<L> *lds,
+                                            const Ar &ar) {
+    typedef RowTile<L> R;
+    typename R::LowTw low;
+    R::template fwd<0>(v, b, tid, tw, low, ar);
+    R::template put<0>(v, tid, lds[0]);
+    __syncthreads();
+    R::template get<1>(v, tid, lds[0]);
+    R::level(b);
+    R::template fwd<1>(v, b, tid, tw, low, ar);
+    R::template put<1>(v, tid, lds[1]);
+    low = R::low_twiddles(tw, tid);
+    __syncthreads();
+    R::template get<2>(v, tid, lds[1]);
+    R::level(b);
+#pragma unroll
+    for (int x = 0; x < (1 << R::EX); ++x) R::fwd_group(v, b, x, low, ar);
+}
+
+template <int L, class Ar>
+__device__ __forceinline__ void row_inverse(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, RowLds<L> *lds,
+                                            const Ar &ar) {
+    typedef RowTile<L> R;
+    const typename R::LowTw low = R::low_twiddles(tw, tid);
+    R::template inv<2>(v, b, tid, tw, low, ar);
+    R::template put<2>(v, tid, lds[0]);
+    __syncthreads();
+    R::template get<1>(v, tid, lds[0]);
+    R::level(b);
+    R::template inv<1>(v, b, tid, tw, low, ar);
+    R::template put<1>(v, tid, lds[1]);
+    __syncthreads();
+    R::template get<0>(v, tid, lds[1]);
+    R::level(b);
+    R::template inv<0>(v, b, tid, tw, low, ar);
+}
+
+// NTT-domain entries of geometry C: register i sits bitrev(t) rows from the
+// thread's first, the 2^EX columns of a thread adjacent and 16-byte aligned.
+template <int L>
+__device__ __forceinline__ void natural_read(u64 (&w)[8], const u64 *k, u32 n1, u32 nat0) {
+    typedef RowTile<L> R;
+#pragma unroll
+    for (int i = 0; i < 8; i += R::EX ? 2 : 1) {
+        const u64 *at = k + (bitrev((u32)i >> R::EX, L) << n1) + (i & ((1 << R::EX) - 1));
+        if constexpr (R::EX > 0) {
+            const u64x2 p = load2_at(at, nat0);
+            w[i] = p.x;
+            w[i + 1] = p.y;
+        } else {
+            w[i] = load_at(at, nat0);
+        }
+    }
+}
+
 template <int L, class Ar, class Sum>
 struct RowMacBody {
     typedef RowTile<L> R;
@@ -478,9 +572,6 @@ struct RowMacBody {
     u64 (*lds)[RowTile<L>::LDS];
     u32 tid;
 
-    // An exchange writes one of two LDS buffers and reads it after the barrier;
-    // the buffer's previous readers passed the other exchange's barrier in
-    // between, so one barrier per exchange is enough.
     __device__ __forceinline__ void run(const RowBlock &blk) {
         const u32 logn = a.grid.logn, n1 = logn - L;
         const u64 N = (u64)1 << logn;
@@ -504,21 +595,6 @@ struct RowMacBody {
             for (int i = 0; i < 8; ++i) v[i] = nx[i];
             R::set(b, Ar::kZ);
             tid = opaque(tid);
-            // (natural position of register i: rows bitrev(t) apart, the 2^EX
-            // columns of a thread adjacent and 16-byte aligned)
-            auto key = [&](u64 (&w)[8], const u64 *k) {
-#pragma unroll
-                for (int i = 0; i < 8; i += R::EX ? 2 : 1) {
-                    const u64 *at = k + (bitrev((u32)i >> R::EX, L) << n1) + (i & ((1 << R::EX) - 1));
-                    if constexpr (R::EX > 0) {
-                        const u64x2 p = load2_at(at, nat0);
-                        w[i] = p.x;
-                        w[i + 1] = p.y;
-                    } else {
-                        w[i] = load_at(at, nat0);
-                    }
-                }
-            };
             auto next = [&]() {
                 src += N;
                 if (j + 1 < D) {
@@ -528,7 +604,7 @@ struct RowMacBody {
             };
             // the key entries and the next digit are on their way while the
             // stages run, each requested as late as registers allow
-            key(wb, kb);
+            natural_read<L>(wb, kb, n1, nat0);
             R::template fwd<0>(v, b, tid, P.fwd, low, ar);
             R::template put<0>(v, tid, lds[0]);
             next();
@@ -537,7 +613,7 @@ struct RowMacBody {
             R::level(b);
             R::template fwd<1>(v, b, tid, P.fwd, low, ar);
             R::template put<1>(v, tid, lds[1]);
-            key(wa, ka);
+            natural_read<L>(wa, ka, n1, nat0);
             low = R::low_twiddles(P.fwd, tid);
             __syncthreads();
             R::template get<2>(v, tid, lds[1]);
@@ -565,24 +641,13 @@ struct RowMacBody {
             }
         }
         tid = opaque(tid);
-        low = R::low_twiddles(P.inv, tid);
         u64 *out = a.out + ((u64)blk.limb * a.grid.n_cts + blk.ct) * 2 * N;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = sum.total(c ? sa[i] : sb[i]);
             R::set(b, Sum::kIn);
-            R::template inv<2>(v, b, tid, P.inv, low, ar);
-            R::template put<2>(v, tid, lds[0]);
-            __syncthreads();
-            R::template get<1>(v, tid, lds[0]);
-            R::level(b);
-            R::template inv<1>(v, b, tid, P.inv, low, ar);
-            R::template put<1>(v, tid, lds[1]);
-            __syncthreads();
-            R::template get<0>(v, tid, lds[1]);
-            R::level(b);
-            R::template inv<0>(v, b, tid, P.inv, low, ar);
+            row_inverse<L>(v, b, tid, P.inv, lds, ar);
 #pragma unroll
             for (int i = 0; i < 8; ++i) *(u64 *)((char *)(out + c * N + (i << (L - 3))) + off0) = v[i];
         }
@@ -618,6 +683,202 @@ int launch_row_mac(ckks_context *ctx, const RowMac &m) {
         case 7: hipLaunchKernelGGL(k_row_mac<7>, g, t, 0, ctx->stream, a); break;
         case 8: hipLaunchKernelGGL(k_row_mac<8>, g, t, 0, ctx->stream, a); break;
         default: hipLaunchKernelGGL(k_row_mac<9>, g, t, 0, ctx->stream, a); break;
+    }
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
+}
+
+// ---- products of polynomials -------------------------------------------------------
+
+// Products for operands the forward pass left lazy.  factor() brings one of
+// them into the range the product wants (FP64: half a q; integer: 4 q, so that
+// T = 16 q 4 q < 2^126 and the Montgomery product stays below 5 q).
+__device__ __forceinline__ void row_factor(u64 (&v)[8], int (&)[8], const RowFp &ar) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = f64_as_u64(fp_reduce(u64_as_f64(v[i]), ar.q, ar.qinv));
+}
+__device__ __forceinline__ void row_factor(u64 (&v)[8], int (&b)[8], const RowInt &ar) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ar.reduce_to(v[i], b[i], 4);
+}
+// s += y w: w from row_factor
+__device__ __forceinline__ void row_mac(double &s, u64 y, u64 w, const SumFp &sum) {
+    s += fp_mulmod_q(u64_as_f64(y), u64_as_f64(w), sum.q, sum.qinv);
+}
+__device__ __forceinline__ void row_mac(u64 &s, u64 y, u64 w, const SumInt &sum) { sum.mac(s, y, w); }
+
+struct RowMulArgs {
+    u64 *x;        // inter-pass [limb][poly][N]
+    const u64 *y;  // inter-pass [limb][N], or null
+    const u64 *w;  // natural [limb][N] at w + (poly / share) w_stride
+    u64 w_stride;
+    u32 share;
+    const DevPrime *primes;
+    RowGrid grid;  // n_cts: polynomials
+};
+
+// Forward, product, inverse of one tile: against separate passes this leaves
+// out two or three passes over the data and as many launches.  With the column
+// passes (memory-bound like this one: 16 bytes a residue) a plaintext product
+// of 16 ciphertexts and its rescale take 224 us at N = 2^15, 13 limbs (308 us
+// with separate passes), an encryption of 8 polynomials there 118 us (184 us).
+template <int L, bool INTER, class Ar, class Sum>
+__device__ __forceinline__ void row_mul_tile(const RowMulArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
+                                             const Sum &sum, RowLds<L> *lds, const RowBlock &blk) {
+    typedef RowTile<L> R;
+    const u32 tid = threadIdx.x, logn = a.grid.logn, n1 = logn - L;
+    const u64 N = (u64)1 << logn;
+    const u32 off0 = R::internal_off(blk.tile, n1, tid, 0) * 8;
+    u64 *x = a.x + ((u64)blk.limb * a.grid.n_cts + blk.ct) * N;
+    u64 v[8], w[8];
+    int b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = load_at(x + (i << (L - 3)), off0);
+    if constexpr (INTER) {
+        const u64 *y = a.y + (u64)blk.limb * N;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = load_at(y + (i << (L - 3)), off0);
+        R::set(b, Ar::kZ);
+        row_forward<L>(w, b, tid, P.fwd, lds, ar);
+        row_factor(w, b, ar);
+    } else {
+        const u64 *k = a.w + blk.ct / a.share * a.w_stride + (u64)blk.limb * N;
+        natural_read<L>(w, k, n1, R::natural_off(blk.tile, n1, tid, 0) * 8);
+    }
+    R::set(b, Ar::kZ);
+    row_forward<L>(v, b, tid, P.fwd, lds, ar);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        typename Sum::S s = 0;
+        if constexpr (INTER) row_mac(s, v[i], w[i], sum);
+        else sum.mac(s, v[i], w[i]);
+        v[i] = sum.total(s);
+    }
+    R::set(b, Sum::kIn);
+    row_inverse<L>(v, b, tid, P.inv, lds, ar);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *(u64 *)((char *)(x + (i << (L - 3))) + off0) = v[i];
+}
+
+template <int L, bool INTER>
+__global__ __launch_bounds__(512, 4) void k_row_mul(RowMulArgs a) {
+    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+    const RowBlock blk = row_block(a.grid, blockIdx.x);
+    if (blk.idle) return;
+    const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
+    if (P.fp)
+        row_mul_tile<L, INTER>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
+    else
+        row_mul_tile<L, INTER>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+}
+
+int launch_row_mul(ckks_context *ctx, const RowMul &m) {
+    if (!fused_rows_apply(m.plan)) return fail(CKKS_ERR_UNSUPPORTED, "fused row passes: 2^13 <= N <= 2^17, primes below 2^60");
+    RowMulArgs a{};
+    a.x = m.x;
+    a.y = m.y;
+    a.w = m.w;
+    a.w_stride = m.w_stride;
+    a.share = (u32)m.share;
+    a.primes = m.plan->d_primes;
+    a.grid = row_grid(m.plan, m.limbs, m.n_polys, true);
+    if ((u64)m.limbs * m.n_polys << (m.plan->logn - 12) >= (1ull << 30))
+        return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
+    const dim3 g(row_blocks(a.grid)), t(512);
+    switch (ntt_n2(m.plan->logn) * 2 + (m.y ? 1 : 0)) {
+#define CK_RM(L)                                                                             \
+    case L * 2: hipLaunchKernelGGL((k_row_mul<L, false>), g, t, 0, ctx->stream, a); break;    \
+    case L * 2 + 1: hipLaunchKernelGGL((k_row_mul<L, true>), g, t, 0, ctx->stream, a); break;
+        CK_RM(7) CK_RM(8) CK_RM(9)
+#undef CK_RM
+    }
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
+}
+
+struct RowTensorArgs {
+    u64 *x[4];  // inter-pass b0, a0, b1, a1, each [limb][ct][N]
+    const DevPrime *primes;
+    RowGrid grid;
+};
+
+// Four forward row passes, the products and three inverse passes of one tile;
+// b0 and a0 stay in registers as factors while b1 and a1 are transformed.
+template <int L, class Ar, class Sum>
+__device__ __forceinline__ void row_tensor_tile(const RowTensorArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
+                                                const Sum &sum, RowLds<L> *lds, const RowBlock &blk) {
+    typedef RowTile<L> R;
+    u32 tid = threadIdx.x;
+    const u32 n1 = a.grid.logn - L;
+    const u64 base = ((u64)blk.limb * a.grid.n_cts + blk.ct) << a.grid.logn;
+    const u32 off0 = R::internal_off(blk.tile, n1, tid, 0) * 8;
+    u64 f[2][8], v[8];  // b0 and a0 as factors
+    typename Sum::S c[3][8];
+    int b[8];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[p][i] = load_at(a.x[p] + base + (i << (L - 3)), off0);
+        R::set(b, Ar::kZ);
+        tid = opaque(tid);
+        row_forward<L>(f[p], b, tid, P.fwd, lds, ar);
+        row_factor(f[p], b, ar);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[k][i] = 0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = load_at(a.x[2 + p] + base + (i << (L - 3)), off0);
+        R::set(b, Ar::kZ);
+        tid = opaque(tid);
+        row_forward<L>(v, b, tid, P.fwd, lds, ar);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            row_mac(c[p][i], v[i], f[0][i], sum);
+            row_mac(c[p + 1][i], v[i], f[1][i], sum);
+            sched_fence();
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = sum.total(c[k][i]);
+        R::set(b, Sum::kIn);
+        tid = opaque(tid);
+        row_inverse<L>(v, b, tid, P.inv, lds, ar);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *(u64 *)((char *)(a.x[k] + base + (i << (L - 3))) + off0) = v[i];
+    }
+}
+
+template <int L>
+__global__ __launch_bounds__(512, 4) void k_row_tensor(RowTensorArgs a) {
+    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+    const RowBlock blk = row_block(a.grid, blockIdx.x);
+    if (blk.idle) return;
+    const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
+    if (P.fp)
+        row_tensor_tile<L>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
+    else
+        row_tensor_tile<L>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+}
+
+int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x[4], size_t n_cts, size_t limbs) {
+    if (!fused_rows_apply(plan)) return fail(CKKS_ERR_UNSUPPORTED, "fused row passes: 2^13 <= N <= 2^17, primes below 2^60");
+    RowTensorArgs a{};
+    for (int p = 0; p < 4; ++p) a.x[p] = x[p];
+    a.primes = plan->d_primes;
+    a.grid = row_grid(plan, limbs, n_cts, true);
+    if ((u64)limbs * n_cts << (plan->logn - 12) >= (1ull << 30))
+        return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
+    const dim3 g(row_blocks(a.grid)), t(512);
+    switch (ntt_n2(plan->logn)) {
+        case 7: hipLaunchKernelGGL(k_row_tensor<7>, g, t, 0, ctx->stream, a); break;
+        case 8: hipLaunchKernelGGL(k_row_tensor<8>, g, t, 0, ctx->stream, a); break;
+        default: hipLaunchKernelGGL(k_row_tensor<9>, g, t, 0, ctx->stream, a); break;
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;

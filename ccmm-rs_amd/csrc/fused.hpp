@@ -18,6 +18,13 @@ enum ColKind {
     kColResidue = 1,  // digit j of a ciphertext is its limb j ([ct][digits][N]), lifted to every limb
     kColDigit = 2,    // balanced digits, int64 [ct][digits][N], |d| <= limit, lifted to every limb
     kColBlock = 3,    // digit j is given by its mixed-radix digits ([ct][.][N], see ColBlock)
+    kColInt8 = 4,     // signed bytes [p][N], the same in every limb
+};
+// What the inverse column pass adds to its result v on the way out.
+enum ColAdd {
+    kAddNone = 0,
+    kAddMessage = 1,  // m + e - v: m like the output, e int64 [p][N]
+    kAddBody = 2,     // m + v
 };
 // A gadget block as kColBlock evaluates it: the block's value is sum_t c_t W_t,
 // c_t < 2^41 the mixed-radix digits (limbs first .. of the ciphertext's data);
@@ -43,6 +50,10 @@ struct ColCall {
     size_t digits = 1;  // polynomials per ciphertext (lifts)
     u64 limit = 0;      // kColDigit
     const ColBlock *blocks = nullptr;  // kColBlock: one per digit, device memory
+    int add = kAddNone;                // inverse
+    const u64 *m = nullptr;
+    size_t m_stride = 0;
+    const int64_t *e = nullptr;
 };
 int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward);
 
@@ -59,5 +70,24 @@ struct RowMac {
     bool xcd_order;  // ciphertexts of one key tile on one XCD
 };
 int launch_row_mac(ckks_context *ctx, const RowMac &m);
+
+// Products between the column passes, in place of the first operand's
+// inter-pass data (n_polys polynomials of `limbs` limbs).
+struct RowMul {
+    const ckks_rns_plan *plan;
+    u64 *x;
+    size_t n_polys, limbs;
+    // the other operand: inter-pass data of one polynomial for all of them, or
+    const u64 *y = nullptr;
+    // NTT-domain values in natural order, [limb][N] for every `share`
+    // polynomials, w_stride apart
+    const u64 *w = nullptr;
+    size_t share = 1, w_stride = 0;
+};
+int launch_row_mul(ckks_context *ctx, const RowMul &m);
+
+// Tensor of ciphertext pairs: inter-pass b0, a0, b1, a1 (n_cts polynomials
+// each) to inter-pass b0 b1, b0 a1 + a0 b1, a0 a1 in the place of b0, a0, b1.
+int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x[4], size_t n_cts, size_t limbs);
 
 }  // namespace ck

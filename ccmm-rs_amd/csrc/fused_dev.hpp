@@ -20,7 +20,8 @@ __device__ __forceinline__ double load_z(const double *base, u32 off) {
     return *(const double *)((const char *)base + off * 8);
 }
 __device__ __forceinline__ Tw load_z(const Tw *base, u32 off) { return *(const Tw *)((const char *)base + off * 16); }
-typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+// two residues; callers' strides leave 8-byte alignment only
+typedef u64 u64x2 __attribute__((ext_vector_type(2), aligned(8)));
 __device__ __forceinline__ u64x2 load2_at(const u64 *base, u32 byte_off) {
     return *(const u64x2 *)((const char *)base + byte_off);
 }

@@ -4,6 +4,7 @@
 // limb so loads/stores are 16-byte and a block never straddles limbs.
 #include <algorithm>
 
+#include "fused.hpp"
 #include "host_math.hpp"
 #include "internal.hpp"
 
@@ -466,6 +467,16 @@ static int tensor(const ckks_rns_plan *plan, const u64 *ct0, const u64 *ct1, u64
     if ((rc = ctx->workspace(1, n_cts * 4 * poly * sizeof(u64), &w1))) return rc;
     if ((rc = ctx->workspace(2, n_cts * 3 * poly * sizeof(u64), &w2))) return rc;
     u64 *x = (u64 *)w1, *y = (u64 *)w2;
+    if (fused_rows_apply(plan)) {
+        const size_t each = n_cts * poly;
+        u64 *const p[4] = {x, x + each, x + 2 * each, x + 3 * each};
+        ColCall f[4], iv[3];
+        for (int i = 0; i < 4; ++i)
+            f[i] = ColCall{plan, (i < 2 ? ct0 : ct1) + (i & 1) * poly, p[i], n_cts, n_limbs, in_stride};
+        for (int i = 0; i < 3; ++i) iv[i] = ColCall{plan, p[i], out + i * poly, n_cts, n_limbs, out_stride};
+        if ((rc = launch_columns(ctx, f, 4, true)) || (rc = launch_row_tensor(ctx, plan, p, n_cts, n_limbs))) return rc;
+        return launch_columns(ctx, iv, 3, false);
+    }
     // x = [ct][b0, a0, b1, a1][limb][N] in the NTT domain
     NttCall fwd[4] = {
         {plan, ct0, x, n_cts, n_limbs, in_stride, 4 * poly},
@@ -536,6 +547,23 @@ static int multiply_plain(const ckks_rns_plan *plan, const u64 *in, const u64 *p
     void *w;
     if ((rc = ctx->workspace(1, n_cts * 2 * poly * sizeof(u64), &w))) return rc;
     u64 *x = (u64 *)w;
+    if (fused_rows_apply(plan)) {
+        // one entry for both components where they are evenly spaced
+        const bool even = in_stride == 2 * poly && out_stride == 2 * poly;
+        const size_t comps = even ? 1 : 2, polys = even ? 2 * n_cts : n_cts;
+        const size_t is = even ? poly : in_stride, os = even ? poly : out_stride;
+        ColCall f[2], iv[2];
+        for (size_t c = 0; c < comps; ++c) {
+            u64 *xc = x + c * polys * poly;
+            f[c] = ColCall{plan, in + c * poly, xc, polys, n_limbs, is};
+            iv[c] = ColCall{plan, xc, out + c * poly, polys, n_limbs, os};
+        }
+        if ((rc = launch_columns(ctx, f, comps, true))) return rc;
+        for (size_t c = 0; c < comps; ++c)
+            if ((rc = launch_row_mul(ctx, RowMul{plan, x + c * polys * poly, polys, n_limbs, nullptr, pt, polys / n_cts, pt_stride})))
+                return rc;
+        return launch_columns(ctx, iv, comps, false);
+    }
     NttCall fwd[2] = {{plan, in, x, n_cts, n_limbs, in_stride, 2 * poly},
                       {plan, in + poly, x + poly, n_cts, n_limbs, in_stride, 2 * poly}};
     if ((rc = launch_ntt(ctx, fwd, 2, true))) return rc;
@@ -655,6 +683,19 @@ static int rlwe_raw(const ckks_rns_plan *plan, const u64 *m, size_t m_stride, co
     void *w;
     if ((rc = ctx->workspace(1, (1 + n_polys) * poly * sizeof(u64), &w))) return rc;
     u64 *s_ntt = (u64 *)w, *as = s_ntt + poly;
+    if (fused_rows_apply(plan)) {
+        ColCall f[2] = {{plan, a_in, as, n_polys, n_limbs, a_stride}, {plan, (const u64 *)secret, s_ntt, 1, n_limbs}};
+        f[1].kind = kColInt8;
+        ColCall iv{plan, as, out, n_polys, n_limbs, out_stride};
+        iv.add = encrypt ? kAddMessage : kAddBody;
+        iv.m = m;
+        iv.m_stride = m_stride;
+        iv.e = e;
+        if ((rc = launch_columns(ctx, f, 2, true)) ||
+            (rc = launch_row_mul(ctx, RowMul{plan, as, n_polys, n_limbs, s_ntt})))
+            return rc;
+        return launch_columns(ctx, &iv, 1, false);
+    }
     ProjectArgs pa{secret, s_ntt, plan->d_primes, (u32)n_limbs, plan->logn};
     hipLaunchKernelGGL(k_project_secret, dim3((u32)((poly + kEwThreads - 1) / kEwThreads)), dim3(kEwThreads), 0,
                        ctx->stream, pa);

@@ -1,0 +1,111 @@
+"""Paths through the fused row and column passes against the separate
+transforms and pointwise kernels: whole residues, so equality."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import rand_residues
+
+pytestmark = pytest.mark.gpu
+
+# FP64 limbs (up to 41 bits) beside integer limbs (up to 60), and a limb above
+# 2^60 that keeps a plan on the separate passes
+MIXES = {"fp": [40, 30, 41], "int": [60, 42], "both": [60, 40, 55, 36, 41], "wide": [61, 40]}
+
+
+def _moduli(pkg, n, bits):
+    out = []
+    for b in bits:
+        out += pkg.find_ntt_primes(b, n, 1, skip=out)
+    return out
+
+
+def _extremes(rng, moduli, n, polys):
+    x = rand_residues(rng, moduli, n, polys)
+    x[0, :, : n // 2] = np.array(moduli, dtype=np.uint64)[:, None] - 1
+    x[-1, :, n // 2:] = 0
+    return x
+
+
+def _mul(pkg, plan, x, y_ntt):
+    """x [p][limbs][N] times y_ntt (the same shape, NTT domain), separate passes."""
+    t = pkg.empty(tuple(x.shape))
+    plan.forward(x, t)
+    plan.pointwise_mul(t, y_ntt, t)
+    plan.inverse(t)
+    return t
+
+
+@pytest.mark.parametrize("mix", sorted(MIXES))
+@pytest.mark.parametrize("logn", [13, 14, 15, 16, 17])
+def test_products_match_separate_passes(pkg, ctx, logn, mix):
+    import torch
+
+    n, bits = 1 << logn, MIXES[mix]
+    moduli = _moduli(pkg, n, bits)
+    L, n_cts = len(moduli), 3
+    rng = np.random.default_rng(logn * 10 + L)
+    plan = pkg.PreparedRnsNttPlan(ctx, moduli, n)
+    ct = pkg.to_device(_extremes(rng, moduli, n, 2 * n_cts))
+    other = pkg.to_device(_extremes(rng, moduli, n, 2 * n_cts))
+    pt = pkg.to_device(_extremes(rng, moduli, n, n_cts))
+
+    # plaintext products: one plaintext for all ciphertexts, one per ciphertext
+    c4 = ct.reshape(n_cts, 2, L, n)
+    for per_ct in (False, True):
+        w = pt if per_ct else pt[:1]
+        y = w.reshape(-1, 1, L, n).expand(n_cts, 2, L, n).contiguous().reshape(2 * n_cts, L, n)
+        want = _mul(pkg, plan, ct, y)
+        got = plan.multiply_plain(c4, w.contiguous(), L)
+        assert torch.equal(got.reshape(2 * n_cts, L, n), want), f"plain {per_ct}"
+    inplace = c4.clone()
+    assert torch.equal(plan.multiply_plain(inplace, pt[:1].contiguous(), L, out=inplace),
+                       plan.multiply_plain(c4, pt[:1].contiguous(), L))
+
+    # tensor
+    o4 = other.reshape(n_cts, 2, L, n)
+    f, g = pkg.empty(tuple(ct.shape)), pkg.empty(tuple(ct.shape))
+    plan.forward(ct, f)
+    plan.forward(other, g)
+    f, g = f.reshape(n_cts, 2, L, n), g.reshape(n_cts, 2, L, n)
+    parts = []
+    for pairs in (((0, 0),), ((0, 1), (1, 0)), ((1, 1),)):
+        acc = None
+        for i, j in pairs:
+            t = pkg.empty((n_cts, L, n))
+            plan.pointwise_mul(f[:, i].contiguous(), g[:, j].contiguous(), t)
+            if acc is None:
+                acc = t
+            else:
+                plan.add(acc, t, acc)
+        plan.inverse(acc)
+        parts.append(acc)
+    got = plan.tensor(c4, o4, L)
+    for k in range(3):
+        assert torch.equal(got[:, k], parts[k]), f"tensor part {k}"
+
+    # encryption and decryption; errors at the ends of int64, secret at int8's
+    s = rng.integers(-1, 2, n).astype(np.int8)
+    s[:4] = [127, -128, 1, -1]
+    e = rng.integers(-(1 << 63), (1 << 63) - 1, (2 * n_cts, n))
+    e[0, :4] = [-(1 << 63), (1 << 63) - 1, 0, -1]
+    e[-1] = rng.integers(-40, 41, n)
+    q = np.array(moduli, dtype=object)[:, None]
+    sr = np.array(s.astype(object)[None] % q, dtype=np.uint64)
+    er = np.stack([np.array(x.astype(object)[None] % q, dtype=np.uint64) for x in e])
+    ds = pkg.to_device(sr)
+    plan.forward(ds.reshape(1, L, n), ds.reshape(1, L, n))
+    s_ntt = ds.reshape(1, L, n).expand(2 * n_cts, L, n).contiguous()
+    as_ = _mul(pkg, plan, other, s_ntt)
+    sec = torch.from_numpy(s).cuda()
+    b = plan.encrypt_raw(ct, torch.from_numpy(e).cuda(), sec, other)
+    want = pkg.empty(tuple(ct.shape))
+    plan.add(ct, pkg.to_device(er), want)
+    plan.sub(want, as_, want)
+    assert torch.equal(b, want), "encrypt"
+    got = plan.decrypt_raw(ct, other, sec)
+    plan.add(ct, as_, want)
+    assert torch.equal(got, want), "decrypt"
+    one = plan.decrypt_raw(ct[:1].contiguous(), other[:1].contiguous(), sec, out=ct[:1].clone())
+    assert torch.equal(one, want[:1]), "decrypt one"

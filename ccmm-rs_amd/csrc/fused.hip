@@ -527,19 +527,19 @@ __device__ __forceinline__ void row_forward(u64 (&v)[8], int (&b)[8], u32 tid, c
 }
 
 template <int L, class Ar>
-__device__ __forceinline__ void row_inverse(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, RowLds<L> *lds,
+__device__ __forceinline__ void row_inverse(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, u64 *l0, u64 *l1,
                                             const Ar &ar) {
     typedef RowTile<L> R;
     const typename R::LowTw low = R::low_twiddles(tw, tid);
     R::template inv<2>(v, b, tid, tw, low, ar);
-    R::template put<2>(v, tid, lds[0]);
+    R::template put<2>(v, tid, l0);
     __syncthreads();
-    R::template get<1>(v, tid, lds[0]);
+    R::template get<1>(v, tid, l0);
     R::level(b);
     R::template inv<1>(v, b, tid, tw, low, ar);
-    R::template put<1>(v, tid, lds[1]);
+    R::template put<1>(v, tid, l1);
     __syncthreads();
-    R::template get<0>(v, tid, lds[1]);
+    R::template get<0>(v, tid, l1);
     R::level(b);
     R::template inv<0>(v, b, tid, tw, low, ar);
 }
@@ -647,7 +647,7 @@ struct RowMacBody {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = sum.total(c ? sa[i] : sb[i]);
             R::set(b, Sum::kIn);
-            row_inverse<L>(v, b, tid, P.inv, lds, ar);
+            row_inverse<L>(v, b, tid, P.inv, lds[0], lds[1], ar);
 #pragma unroll
             for (int i = 0; i < 8; ++i) *(u64 *)((char *)(out + c * N + (i << (L - 3))) + off0) = v[i];
         }
@@ -755,7 +755,7 @@ __device__ __forceinline__ void row_mul_tile(const RowMulArgs &a, const CK_CONST
         v[i] = sum.total(s);
     }
     R::set(b, Sum::kIn);
-    row_inverse<L>(v, b, tid, P.inv, lds, ar);
+    row_inverse<L>(v, b, tid, P.inv, lds[0], lds[1], ar);
 #pragma unroll
     for (int i = 0; i < 8; ++i) *(u64 *)((char *)(x + (i << (L - 3))) + off0) = v[i];
 }
@@ -848,7 +848,7 @@ __device__ __forceinline__ void row_tensor_tile(const RowTensorArgs &a, const CK
         for (int i = 0; i < 8; ++i) v[i] = sum.total(c[k][i]);
         R::set(b, Sum::kIn);
         tid = opaque(tid);
-        row_inverse<L>(v, b, tid, P.inv, lds, ar);
+        row_inverse<L>(v, b, tid, P.inv, lds[0], lds[1], ar);
 #pragma unroll
         for (int i = 0; i < 8; ++i) *(u64 *)((char *)(a.x[k] + base + (i << (L - 3))) + off0) = v[i];
     }
@@ -879,6 +879,159 @@ int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x
         case 7: hipLaunchKernelGGL(k_row_tensor<7>, g, t, 0, ctx->stream, a); break;
         case 8: hipLaunchKernelGGL(k_row_tensor<8>, g, t, 0, ctx->stream, a); break;
         default: hipLaunchKernelGGL(k_row_tensor<9>, g, t, 0, ctx->stream, a); break;
+    }
+    CK_HIP(hipGetLastError());
+    return CKKS_OK;
+}
+
+// ---- hoisted rotations -------------------------------------------------------------
+
+struct RowRotateArgs {
+    const u64 *digits, *bhat;
+    const DevPrime *primes;
+    RowRotation e[kRowRotations];
+    RowGrid grid;  // n_cts: rotations of every ciphertext, the exponent fastest
+    u32 count, dnum, q_limbs;
+};
+
+__device__ __forceinline__ u64 sum_input(u64 x, const RowFp &) { return f64_as_u64(small_to_f64(x)); }
+__device__ __forceinline__ u64 sum_input(u64 x, const RowInt &) { return x; }
+// v + a canonical x; `b` grows by kCanonical
+__device__ __forceinline__ u64 plus(u64 v, u64 x, const RowFp &) { return f64_as_u64(u64_as_f64(v) + small_to_f64(x)); }
+__device__ __forceinline__ u64 plus(u64 v, u64 x, const RowInt &) { return v + x; }
+
+// Key products of the digits of one tile, sigma_k and the inverse row pass.
+// Evaluation point n = T N1 + u of the result is point ((2n + 1) k - 1) / 2 of
+// the sums, so sigma_k takes row u to row u' as a whole ((2u' + 1) k = 2u + 1
+// mod 2 N1: the store goes to another 2^L-residue run) and permutes within it,
+// T -> T k^-1 + c(u): one more exchange through LDS.  The permuted sums never
+// reach HBM.  4 rotations of 16 ciphertexts at N = 2^16, 25 + 7 limbs, dnum 3:
+// 1.58 ms, where the products (0.81 ms) and a permuting first inverse pass
+// (1.23 ms) took two launches.  What bounds it is the entries each workgroup
+// reads from L2 (keys alone: 1.18 ms without them); sharing them between two
+// ciphertexts of a workgroup took the registers that it saved in loads
+// (1.55 ms with spills), one workgroup per sum 1.83 ms.
+template <int L, class Ar, class Sum>
+__device__ __forceinline__ void row_rotate_tile(const RowRotateArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
+                                                const Sum &sum, RowLds<L> *lds, const RowBlock &blk) {
+    typedef RowTile<L> R;
+    constexpr int KC = R::KC, EX = R::EX, CL = R::CL;
+    constexpr int kCanonical = Ar::kFp ? 2 : 1;
+    u32 tid = threadIdx.x;
+    const u32 logn = a.grid.logn, n1 = logn - L;
+    const u64 N = (u64)1 << logn, stride = (u64)a.grid.limbs * N;
+    const u32 ct = blk.ct / a.count;
+    const RowRotation &e = a.e[blk.ct % a.count];
+    const u32 nat0 = R::natural_off(blk.tile, n1, tid, 0) * 8;
+    const u64 *src = a.digits + (u64)ct * a.dnum * stride + (u64)blk.limb * N;
+    const u64 *kb = e.kb + (u64)blk.limb * N, *ka = e.ka + (u64)blk.limb * N;
+    typename Sum::S sb[8], sa[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sb[i] = sa[i] = 0;
+    u64 v[8], w[8];
+#pragma unroll 1
+    for (u32 j = 0;; ++j) {
+        u64 wa[8];
+        natural_read<L>(v, src, n1, nat0);
+        natural_read<L>(w, kb, n1, nat0);
+        natural_read<L>(wa, ka, n1, nat0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const u64 y = sum_input(v[i], ar);
+            sum.mac(sb[i], y, w[i]);
+            sum.mac(sa[i], y, wa[i]);
+            if (!Ar::kFp || (i & 1)) sched_fence();
+        }
+        if (j + 1 == a.dnum) break;
+        if (Sum::full(j)) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                sb[i] = sum.reduced(sb[i]);
+                sa[i] = sum.reduced(sa[i]);
+            }
+        }
+        src += stride;
+        kb += stride;
+        ka += stride;
+    }
+    const u32 mask2 = (2u << logn) - 1, rows = (1u << L) - 1;
+    u64 *out = e.out + ((u64)blk.limb * (a.grid.n_cts / a.count) + ct) * 2 * N;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        int b[8], bound = Sum::kIn;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = sum.total(c ? sa[i] : sb[i]);
+        if (e.tb) {
+            natural_read<L>(w, (c ? e.ta : e.tb) + (u64)blk.limb * N, n1, nat0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = plus(v[i], w[i], ar);
+        }
+        bound += kCanonical;
+        if (c == 0 && a.bhat && blk.limb < a.q_limbs) {
+            natural_read<L>(w, a.bhat + ((u64)ct * a.q_limbs + blk.limb) * N, n1, nat0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = plus(v[i], w[i], ar);
+        }
+        if (c == 0) bound += kCanonical;
+        // sigma_k: the two sums take turns with the buffers, so that no put
+        // meets a get of the same buffer without a barrier between them
+        tid = opaque(tid);
+        {
+            const u32 T0 = bitrev(R::t_of(2, tid, 0), L) * e.kinv;
+            const u32 u0 = (blk.tile << CL) + R::col_of(2, tid, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const u32 col = (u32)i & ((1u << EX) - 1), x = bitrev((u32)i >> EX, L);
+                const u32 carry = (((2 * (u0 + col) + 1) * e.kinv) & mask2) >> (n1 + 1);
+                const u32 t = bitrev((T0 + x * e.kinv + carry) & rows, L);
+                const u32 at = R::slot((t << CL) | (R::col_of(2, tid, 0) + col));
+                CK_BOUNDS(at, (u32)R::LDS);
+                lds[c][at] = v[i];
+            }
+        }
+        __syncthreads();
+        R::template get<2>(v, tid, lds[c]);
+        R::set(b, bound);
+        row_inverse<L>(v, b, tid, P.inv, lds[1 - c], lds[c], ar);
+        const u32 u = (blk.tile << CL) + R::col_of(0, tid, 0);
+        const u32 to = (((2 * u + 1) * e.kinv) & ((2u << n1) - 1)) >> 1;
+        const u32 off = ((bitrev(to, n1) << L) + R::t_of(0, tid, 0)) * 8;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *(u64 *)((char *)(out + c * N + (i << (L - 3))) + off) = v[i];
+    }
+}
+
+template <int L>
+__global__ __launch_bounds__(512, 4) void k_row_rotate(RowRotateArgs a) {
+    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+    const RowBlock blk = row_block(a.grid, blockIdx.x);
+    if (blk.idle) return;
+    const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
+    if (P.fp)
+        row_rotate_tile<L>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
+    else
+        row_rotate_tile<L>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+}
+
+int launch_row_rotate(ckks_context *ctx, const RowRotate &r) {
+    if (!fused_rows_apply(r.plan)) return fail(CKKS_ERR_UNSUPPORTED, "fused row passes: 2^13 <= N <= 2^17, primes below 2^60");
+    if (r.count == 0 || r.count > (size_t)kRowRotations) return fail(CKKS_ERR_INVALID, "1..16 exponents a launch");
+    RowRotateArgs a{};
+    a.digits = r.digits;
+    a.bhat = r.bhat;
+    a.primes = r.plan->d_primes;
+    for (size_t i = 0; i < r.count; ++i) a.e[i] = r.e[i];
+    a.count = (u32)r.count;
+    a.dnum = (u32)r.dnum;
+    a.q_limbs = (u32)r.q_limbs;
+    a.grid = row_grid(r.plan, r.limbs, r.n_cts * r.count, true);
+    if ((u64)r.limbs * r.n_cts * r.count << (r.plan->logn - 12) >= (1ull << 30))
+        return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
+    const dim3 g(row_blocks(a.grid)), t(512);
+    switch (ntt_n2(r.plan->logn)) {
+        case 7: hipLaunchKernelGGL(k_row_rotate<7>, g, t, 0, ctx->stream, a); break;
+        case 8: hipLaunchKernelGGL(k_row_rotate<8>, g, t, 0, ctx->stream, a); break;
+        default: hipLaunchKernelGGL(k_row_rotate<9>, g, t, 0, ctx->stream, a); break;
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;

@@ -90,4 +90,24 @@ int launch_row_mul(ckks_context *ctx, const RowMul &m);
 // each) to inter-pass b0 b1, b0 a1 + a0 b1, a0 a1 in the place of b0, a0, b1.
 int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x[4], size_t n_cts, size_t limbs);
 
+// Hoisted rotations of one batch of digits by several exponents: for each, the
+// products with its key (entries permuted by k^-1), the corrections, sigma_k
+// and the inverse row pass of both sums.
+constexpr int kRowRotations = 16;
+struct RowRotation {
+    const u64 *kb, *ka;  // [dnum][limbs][N], NTT domain, natural order
+    const u64 *tb, *ta;  // [limbs][N] added to the sums, or null
+    u64 *out;            // inter-pass, polynomials [ct][2]
+    u32 kinv;            // k^-1 modulo 2N
+};
+struct RowRotate {
+    const ckks_rns_plan *plan;
+    const u64 *digits;  // [ct][dnum][limbs][N], NTT domain
+    const u64 *bhat;    // added to every first sum on limbs below q_limbs, [ct][q_limbs][N], or null
+    size_t n_cts, dnum, limbs, q_limbs;
+    const RowRotation *e;
+    size_t count;
+};
+int launch_row_rotate(ckks_context *ctx, const RowRotate &r);
+
 }  // namespace ck

@@ -2200,6 +2200,35 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
     return rc ? rc : launch_columns(ctx, inv.data(), count, false);
 }
 
+// k^-1 mod 2N for an odd Galois exponent (Newton iteration on a power of two).
+static u64 galois_inverse(u64 k, u64 two_n) {
+    u64 inv = k;
+    for (int it = 0; it < 6; ++it) inv = inv * (2 - k * inv);
+    return inv & (two_n - 1);
+}
+
+// Steps 2 to 4 of hoisted jobs whose keys are fused (ks_fused) and which share
+// their digits, key shape and plan: sums into each job's mac_out, inverse
+// column pass into its accumulators.
+static int ks_rotate_middle(ckks_context *ctx, const KsJob *const *jobs, size_t count) {
+    const KsJob &j0 = *jobs[0];
+    const ckks_ksk *k = j0.k;
+    const u32 two_n = 2 * (u32)k->degree;
+    RowRotation e[kRowRotations];
+    ColCall inv[kRowRotations];
+    if (count > (size_t)kRowRotations) return fail(CKKS_ERR_INVALID, "a hoisted rotation batch holds at most 16 entries");
+    for (size_t i = 0; i < count; ++i) {
+        const KsJob &j = *jobs[i];
+        const HoistedMac &h = *j.hm;
+        e[i] = RowRotation{h.kb, h.ka, h.tb, h.ta, j.mac_out, (u32)galois_inverse(h.k, two_n)};
+        inv[i] = ColCall{k->plan, j.mac_out, j.acc, j.n_cts * 2, k->limbs, k->limbs * k->degree};
+    }
+    const RowRotate r{k->plan, j0.hm->digits, ks_mac_takes_b(j0) ? j0.hm->bhat : nullptr, j0.n_cts, k->dnum,
+                      k->limbs, k->q_limbs, e, count};
+    if (int rc = launch_row_rotate(ctx, r)) return rc;
+    return launch_columns(ctx, inv, count, false);
+}
+
 static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const u64 *add0,
                            const u64 *add1, u64 add_stride, u64 *out, u64 out_stride, size_t n_cts,
                            u64 galois_kinv, const int64_t *hoisted, const HoistedMac *hm) {
@@ -2229,6 +2258,11 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
         if ((rc = ctx->workspace(0, n_cts * D * B * N * sizeof(u64), &wc))) return rc;
         const KsJob *jp = &j;
         if ((rc = ks_fused_middle(ctx, &jp, 1, (u64 *)wc))) return rc;
+        return ks_moddown(j, s);
+    }
+    if (hm && ks_fused(k)) {
+        const KsJob *jp = &j;
+        if ((rc = ks_rotate_middle(ctx, &jp, 1))) return rc;
         return ks_moddown(j, s);
     }
     // 1. ModUp
@@ -2444,13 +2478,6 @@ int ckks_bounded_digits(const ckks_rns_plan *plan, size_t q_limbs, unsigned base
                         int64_t *out, size_t n_polys, size_t in_stride) {
     if (n_polys && !out) return fail(CKKS_ERR_INVALID, "null argument");
     return bounded_decompose_impl(plan, q_limbs, base_log, in, nullptr, out, n_polys, in_stride);
-}
-
-// k^-1 mod 2N for an odd Galois exponent (Newton iteration on a power of two).
-static u64 galois_inverse(u64 k, u64 two_n) {
-    u64 inv = k;
-    for (int it = 0; it < 6; ++it) inv = inv * (2 - k * inv);
-    return inv & (two_n - 1);
 }
 
 int ckks_bounded_digits_automorphism(const ckks_rns_plan *plan, size_t q_limbs, unsigned base_log,
@@ -3162,10 +3189,10 @@ int ckks_rotate_hoisted_batch(ckks_context *ctx, const ckks_hoisted_rotation *e,
         fast.push_back(Fast{h, key, r.in, r.out, in_stride, out_stride, k, pk});
     }
     if (fast.empty()) return CKKS_OK;
-    // every entry's MAC in the first inverse pass, or none
+    // every entry's MAC in the first inverse pass (CKKS_KS_FUSION_INVERSE), or none
     bool fused = true;
     for (const Fast &f : fast)
-        fused = fused && !f.h->d_bhat && hoisted_mac_fused(ctx, f.key->plan->logn, f.key->dnum);
+        fused = fused && !ks_fused(f.key) && !f.h->d_bhat && hoisted_mac_fused(ctx, f.key->plan->logn, f.key->dnum);
     // the MAC outputs (slot 4, unfused only) and the accumulators (slot 5)
     size_t total = 0;
     for (const Fast &f : fast) total += f.h->n_cts * 2 * f.key->limbs * f.key->degree;
@@ -3203,27 +3230,34 @@ int ckks_rotate_hoisted_batch(ckks_context *ctx, const ckks_hoisted_rotation *e,
         pc.key_switches += f.h->n_cts;
         (f.k == 2 * (u64)N - 1 ? pc.automorphisms : pc.rotations) += f.h->n_cts;
     }
-    // the MACs: entries of one hoisted batch share their digit reads, up to
-    // kMacMaxExp exponents per launch
-    if (!fused) {
-        std::vector<bool> done(fast.size(), false);
-        for (size_t i = 0; i < fast.size(); ++i) {
-            if (done[i]) continue;
-            std::vector<size_t> grp{i};
-            done[i] = true;
-            for (size_t m = i + 1; m < fast.size() && grp.size() < (size_t)kMacMaxExp; ++m)
-                if (!done[m] && fast[m].h == fast[i].h && fast[m].key->dnum == fast[i].key->dnum &&
-                    fast[m].key->limbs == fast[i].key->limbs) {
-                    grp.push_back(m);
-                    done[m] = true;
-                }
-            if ((rc = ks_mac_group(jobs, grp, s))) return rc;
+    // entries of one hoisted batch share their digit reads: the fused ones in
+    // one launch, the others in MACs of up to kMacMaxExp exponents
+    std::vector<bool> done(fast.size(), false);
+    for (size_t i = 0; i < fast.size(); ++i) {
+        const bool rows = ks_fused(fast[i].key);
+        if (done[i] || (fused && !rows)) continue;
+        std::vector<size_t> grp{i};
+        for (size_t m = i + 1; m < fast.size() && (rows || grp.size() < (size_t)kMacMaxExp); ++m)
+            if (!done[m] && fast[m].h == fast[i].h && fast[m].key->dnum == fast[i].key->dnum &&
+                fast[m].key->limbs == fast[i].key->limbs && ks_fused(fast[m].key) == rows) {
+                grp.push_back(m);
+            }
+        for (size_t m : grp) done[m] = true;
+        if (rows) {
+            std::vector<const KsJob *> jp;
+            for (size_t m : grp) jp.push_back(&jobs[m]);
+            if ((rc = ks_rotate_middle(ctx, jp.data(), jp.size()))) return rc;
+        } else if ((rc = ks_mac_group(jobs, grp, s))) {
+            return rc;
         }
     }
-    // one inverse NTT launch per pass for every entry, each reading its MAC
-    // (computed in the first pass when fused) through its own Galois
+    // one inverse NTT launch per pass for the entries left, each reading its
+    // MAC (computed in the first pass when fused) through its own Galois
     // permutation
-    if ((rc = launch_ntt(ctx, inv.data(), inv.size(), false))) return rc;
+    std::vector<NttCall> rest;
+    for (size_t i = 0; i < fast.size(); ++i)
+        if (!ks_fused(fast[i].key)) rest.push_back(inv[i]);
+    if (!rest.empty() && (rc = launch_ntt(ctx, rest.data(), rest.size(), false))) return rc;
     for (KsJob &j : jobs)
         if ((rc = ks_moddown(j, s))) return rc;
     return CKKS_OK;

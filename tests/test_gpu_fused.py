@@ -109,3 +109,33 @@ def test_products_match_separate_passes(pkg, ctx, logn, mix):
     assert torch.equal(got, want), "decrypt"
     one = plan.decrypt_raw(ct[:1].contiguous(), other[:1].contiguous(), sec, out=ct[:1].clone())
     assert torch.equal(one, want[:1]), "decrypt one"
+
+
+@pytest.mark.parametrize("with_b", [False, True])
+@pytest.mark.parametrize("mix", ["fp", "both"])
+@pytest.mark.parametrize("logn", [13, 14, 15, 16, 17])
+def test_hoisted_rotations_match_rotations(pkg, ctx, logn, mix, with_b):
+    """sigma_k of the sums inside a tile, for conjugation and exponents of both
+    halves, against the rotation that permutes its input instead."""
+    import torch
+
+    n, bits = 1 << logn, MIXES[mix]
+    q = _moduli(pkg, n, bits)
+    qp = q + pkg.find_ntt_primes(59, n, 2, skip=q)
+    L = len(q)
+    blocks = [L - L // 2, L // 2]
+    rng = np.random.default_rng(logn * 10 + L)
+    plan = pkg.PreparedRnsNttPlan(ctx, qp, n)
+    keys = [pkg.HybridKeySwitchKey(plan, L, blocks, rand_residues(rng, qp, n, 2), rand_residues(rng, qp, n, 2))
+            for _ in range(2)]
+    ct = rand_residues(rng, q, n, 6).reshape(3, 2, L, n)
+    ct[1, 1, :, 1:3] = np.array(q, dtype=np.uint64)[:, None] - 1
+    ct = pkg.to_device(ct)
+    hoisted = keys[0].hoist(ct, with_b=with_b)
+    exps = [(0, 5), (1, 2 * n - 1), (0, n + 1), (1, 2 * n - 5)]
+    outs = [pkg.empty(tuple(ct.shape)) for _ in exps]
+    pkg.rotate_hoisted_batch(ctx, [(hoisted, keys[i], e, ct, o) for (i, e), o in zip(exps, outs)])
+    for (i, e), o in zip(exps, outs):
+        want = keys[i].apply_galois(ct, e)
+        assert torch.equal(o, want), f"batch exponent {e}"
+        assert torch.equal(keys[i].rotate_hoisted(hoisted, ct, e), want), f"exponent {e}"

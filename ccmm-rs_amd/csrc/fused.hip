@@ -444,12 +444,10 @@ __device__ __forceinline__ RowBlock row_block(const RowGrid &g, u32 b) {
 // ---- key inner product ------------------------------------------------------------
 
 struct RowMacArgs {
-    const u64 *digits;   // [limb][ct][j][N], forward column pass output
-    const u64 *kb, *ka;  // [dnum][limbs][N]
-    u64 *out;            // [limb][ct][2][N], input of the inverse column pass
+    RowMacJob e[kRowJobs];
     const DevPrime *primes;
-    RowGrid grid;
-    u32 dnum;
+    RowGrid grid;  // n_cts: of all jobs
+    u32 dnum, count;
 };
 
 // Two sums per residue, 64 bits each.
@@ -578,8 +576,12 @@ struct RowMacBody {
         const u32 off0 = R::internal_off(blk.tile, n1, tid, 0) * 8;
         const u32 nat0 = R::natural_off(blk.tile, n1, tid, 0) * 8;
         const u32 D = a.dnum;
-        const u64 *src = a.digits + ((u64)blk.limb * a.grid.n_cts + blk.ct) * D * N;
-        const u64 *kb = a.kb + (u64)blk.limb * N, *ka = a.ka + (u64)blk.limb * N;
+        u32 job = 0;
+        while (job + 1 < a.count && blk.ct >= a.e[job + 1].first) ++job;
+        const RowMacJob &e = a.e[job];
+        const u64 poly = (u64)blk.limb * e.n_cts + (blk.ct - e.first);
+        const u64 *src = e.digits + poly * D * N;
+        const u64 *kb = e.kb + (u64)blk.limb * N, *ka = e.ka + (u64)blk.limb * N;
         const u64 kstride = (u64)a.grid.limbs * N;
         typename Sum::S sb[8], sa[8];
 #pragma unroll
@@ -641,7 +643,7 @@ struct RowMacBody {
             }
         }
         tid = opaque(tid);
-        u64 *out = a.out + ((u64)blk.limb * a.grid.n_cts + blk.ct) * 2 * N;
+        u64 *out = e.out + poly * 2 * N;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
 #pragma unroll
@@ -666,17 +668,21 @@ __global__ __launch_bounds__(512, 4) void k_row_mac(RowMacArgs a) {
         RowMacBody<L, RowInt, SumInt>{a, P, RowInt{P.q}, SumInt(P), lds, threadIdx.x}.run(blk);
 }
 
-int launch_row_mac(ckks_context *ctx, const RowMac &m) {
+int launch_row_mac(ckks_context *ctx, RowMac &m) {
     if (!fused_rows_apply(m.plan)) return fail(CKKS_ERR_UNSUPPORTED, "fused row passes: 2^13 <= N <= 2^17, primes below 2^60");
+    if (m.count == 0 || m.count > kRowJobs) return fail(CKKS_ERR_INVALID, "1..16 key switches a launch");
     RowMacArgs a{};
-    a.digits = m.digits;
-    a.kb = m.kb;
-    a.ka = m.ka;
-    a.out = m.out;
+    size_t n_cts = 0;
+    for (size_t i = 0; i < m.count; ++i) {
+        m.e[i].first = (u32)n_cts;
+        a.e[i] = m.e[i];
+        n_cts += m.e[i].n_cts;
+    }
+    a.count = (u32)m.count;
     a.primes = m.plan->d_primes;
-    a.grid = row_grid(m.plan, m.limbs, m.n_cts, m.xcd_order);
+    a.grid = row_grid(m.plan, m.limbs, n_cts, m.xcd_order);
     a.dnum = (u32)m.dnum;
-    if ((u64)m.limbs * m.n_cts << (m.plan->logn - 12) >= (1ull << 30))
+    if ((u64)m.limbs * n_cts << (m.plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "key-switch batch too large for one launch");
     const dim3 g(row_blocks(a.grid)), t(512);
     switch (ntt_n2(m.plan->logn)) {

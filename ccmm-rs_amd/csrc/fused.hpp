@@ -57,19 +57,24 @@ struct ColCall {
 };
 int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward);
 
-// Key inner product between the column passes of a key switch: the forward
-// row pass of the digits, the products with the key and the inverse row pass
-// of both sums.  digits: inter-pass, polynomials [ct][j]; out: inter-pass,
-// polynomials [ct][2].
+// Key inner products between the column passes of key switches by up to
+// kRowJobs keys of one shape: the forward row pass of the digits, the products
+// with the key and the inverse row pass of both sums.
+constexpr size_t kRowJobs = 16;
+struct RowMacJob {
+    const u64 *digits;   // inter-pass, polynomials [ct][j]
+    const u64 *kb, *ka;  // [dnum][limbs][N], NTT domain, natural order
+    u64 *out;            // inter-pass, polynomials [ct][2]
+    u32 n_cts, first;    // first: set by the launch
+};
 struct RowMac {
     const ckks_rns_plan *plan;
-    const u64 *digits;
-    const u64 *kb, *ka;  // [dnum][limbs][N], NTT domain, natural order
-    u64 *out;
-    size_t n_cts, dnum, limbs;
+    size_t dnum, limbs;
     bool xcd_order;  // ciphertexts of one key tile on one XCD
+    size_t count;
+    RowMacJob e[kRowJobs];
 };
-int launch_row_mac(ckks_context *ctx, const RowMac &m);
+int launch_row_mac(ckks_context *ctx, RowMac &m);
 
 // Products between the column passes, in place of the first operand's
 // inter-pass data (n_polys polynomials of `limbs` limbs).

@@ -314,10 +314,27 @@ __global__ __launch_bounds__(kKsThreads) void k_modup(ModUpArgs a, u32 j_first, 
 // The mixed-radix digits alone, [ct][q_limbs][N] in the block's limb order: what
 // the fused column pass evaluates at every limb (kColBlock).  Same digits as
 // modup_thread's FP64 modes; one launch for blocks of every size up to AMAX.
-struct GarnerArgs {
+// Batches of keys of one shape that share a launch: ciphertexts are numbered
+// through, entry i holding those from e[i].first on.
+constexpr size_t kKsJobs = 16;
+
+template <class Args>
+__device__ __forceinline__ u32 job_of(const Args &a, u32 ct) {
+    u32 i = 0;
+    while (i + 1 < a.count && ct >= a.e[i + 1].first) ++i;
+    return i;
+}
+
+struct GarnerJob {
     const u64 *in;  // as ModUpArgs
     u64 in_stride, kinv;
     u64 *out;       // [ct][q_limbs][N]
+    u64 first;
+};
+
+struct GarnerArgs {
+    GarnerJob e[kKsJobs];
+    u32 count;
     const ModUpBlock *blocks;
     const DevPrime *primes;
     u32 dnum, q_limbs, logn, chunks;
@@ -328,9 +345,11 @@ __device__ __forceinline__ void garner_thread(const GarnerArgs &a, const CK_CONS
     const u64 N = (u64)1 << a.logn;
     const CK_CONST_AS DevPrime *primes = const_table(a.primes);
     const u32 start = blk->start;
-    const Gather gi = galois_gather(n, a.kinv, a.logn);
-    const u64 *src = a.in + ct * a.in_stride + (u64)start * N + gi.idx;
-    u64 *dst = a.out + ((u64)ct * a.q_limbs + start) * N + n;
+    const GarnerJob &e = a.e[job_of(a, ct)];
+    ct -= (u32)e.first;
+    const Gather gi = galois_gather(n, e.kinv, a.logn);
+    const u64 *src = e.in + ct * e.in_stride + (u64)start * N + gi.idx;
+    u64 *dst = e.out + ((u64)ct * a.q_limbs + start) * N + n;
     u64 x[A];
 #pragma unroll
     for (int m = 0; m < A; ++m) {
@@ -886,13 +905,19 @@ __global__ __launch_bounds__(kKsThreads) void k_ks_mac_any(MacArgs a) {
 
 // ---- 5. ModDown / finalize ---------------------------------------------------------
 
-struct DownArgs {
+struct DownJob {
     const u64 *acc;  // [ct][2][B][N] coefficient domain
     const u64 *add0, *add1;  // pass-through for component 0 / 1 (may be null)
     u64 add_stride;
     u64 kinv;  // nonzero: component 0 pass-through is sigma_k(add0)
     u64 *out;  // [ct][2][q_limbs][N] with out_stride
     u64 out_stride;
+    u64 first;
+};
+
+struct DownArgs {
+    DownJob e[kKsJobs];
+    u32 count;
     const ModDownTable *md;  // null: no special primes
     const DevPrime *primes;  // key basis
     u64 fp_targets;  // bit i: Q limb i takes the FP64 target path
@@ -905,15 +930,17 @@ __global__ __launch_bounds__(kKsThreads) void k_moddown(DownArgs a) {
     const u32 b = xcd_contiguous_block(blockIdx.x, gridDim.x);
     const u32 chunk = b % a.chunks;
     const u32 rest = b / a.chunks;
-    const u32 comp = rest % 2, ct = rest / 2;
+    const u32 comp = rest % 2;
+    const DownJob &e = a.e[job_of(a, rest / 2)];
+    const u32 ct = rest / 2 - (u32)e.first;
     const u64 N = (u64)1 << a.logn;
     const u64 n = (u64)chunk * kKsThreads + threadIdx.x;
     const CK_CONST_AS DevPrime *primes = const_table(a.primes);
-    const u64 *x = a.acc + ((u64)ct * 2 + comp) * a.limbs * N + n;
-    const u64 *add = comp == 0 ? a.add0 : a.add1;
-    const Gather ga = galois_gather(n, comp == 0 ? a.kinv : 0, a.logn);
-    if (add) add += ct * a.add_stride + ga.idx;
-    u64 *o = a.out + ct * a.out_stride + (u64)comp * a.q_limbs * N + n;
+    const u64 *x = e.acc + ((u64)ct * 2 + comp) * a.limbs * N + n;
+    const u64 *add = comp == 0 ? e.add0 : e.add1;
+    const Gather ga = galois_gather(n, comp == 0 ? e.kinv : 0, a.logn);
+    if (add) add += ct * e.add_stride + ga.idx;
+    u64 *o = e.out + ct * e.out_stride + (u64)comp * a.q_limbs * N + n;
     if (K == 0) {
         for (u32 i = 0; i < a.q_limbs; ++i) {
             u64 v = x[(u64)i * N];
@@ -1175,6 +1202,7 @@ __global__ __launch_bounds__(256) void k_moddown_mfma(ModDownMfmaArgs args) {
     __shared__ int lds_e[4][64 * 33];
     __shared__ unsigned char lds_neg[kBcRows];
     const DownArgs &a = args.base;
+    const DownJob &job = a.e[0];
     const BcPlan &bp = *args.plan;
     const ModDownTable &md = *a.md;
     const u32 N = 1u << a.logn;
@@ -1183,7 +1211,7 @@ __global__ __launch_bounds__(256) void k_moddown_mfma(ModDownMfmaArgs args) {
     const u32 chunk = b % chunks, rest = b / chunks;
     const u32 comp = rest % 2, ct = rest / 2;
     const u32 tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const u64 *x = a.acc + ((u64)ct * 2 + comp) * a.limbs * N;
+    const u64 *x = job.acc + ((u64)ct * 2 + comp) * a.limbs * N;
     // ---- P-side mixed-radix digits and the centering decision (VALU)
     {
         const u64 n = (u64)chunk * kBcRows + tid;
@@ -1210,11 +1238,11 @@ __global__ __launch_bounds__(256) void k_moddown_mfma(ModDownMfmaArgs args) {
         bc_store_row<K>(c, lds_a + tid * KR);
     }
     __syncthreads();
-    const u64 *add = comp == 0 ? a.add0 : a.add1;
+    const u64 *add = comp == 0 ? job.add0 : job.add1;
     const u64 row_n = (u64)chunk * kBcRows + wave * 64 + lane;
-    const Gather ga = galois_gather(row_n, comp == 0 ? a.kinv : 0, a.logn);
-    if (add) add += ct * a.add_stride + ga.idx;
-    u64 *o = a.out + ct * a.out_stride + (u64)comp * a.q_limbs * N + row_n;
+    const Gather ga = galois_gather(row_n, comp == 0 ? job.kinv : 0, a.logn);
+    if (add) add += ct * job.add_stride + ga.idx;
+    u64 *o = job.out + ct * job.out_stride + (u64)comp * a.q_limbs * N + row_n;
     const bool neg = lds_neg[wave * 64 + lane] != 0;
     int *e = lds_e[wave];
     for (u32 tile = 0; tile < bp.n_tiles; ++tile) {
@@ -2023,20 +2051,51 @@ static int ks_mac_group(const std::vector<KsJob> &jobs, const std::vector<size_t
     return CKKS_OK;
 }
 
-// 5. ModDown (or plain finalize) of the coefficient-domain accumulators
-// with the pass-through adds
-static int ks_moddown(const KsJob &j, hipStream_t s) {
-    const ckks_ksk *k = j.k;
+// Jobs that may share a launch: every table of their keys but the entries
+// themselves is the same.
+static bool ks_same_shape(const KsJob &a, const KsJob &b) {
+    const ckks_ksk *x = a.k, *y = b.k;
+    return a.mfma == b.mfma && x->plan == y->plan && x->q_limbs == y->q_limbs && x->limbs == y->limbs && x->dnum == y->dnum &&
+           x->block_size == y->block_size && x->bounded == y->bounded && x->base_log == y->base_log;
+}
+
+// Runs launch(group) over the jobs (in[i]), up to kKsJobs of one shape at a time.
+template <class Launch>
+static int ks_by_shape(const KsJob *const *in, size_t count, const Launch &launch) {
+    std::vector<bool> done(count, false);
+    for (size_t i = 0; i < count; ++i) {
+        if (done[i]) continue;
+        std::vector<size_t> grp;
+        for (size_t m = i; m < count && grp.size() < kKsJobs; ++m)
+            if (!done[m] && ks_same_shape(*in[i], *in[m])) {
+                grp.push_back(m);
+                done[m] = true;
+            }
+        if (int rc = launch(grp)) return rc;
+    }
+    return CKKS_OK;
+}
+
+// 5. ModDown (or plain finalize) of the coefficient-domain accumulators of
+// jobs of one shape, with the pass-through adds
+static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
+    const ckks_ksk *k = jobs[0]->k;
     const u64 N = k->degree, B = k->limbs, D = k->dnum;
     const u32 chunks = (u32)(N / kKsThreads);
+    if (jobs[0]->mfma && count > 1) {
+        for (size_t i = 0; i < count; ++i)
+            if (int rc = ks_moddown(jobs + i, 1, s)) return rc;
+        return CKKS_OK;
+    }
     DownArgs da{};
-    da.acc = j.acc;
-    da.add0 = ks_mac_takes_b(j) ? nullptr : j.add0;
-    da.add1 = j.add1;
-    da.add_stride = j.add_stride;
-    da.kinv = j.galois_kinv;
-    da.out = j.out;
-    da.out_stride = j.out_stride;
+    size_t n_cts = 0;
+    for (size_t i = 0; i < count; ++i) {
+        const KsJob &j = *jobs[i];
+        da.e[i] = DownJob{j.acc, ks_mac_takes_b(j) ? nullptr : j.add0, j.add1, j.add_stride, j.galois_kinv, j.out,
+                          j.out_stride, n_cts};
+        n_cts += j.n_cts;
+    }
+    da.count = (u32)count;
     da.md = k->d_moddown;
     da.primes = k->plan->d_primes;
     da.fp_targets = k->fp_q_targets;
@@ -2045,10 +2104,10 @@ static int ks_moddown(const KsJob &j, hipStream_t s) {
     da.q_limbs = (u32)k->q_limbs;
     da.logn = k->plan->logn;
     da.chunks = chunks;
-    dim3 g((u32)(j.n_cts * 2 * chunks));
-    if (j.mfma) {
+    dim3 g((u32)(n_cts * 2 * chunks));
+    if (jobs[0]->mfma) {
         ModDownMfmaArgs dm{da, k->d_bc + D};
-        dim3 gm((u32)(j.n_cts * 2 * (N / kBcRows)));
+        dim3 gm((u32)(n_cts * 2 * (N / kBcRows)));
         switch (k->p_limbs) {
 #define CK_MDM(KK) \
     case KK: hipLaunchKernelGGL(k_moddown_mfma<KK>, gm, dim3(256), 0, s, dm); break;
@@ -2068,6 +2127,19 @@ static int ks_moddown(const KsJob &j, hipStream_t s) {
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
+}
+
+static int ks_moddown(const KsJob &j, hipStream_t s) {
+    const KsJob *jp = &j;
+    return ks_moddown(&jp, 1, s);
+}
+
+static int ks_moddown_all(const KsJob *const *jobs, size_t count, hipStream_t s) {
+    return ks_by_shape(jobs, count, [&](const std::vector<size_t> &grp) {
+        const KsJob *jp[kKsJobs];
+        for (size_t g = 0; g < grp.size(); ++g) jp[g] = jobs[grp[g]];
+        return ks_moddown(jp, grp.size(), s);
+    });
 }
 
 // With CKKS_KS_FUSION_INVERSE set on the context, hoisted rotations of
@@ -2124,11 +2196,23 @@ static ColKind ks_lift(const ckks_ksk *k, size_t n_cts) {
     return most >= kLiftInHbmBlock && lifted > kLiftInHbmBytes ? kColPlain : kColBlock;
 }
 
-static int launch_garner(const ckks_ksk *k, const u64 *in, u64 in_stride, u64 kinv, u64 *out, size_t n_cts,
-                         hipStream_t s) {
+static int launch_garner(const KsJob *const *jobs, size_t count, hipStream_t s) {
+    const ckks_ksk *k = jobs[0]->k;
     const u32 chunks = (u32)(k->degree / kKsThreads);
-    const GarnerArgs a{in, in_stride, kinv, out, k->d_modup, k->plan->d_primes, (u32)k->dnum, (u32)k->q_limbs,
-                       k->plan->logn, chunks};
+    GarnerArgs a{};
+    size_t n_cts = 0;
+    for (size_t i = 0; i < count; ++i) {
+        const KsJob &j = *jobs[i];
+        a.e[i] = GarnerJob{j.x, j.x_stride, j.galois_kinv, j.digits, n_cts};
+        n_cts += j.n_cts;
+    }
+    a.count = (u32)count;
+    a.blocks = k->d_modup;
+    a.primes = k->plan->d_primes;
+    a.dnum = (u32)k->dnum;
+    a.q_limbs = (u32)k->q_limbs;
+    a.logn = k->plan->logn;
+    a.chunks = chunks;
     size_t most = 0;
     for (size_t z : k->block_size) most = std::max(most, z);
     const dim3 g((u32)(n_cts * k->dnum * chunks)), t(kKsThreads);
@@ -2154,6 +2238,7 @@ static size_t ks_digit_residues(const ckks_ksk *k, size_t n_cts) {
 // the digit buffer, inverse column pass into the accumulators.
 static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t count, u64 *cols) {
     std::vector<ColCall> fwd(count), inv(count);
+    std::vector<const KsJob *> garner;
     u64 *c = cols;
     int rc = CKKS_OK;
     for (size_t i = 0; i < count && !rc; ++i) {
@@ -2178,7 +2263,7 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
             f.digits = D;
             f.stride = k->q_limbs * N;
             f.blocks = k->d_col;
-            rc = launch_garner(k, j.x, j.x_stride, j.galois_kinv, j.digits, j.n_cts, ctx->stream);
+            garner.push_back(&j);
         } else {
             if (f.kind == kColDigit) {
                 f.digits = D;
@@ -2190,13 +2275,23 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
         inv[i] = ColCall{k->plan, j.digits, j.acc, j.n_cts * 2, B, B * N};
         c += j.n_cts * D * B * N;
     }
+    if (!rc)
+        rc = ks_by_shape(garner.data(), garner.size(), [&](const std::vector<size_t> &grp) {
+            const KsJob *jp[kKsJobs];
+            for (size_t g = 0; g < grp.size(); ++g) jp[g] = garner[grp[g]];
+            return launch_garner(jp, grp.size(), ctx->stream);
+        });
     if (!rc) rc = launch_columns(ctx, fwd.data(), count, true);
-    for (size_t i = 0; i < count && !rc; ++i) {
-        const KsJob &j = *jobs[i];
-        const RowMac m{j.k->plan, fwd[i].out, j.k->d_kb, j.k->d_ka, j.digits, j.n_cts, j.k->dnum, j.k->limbs,
-                       ks_fusion(j.k) == CKKS_KS_FUSION_XCD};
-        rc = launch_row_mac(ctx, m);
-    }
+    if (!rc)
+        rc = ks_by_shape(jobs, count, [&](const std::vector<size_t> &grp) {
+            const ckks_ksk *k = jobs[grp[0]]->k;
+            RowMac m{k->plan, k->dnum, k->limbs, ks_fusion(k) == CKKS_KS_FUSION_XCD, grp.size()};
+            for (size_t g = 0; g < grp.size(); ++g) {
+                const KsJob &j = *jobs[grp[g]];
+                m.e[g] = RowMacJob{fwd[grp[g]].out, j.k->d_kb, j.k->d_ka, j.digits, (u32)j.n_cts, 0};
+            }
+            return launch_row_mac(ctx, m);
+        });
     return rc ? rc : launch_columns(ctx, inv.data(), count, false);
 }
 
@@ -2361,9 +2456,9 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
     for (size_t i = 0; i < count; ++i)
         if (!ks_fused(e[i].k) && (rc = ks_mac(jobs[i], s))) return rc;
     if ((rc = launch_ntt(ctx, back.data(), back.size(), false))) return rc;
-    for (size_t i = 0; i < count; ++i)
-        if ((rc = ks_moddown(jobs[i], s))) return rc;
-    return CKKS_OK;
+    std::vector<const KsJob *> all(count);
+    for (size_t i = 0; i < count; ++i) all[i] = &jobs[i];
+    return ks_moddown_all(all.data(), count, s);
 }
 
 size_t ksk_bytes(const ckks_ksk *k) {
@@ -2533,9 +2628,10 @@ int ckks_mod_down(const ckks_rns_plan *qp_plan, size_t q_limbs, const uint64_t *
     }
     const size_t N = qp_plan->degree;
     DownArgs da{};
-    da.acc = in;
-    da.out = out;
-    da.out_stride = 2 * q_limbs * N;  // polynomials are consecutive [p][q_limbs][N]
+    da.count = 1;
+    da.e[0].acc = in;
+    da.e[0].out = out;
+    da.e[0].out_stride = 2 * q_limbs * N;  // polynomials are consecutive [p][q_limbs][N]
     da.md = (const ModDownTable *)it->second.second;
     da.primes = qp_plan->d_primes;
     da.fp_targets = fp_target_mask(qp_plan->moduli, q_limbs);
@@ -3258,9 +3354,9 @@ int ckks_rotate_hoisted_batch(ckks_context *ctx, const ckks_hoisted_rotation *e,
     for (size_t i = 0; i < fast.size(); ++i)
         if (!ks_fused(fast[i].key)) rest.push_back(inv[i]);
     if (!rest.empty() && (rc = launch_ntt(ctx, rest.data(), rest.size(), false))) return rc;
-    for (KsJob &j : jobs)
-        if ((rc = ks_moddown(j, s))) return rc;
-    return CKKS_OK;
+    std::vector<const KsJob *> all;
+    for (const KsJob &j : jobs) all.push_back(&j);
+    return ks_moddown_all(all.data(), all.size(), s);
 }
 
 int ckks_relinearize(const ckks_ksk *key, const uint64_t *in3, uint64_t *out, size_t n_cts,

@@ -13,7 +13,7 @@ import ctypes as C
 from dataclasses import dataclass, field
 from typing import Optional
 
-from . import PreparedRnsNttPlan, _check, _p, _ptr, _sz, lib
+from . import GaloisBatchEntry, NttBatchEntry, PreparedRnsNttPlan, _check, _p, _ptr, _sz, lib
 
 OP_ROTATE, OP_MUL_PLAIN, OP_ADD, OP_RESCALE, OP_MUL_RELIN_RESCALE, OP_COPY, OP_MOD_SWITCH, OP_SUB = 1, 2, 3, 4, 5, 6, 7, 8
 OP_NTT, OP_INTT, OP_MAC_PLAIN = 9, 10, 11
@@ -253,16 +253,160 @@ class Server:
             pass
 
 
+_LEVEL_DROP = (OP_RESCALE, OP_MOD_SWITCH, OP_MUL_RELIN_RESCALE)
+_TOGETHER = 16  # rotations or transforms of one library call
+
+
+@dataclass
+class _Value:
+    """One result of a program: the registers' contents over time."""
+    limbs: int
+    reads: int = 0    # ops that still read it
+    home: int = -1    # the register whose row it has to end in (-1: any)
+    row: int = -1
+
+
+def schedule(prog: Program, n_limbs: int, spare: int):
+    """Groups of independent ops of one kind, in an order that gives every op
+    the values it reads in program order.  Every op writes a row of its own
+    (a register reused for unrelated results orders nothing), out of n_regs +
+    2 + spare rows; copies only rename.  Ops behind the oldest unfinished one
+    hold at most `spare` rows, so the oldest always finds one: the values that
+    program order keeps alive take n_regs rows at most.
+
+    Returns (groups, rows used): a group is (code, limbs, [(out row, [input
+    rows], op)]), code OP_COPY for the final moves of registers whose contents
+    outlive the run (the output, and what the program reads before writing)."""
+    n = prog.n_regs
+    cur = [_Value(n_limbs if i < prog.n_inputs else 0, row=i) for i in range(n)]
+    first = list(cur)
+    written, carried = set(), {prog.out_reg}
+    todo = []  # [op index, code, inputs, output, waits, dependants]
+    source = {}
+    for i, op in enumerate(prog.ops):
+        code, dst, a, b = op[:4]
+        regs = list(range(a, a + b)) if code == OP_MAC_PLAIN else \
+            [a, b] if code in (OP_ADD, OP_SUB, OP_MUL_RELIN_RESCALE) else [a]
+        carried.update(r for r in regs if r not in written)
+        written.add(dst)
+        if code == OP_COPY:
+            cur[dst] = cur[a]
+            continue
+        ins = [cur[r] for r in regs]
+        out = _Value(ins[0].limbs - (1 if code in _LEVEL_DROP else 0))
+        node = [i, code, ins, out, 0, []]
+        for v in {id(v): v for v in ins}.values():
+            if id(v) in source:
+                source[id(v)][5].append(node)
+                node[4] += 1
+        for v in ins:
+            v.reads += 1
+        source[id(out)] = node
+        cur[dst] = out
+        todo.append(node)
+    final = [(r, cur[r]) for r in sorted(carried)]
+    for r, v in final:
+        v.reads += 1  # by the end of the run
+        if v.home < 0:
+            v.home = r
+
+    free = set(range(n + 2 + spare)) - {v.row for v in first if v.reads}
+    used = n
+    groups = []
+    ready = [t for t in todo if t[4] == 0]
+    done, oldest = set(), 0
+    early = {}  # rows of results behind the oldest unfinished op -> their op
+
+    def place(t):
+        """Row of t's output, or None."""
+        code, ins, out = t[1], t[2], t[3]
+        if code in (OP_NTT, OP_INTT, OP_ADD, OP_SUB, OP_MUL_PLAIN) and ins[0].reads == 1 and ins[0].limbs:
+            return ins[0].row  # in place: nothing else reads it
+        if not free:
+            return None
+        if out.home in free:
+            return out.home
+        return min(free, key=lambda r: (r < n, r))
+
+    while oldest < len(todo):
+        kinds = {}
+        for t in ready:
+            kinds.setdefault((t[1], t[2][0].limbs), []).append(t)
+        # the fullest group first: what waits on it is then ready together
+        members = max(kinds.values(), key=lambda g: (len(g), -g[0][0]))
+        group = []
+        for attempt in (members, [todo[oldest]]):
+            for t in sorted(attempt, key=lambda t: t[0])[:_TOGETHER]:
+                row = place(t)
+                if row is None or (t is not todo[oldest] and row not in early and len(early) >= spare):
+                    break
+                t[3].row = row
+                free.discard(row)
+                used = max(used, row + 1)
+                early[row] = t[0]
+                group.append(t)
+            if group:
+                break
+        groups.append((group[0][1], group[0][2][0].limbs,
+                       [(t[3].row, [v.row for v in t[2]], prog.ops[t[0]]) for t in group]))
+        for t in group:
+            done.add(t[0])
+            ready.remove(t)
+            for v in t[2]:
+                v.reads -= 1
+                if v.reads == 0 and all(u[3].row != v.row for u in group):
+                    free.add(v.row)
+                    early.pop(v.row, None)
+            if t[3].reads == 0:  # written for nobody: the row is free again
+                free.add(t[3].row)
+                early.pop(t[3].row, None)
+            for d in t[5]:
+                d[4] -= 1
+                if d[4] == 0:
+                    ready.append(d)
+        while oldest < len(todo) and todo[oldest][0] in done:
+            oldest += 1
+        if oldest < len(todo):
+            early = {r: i for r, i in early.items() if i >= todo[oldest][0]}
+    # the registers that outlive the run move to their own rows
+    moves = []
+    at = {r: v.row for r, v in final}
+    for r, _ in final:
+        if at[r] == r:
+            continue
+        for q in at:
+            if q != r and at[q] == r:  # another one sits there: aside first
+                aside = next(x for x in range(n + 2 + spare) if x not in at.values() and x not in at)
+                moves.append((aside, [r], (OP_COPY, q, r, 0, None, 0, None)))
+                used = max(used, aside + 1)
+                for z in at:
+                    if at[z] == r:
+                        at[z] = aside
+        moves.append((r, [at[r]], (OP_COPY, r, at[r], 0, None, 0, None)))
+        at[r] = r
+    for m in moves:
+        groups.append((OP_COPY, n_limbs, [m]))
+    return groups, used
+
+
 class ProgramRunner:
-    """Runs one Program directly -- one library call per op on registers it
-    owns -- outside the serving loop, so that a whole rotation schedule can
-    be captured once as a hipGraph (capture()) and replayed (replay())
-    without per-op host work.  Registers hold compact [2][limbs][N]
+    """Runs one Program directly on registers it owns, outside the serving
+    loop, so that a whole rotation schedule can be captured once as a hipGraph
+    (capture()) and replayed (replay()) without per-op host work.  Independent
+    rotations and transforms go out together, one library call for up to 16
+    of them (schedule): a baby-step / giant-step request at N = 2^14 is 30
+    rotations of one ciphertext, whose kernels each fill a third of the chip
+    one at a time (256 x 256, 8 limbs: 3.06 ms one by one, 0.75 ms).  Registers hold compact [2][limbs][N]
     ciphertexts at their current level (as the server's).  The program's
     keys must belong to the plan's context; each run switches that context
     to the runner's own (non-null, default-priority) stream and back, which
     waits for the run.  The first run() sizes every library workspace, so
     run() must precede capture(); nothing is allocated while capturing."""
+
+    # rows of results that wait for others of their kind, and the library's
+    # workspaces per group grow with them: bounded at large degrees, where a
+    # single rotation fills the chip
+    _SPARE_BYTES = 512 << 20
 
     def __init__(self, plan: PreparedRnsNttPlan, n_limbs: int, program: Program, stream=None):
         import torch
@@ -272,11 +416,16 @@ class ProgramRunner:
         self.L = int(n_limbs)
         n = plan.degree
         self.per = 2 * self.L * n
-        # two extra registers: the output of ops that cannot run in place
-        self.regs = torch.empty((program.n_regs + 2, self.per), dtype=torch.int64, device="cuda")
-        self.tmp = program.n_regs
+        self.spare = max(0, min(2 * _TOGETHER, self._SPARE_BYTES // (8 * self.per) - 1))
         self.limbs = program.register_limbs(self.L)
+        self._plan_ops()
+        self.regs = torch.empty((max(self.rows, program.n_regs + 2), self.per), dtype=torch.int64, device="cuda")
         self.graph = None
+
+    def _plan_ops(self):
+        self.groups, self.rows = schedule(self.prog, self.L, self.spare)
+        self.planned = len(self.prog.ops)
+        self.calls = None
 
     def _reg(self, i, limbs):
         return self.regs[i, : 2 * limbs * self.plan.degree]
@@ -284,44 +433,82 @@ class ProgramRunner:
     def _ct(self, i, limbs):
         return self._reg(i, limbs).view(1, 2, limbs, self.plan.degree)
 
-    def _run_ops(self):
-        plan, n = self.plan, self.plan.degree
-        regs = [self.L if i < self.prog.n_inputs else 0 for i in range(self.prog.n_regs)]
-        for (code, dst, a, b, key, exp, pt) in self.prog.ops:
-            la = regs[a]
-            out_l = la - 1 if code in (OP_RESCALE, OP_MOD_SWITCH, OP_MUL_RELIN_RESCALE) else la
-            # ops whose output may not alias an input write the spare register
-            spare = code in (OP_ROTATE, OP_RESCALE, OP_MOD_SWITCH, OP_MUL_RELIN_RESCALE) and \
-                (dst == a or (code == OP_MUL_RELIN_RESCALE and dst == b))
-            d = self.tmp if spare else dst
-            if code == OP_ROTATE:
-                key.apply_galois(self._ct(a, la), exp, out=self._ct(d, la))
+    def _call(self, code, la, items):
+        """The library call of one group as a function without arguments."""
+        plan, ctx, n = self.plan, self.ctx, self.plan.degree
+        if code == OP_ROTATE:
+            keys = [op[4] for _, _, op in items]
+            arr = (GaloisBatchEntry * len(items))()
+            for e, (out, (a,), op) in zip(arr, items):
+                key = op[4]
+                p_ct, p_out = key._ct_ptrs(1, [("ct", self._ct(a, la), 2)], self._ct(out, la))
+                e.exponent, e.input, e.output, e.n_cts = op[5], p_ct, p_out, 1
+            ptr = C.cast(arr, _p)
+
+            def rotate():
+                for e, key in zip(arr, keys):
+                    e.key = key.handle
+                _check(lib().ckks_apply_galois_batch(ctx.handle, ptr, len(arr)))
+            return rotate
+        if code in (OP_NTT, OP_INTT):
+            arr = (NttBatchEntry * len(items))()
+            for e, (out, (a,), _) in zip(arr, items):
+                p_in, p_out = (_ptr(self._reg(i, la)) for i in (a, out))
+                e.input, e.output, e.n_polys, e.n_limbs, e.poly_stride = p_in, p_out, 2, la, la * n
+            ptr = C.cast(arr, _p)
+
+            def transform():
+                for e in arr:
+                    e.plan = plan.handle
+                fn = lib().ckks_ntt_forward_batch if code == OP_NTT else lib().ckks_ntt_inverse_batch
+                _check(fn(ctx.handle, ptr, len(arr)))
+            return transform
+        steps = []
+        for out, ins, op in items:
+            _, _, _, _, key, _, pt = op
+            if code == OP_MAC_PLAIN:
+                if not ins or len(ins) != len(pt):
+                    raise ValueError("one plaintext per ciphertext, at least one term")
+                ca = (C.c_uint64 * len(ins))(*[_ptr(self._reg(i, la)) for i in ins])
+                pa = (C.c_uint64 * len(ins))(*[_ptr(t, la * n, name="pt") for t in pt])
+
+                def step(ca=ca, pa=pa, out=_ptr(self._reg(out, la))):
+                    _check(lib().ckks_multiply_plain_accumulate_ntt(plan.handle, C.cast(ca, _p), C.cast(pa, _p),
+                                                                    len(ca), out, la))
             elif code == OP_MUL_PLAIN:
-                plan.multiply_plain(self._ct(a, la), pt, la, out=self._ct(d, la))
+                def step(x=self._ct(ins[0], la), pt=pt, out=self._ct(out, la)):
+                    plan.multiply_plain(x, pt, la, out=out)
             elif code in (OP_ADD, OP_SUB):
-                (plan.add if code == OP_ADD else plan.sub)(self._reg(a, la), self._reg(b, la),
-                                                           out=self._reg(d, la), n_limbs=la)
-            elif code == OP_RESCALE:
-                plan.rescale_to_next(self._ct(a, la), la, out=self._ct(d, out_l))
-            elif code == OP_MOD_SWITCH:
-                plan.mod_switch_to_next(self._ct(a, la), la, out=self._ct(d, out_l))
+                def step(fn=plan.add if code == OP_ADD else plan.sub, x=self._reg(ins[0], la),
+                         y=self._reg(ins[1], la), out=self._reg(out, la)):
+                    fn(x, y, out=out, n_limbs=la)
+            elif code in (OP_RESCALE, OP_MOD_SWITCH):
+                def step(fn=plan.rescale_to_next if code == OP_RESCALE else plan.mod_switch_to_next,
+                         x=self._ct(ins[0], la), out=self._ct(out, la - 1)):
+                    fn(x, la, out=out)
             elif code == OP_MUL_RELIN_RESCALE:
-                key.multiply_relinearize_rescale(self._ct(a, la), self._ct(b, la), out=self._ct(d, out_l))
+                def step(key=key, x=self._ct(ins[0], la), y=self._ct(ins[1], la), out=self._ct(out, la - 1)):
+                    key.multiply_relinearize_rescale(x, y, out=out)
             elif code == OP_COPY:
-                if d != a:
-                    self._reg(d, la).copy_(self._reg(a, la))
-            elif code == OP_NTT:
-                plan.forward(self._reg(a, la), out=self._reg(d, la), n_limbs=la)
-            elif code == OP_INTT:
-                plan.inverse(self._reg(a, la), out=self._reg(d, la), n_limbs=la)
-            elif code == OP_MAC_PLAIN:
-                plan.multiply_plain_accumulate_ntt([self._reg(a + t, la) for t in range(b)], pt, la,
-                                                   out=self._reg(d, la))
+                def step(x=self.regs[ins[0]], out=self.regs[out]):
+                    out.copy_(x)
             else:
                 raise ValueError(f"unknown op code {code}")
-            if spare:
-                self._reg(dst, out_l).copy_(self._reg(self.tmp, out_l))
-            regs[dst] = out_l
+            steps.append(step)
+
+        def each():
+            for s in steps:
+                s()
+        return each
+
+    def _run_ops(self):
+        if self.planned != len(self.prog.ops):
+            self.spare = self.regs.shape[0] - self.prog.n_regs - 2
+            self._plan_ops()
+        if self.calls is None:
+            self.calls = [self._call(*g) for g in self.groups]
+        for call in self.calls:
+            call()
 
     def _on_stream(self):
         import contextlib

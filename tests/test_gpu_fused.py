@@ -139,3 +139,29 @@ def test_hoisted_rotations_match_rotations(pkg, ctx, logn, mix, with_b):
         want = keys[i].apply_galois(ct, e)
         assert torch.equal(o, want), f"batch exponent {e}"
         assert torch.equal(keys[i].rotate_hoisted(hoisted, ct, e), want), f"exponent {e}"
+
+
+def test_key_switch_batches_of_one_shape_share_launches(pkg, ctx):
+    """Interleaved keys of three shapes (one with single-limb blocks, one at
+    another level), uneven ciphertext counts, the most entries a call takes."""
+    import torch
+
+    n = 1 << 13
+    q = _moduli(pkg, n, [60, 40, 41, 36])
+    qp = q + pkg.find_ntt_primes(59, n, 2, skip=q)
+    rng = np.random.default_rng(5)
+    plan = pkg.PreparedRnsNttPlan(ctx, qp, n)
+    low = pkg.PreparedRnsNttPlan(ctx, q[:3] + qp[4:], n)
+    shapes = [(plan, 4, [2, 2]), (plan, 4, [1, 1, 1, 1]), (low, 3, [2, 1])]
+    entries = []
+    for i in range(16):
+        p, L, blocks = shapes[i % 3]
+        mods = qp if p is plan else q[:3] + qp[4:]
+        key = pkg.HybridKeySwitchKey(p, L, blocks, rand_residues(rng, mods, n, len(blocks)),
+                                     rand_residues(rng, mods, n, len(blocks)))
+        m = 1 + i % 4
+        ct = pkg.to_device(rand_residues(rng, mods[:L], n, 2 * m).reshape(m, 2, L, n))
+        entries.append((key, 2 * n - 1 if i == 7 else 5 ** i % (2 * n), ct, pkg.empty(tuple(ct.shape))))
+    pkg.apply_galois_batch(ctx, entries)
+    for i, (key, e, ct, out) in enumerate(entries):
+        assert torch.equal(out, key.apply_galois(ct, e)), f"entry {i}"

@@ -115,4 +115,22 @@ struct RowRotate {
 };
 int launch_row_rotate(ckks_context *ctx, const RowRotate &r);
 
+// Single-pass degrees (N <= 4096, every plan prime < 2^60; small.hip).
+bool small_tiles_apply(const ckks_rns_plan *plan);
+constexpr size_t kSmallJobs = 16;
+struct SmallCall {
+    const ckks_rns_plan *plan;
+    const u64 *in;
+    u64 *out;
+    size_t n_polys, n_limbs, in_stride, out_stride;
+    // nonzero: forward, the polynomials are the single-limb gadget digits of
+    // n_polys / digits ciphertexts (in_stride apart, sigma_k of them for kinv
+    // nonzero); inverse, they are the two key products of n_polys / 2
+    // ciphertexts' transformed digits [ct][digit][limb][N]
+    size_t digits = 0;
+    u64 kinv = 0;
+    const u64 *kb = nullptr, *ka = nullptr;
+};
+int launch_small(ckks_context *ctx, const SmallCall *calls, size_t count, bool forward);
+
 }  // namespace ck

@@ -94,6 +94,101 @@ struct BlockSum {
     }
 };
 
+// Input of limb prime P, largest bounds after it (see RowFp, RowInt):
+//   plain: canonical residues;
+//   residue: canonical modulo another prime of the plan (`limit`);
+//   digit: a balanced digit, |d| <= limit <= 2^62.
+// FP64 limbs take values up to 2^44 whole (with eight stages of 0.52 q they
+// stay below 2^45) and cut larger ones at bit 30; integer limbs take residues
+// up to 4q whole, add q to negative digits when limit < q, and reduce the rest
+// (below 2^64) into 3q.  Which of them is the same for a whole block.
+//   bytes: |d| <= 128, below every prime of a two-pass degree;
+//   block: a mixed-radix value, see col_blocks; within 0.54 q or below 2q.
+constexpr int kColFpIn = 16, kColIntIn = 4;
+constexpr u64 kColFpWhole = 1ull << 44;
+
+template <int M>
+__device__ __forceinline__ void col_lift(u64 (&v)[M], u32 kind, u64 limit, const RowFp &ar, const CK_CONST_AS DevPrime &) {
+    if (kind == kColPlain || limit <= kColFpWhole) {  // limit 0 for bytes
+#pragma unroll
+        for (int i = 0; i < M; ++i) v[i] = f64_as_u64(signed_to_f64(v[i]));
+        return;
+    }
+    const double k30 = fp_reduce(1073741824.0, ar.q, ar.qinv);
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        const double hi = signed_to_f64((u64)((int64_t)v[i] >> 30)), lo = (double)(u32)(v[i] & 0x3fffffffu);
+        v[i] = f64_as_u64(lo + fp_mulmod_q(hi, k30, ar.q, ar.qinv));
+        if ((i & 3) == 3) sched_fence();
+    }
+}
+template <int M>
+__device__ __forceinline__ void col_lift(u64 (&v)[M], u32 kind, u64 limit, const RowInt &ar, const CK_CONST_AS DevPrime &P) {
+    if (kind == kColInt8 || (kind == kColDigit && limit < ar.q)) {
+#pragma unroll
+        for (int i = 0; i < M; ++i) v[i] += (int64_t)v[i] < 0 ? ar.q : 0;
+    } else if (kind == kColDigit || (kind == kColResidue && limit > 4 * ar.q)) {
+        // a multiple of q from limit to limit + 2q makes every digit positive
+        const u64 up = kind == kColDigit ? (mulhi64(limit, P.br_hi) + 2) * ar.q : 0;
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+            v[i] = shoup_lazy3(v[i] + up, 1, P.br_hi, ar.q);
+            if ((i & 3) == 3) sched_fence();
+        }
+    }
+}
+
+// Two sums per residue, 64 bits each.
+//   FP64: products within 0.52 q, summed as doubles and reduced every 8 digits
+//     (below 2^45 throughout);
+//   integer: Montgomery products, two 32-bit steps.  With T = d k for a digit
+//     d < 16 q < 2^64 and a canonical key entry k, T < 2^124, each step adds
+//     the multiple m q that clears the lowest word and drops it: T / 2^64
+//     (mod q) below 2q.  Four of them and a reduced sum stay below 11 q; the
+//     factor 2^64 comes back with the last reduction, one product by 2^64 mod
+//     q.  (128-bit sums need no reduction per product but twice the registers,
+//     which then spill.)
+struct SumFp {
+    static constexpr int kIn = 1;  // bound of total()
+    double q, qinv;
+    typedef double S;
+    __device__ __forceinline__ void mac(S &s, u64 y, u64 w) const {
+        s += fp_mulmod_q(u64_as_f64(y), small_to_f64(w), q, qinv);
+    }
+    __device__ __forceinline__ static bool full(u32 j) { return (j & 7) == 7; }
+    __device__ __forceinline__ S reduced(S s) const { return fp_reduce(s, q, qinv); }
+    __device__ __forceinline__ u64 total(S s) const { return f64_as_u64(fp_reduce(s, q, qinv)); }
+};
+struct SumInt {
+    static constexpr int kIn = 3;
+    u64 q, r_hi, r_lo;  // modulus, floor(2^128 / q)
+    u32 qi;             // -q^-1 mod 2^32
+    typedef u64 S;
+    __device__ __forceinline__ SumInt(const CK_CONST_AS DevPrime &P) : q(P.q), r_hi(P.br_hi), r_lo(P.br_lo) {
+        u32 x = (u32)q;  // q q == 1 mod 8; each step doubles the correct bits
+#pragma unroll
+        for (int it = 0; it < 4; ++it) x *= 2u - (u32)q * x;
+        qi = 0u - x;
+    }
+    __device__ __forceinline__ void mac(S &s, u64 y, u64 w) const {
+        const u32 q0 = (u32)q, q1 = (u32)(q >> 32);
+        const unsigned __int128 T = (unsigned __int128)y * w;
+        const u32 m0 = (u32)T * qi;
+        const u64 c0 = (u64)m0 * q1 + (((u64)m0 * q0 + (u32)T) >> 32);
+        const unsigned __int128 U = (T >> 32) + c0;  // three words
+        const u32 m1 = (u32)U * qi;
+        const u64 c1 = (u64)m1 * q1 + (((u64)m1 * q0 + (u32)U) >> 32);
+        s += (u64)(U >> 32) + c1;
+    }
+    __device__ __forceinline__ static bool full(u32 j) { return (j & 3) == 3; }
+    __device__ __forceinline__ S reduced(S s) const { return shoup_lazy3(s, 1, r_hi, q); }
+    __device__ __forceinline__ u64 total(S s) const { return shoup_lazy3(s, 0 - r_hi * q, r_lo, q); }
+};
+
+// a canonical residue as a product's first operand
+__device__ __forceinline__ u64 sum_input(u64 x, const RowFp &) { return f64_as_u64(small_to_f64(x)); }
+__device__ __forceinline__ u64 sum_input(u64 x, const RowInt &) { return x; }
+
 // Integer limbs cost two to three times an FP64 limb: they are spread evenly
 // among the others, one first, so that heavy and light blocks run side by
 // side.  Plans of more limbs run them in order.

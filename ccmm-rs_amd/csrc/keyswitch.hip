@@ -2168,6 +2168,13 @@ static bool ks_fused(const ckks_ksk *k) {
     return (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && fused_rows_apply(k->plan);
 }
 
+// The same switch at single-pass degrees: the digits' transforms read
+// single-limb blocks themselves, the inverse transforms form the products.
+static bool ks_small(const ckks_ksk *k) {
+    const int f = ks_fusion(k);
+    return (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && small_tiles_apply(k->plan);
+}
+
 // What a fused key switch of n_cts ciphertexts hands its forward column pass:
 // the digits of single-limb blocks are the (rotated) input limbs themselves,
 // bounded digits one balanced integer per coefficient, larger blocks their
@@ -2295,6 +2302,32 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
     return rc ? rc : launch_columns(ctx, inv.data(), count, false);
 }
 
+// Steps 1 to 4 of ks_small jobs.
+static int ks_small_middle(ckks_context *ctx, const KsJob *const *jobs, size_t count) {
+    std::vector<SmallCall> fwd(count), inv(count);
+    for (size_t i = 0; i < count; ++i) {
+        const KsJob &j = *jobs[i];
+        const ckks_ksk *k = j.k;
+        const size_t N = k->degree, B = k->limbs, D = k->dnum;
+        fwd[i] = SmallCall{k->plan, j.digits, j.digits, j.n_cts * D, B, B * N, B * N};
+        if (ks_lift(k, j.n_cts) == kColResidue) {
+            fwd[i].in = j.x;
+            fwd[i].in_stride = j.x_stride;
+            fwd[i].digits = D;
+            fwd[i].kinv = j.galois_kinv;
+        } else if (int rc = ks_decompose(j, ctx->stream)) {
+            return rc;
+        }
+        inv[i] = SmallCall{k->plan, j.digits, j.acc, j.n_cts * 2, B, 0, B * N, D, 0, k->d_kb, k->d_ka};
+        ckks_execution_profile &pc = ctx->counts();
+        pc.ntt_forwards += j.n_cts * D;
+        pc.ntt_inverses += j.n_cts * 2;
+        pc.ntt_limb_transforms += j.n_cts * (D + 2) * B;
+    }
+    if (int rc = launch_small(ctx, fwd.data(), count, true)) return rc;
+    return launch_small(ctx, inv.data(), count, false);
+}
+
 // k^-1 mod 2N for an odd Galois exponent (Newton iteration on a power of two).
 static u64 galois_inverse(u64 k, u64 two_n) {
     u64 inv = k;
@@ -2353,6 +2386,11 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
         if ((rc = ctx->workspace(0, n_cts * D * B * N * sizeof(u64), &wc))) return rc;
         const KsJob *jp = &j;
         if ((rc = ks_fused_middle(ctx, &jp, 1, (u64 *)wc))) return rc;
+        return ks_moddown(j, s);
+    }
+    if (!hm && ks_small(k)) {
+        const KsJob *jp = &j;
+        if ((rc = ks_small_middle(ctx, &jp, 1))) return rc;
         return ks_moddown(j, s);
     }
     if (hm && ks_fused(k)) {
@@ -2431,15 +2469,17 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
         pa += e[i].n_cts * 2 * B * N;
         fwd[i] = NttCall{k->plan, j.digits, j.digits, e[i].n_cts * k->dnum, B, B * N, B * N};
         inv[i] = NttCall{k->plan, j.acc, j.acc, e[i].n_cts * 2, B, B * N, B * N};
-        if (!ks_fused(k) && (rc = ks_decompose(j, s))) return rc;
+        if (!ks_fused(k) && !ks_small(k) && (rc = ks_decompose(j, s))) return rc;
     }
     // fused entries (ks_fused) share one launch per column pass, the others
     // one launch per pass of the whole transforms
-    std::vector<const KsJob *> fused;
+    std::vector<const KsJob *> fused, small;
     std::vector<NttCall> plain, back;
     size_t cols = 0;
     for (size_t i = 0; i < count; ++i) {
-        if (ks_fused(e[i].k)) {
+        if (ks_small(e[i].k)) {
+            small.push_back(&jobs[i]);
+        } else if (ks_fused(e[i].k)) {
             fused.push_back(&jobs[i]);
             cols += e[i].n_cts * e[i].k->dnum * e[i].k->limbs * e[i].k->degree;
         } else {
@@ -2452,9 +2492,10 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
         if ((rc = ctx->workspace(0, cols * sizeof(u64), &wc))) return rc;
         if ((rc = ks_fused_middle(ctx, fused.data(), fused.size(), (u64 *)wc))) return rc;
     }
+    if ((rc = ks_small_middle(ctx, small.data(), small.size()))) return rc;
     if ((rc = launch_ntt(ctx, plain.data(), plain.size(), true))) return rc;
     for (size_t i = 0; i < count; ++i)
-        if (!ks_fused(e[i].k) && (rc = ks_mac(jobs[i], s))) return rc;
+        if (!ks_fused(e[i].k) && !ks_small(e[i].k) && (rc = ks_mac(jobs[i], s))) return rc;
     if ((rc = launch_ntt(ctx, back.data(), back.size(), false))) return rc;
     std::vector<const KsJob *> all(count);
     for (size_t i = 0; i < count; ++i) all[i] = &jobs[i];

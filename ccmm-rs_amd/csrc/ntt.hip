@@ -15,6 +15,7 @@
 #include <mutex>
 #include <vector>
 
+#include "fused.hpp"
 #include "host_math.hpp"
 #include "internal.hpp"
 #include "ntt_pass.hpp"
@@ -333,14 +334,20 @@ int launch_ntt(ckks_context *ctx, const NttCall *calls, size_t count, bool forwa
     {
         NttLaunch l{};
         u32 blocks = 0;
+        std::vector<SmallCall> small;
         for (size_t i = 0; i < count; ++i) {
             const NttCall &c = calls[i];
             if (c.n_polys == 0 || two_pass(i)) continue;
             DevNttDesc d = base_desc(c);
+            if (src == kSrcPlain && small_tiles_apply(c.plan)) {
+                small.push_back(SmallCall{c.plan, c.in, c.out, c.n_polys, c.n_limbs, d.in_stride, d.out_stride});
+                continue;
+            }
             d.block_start = blocks;
             l.d[l.n++] = d;
             blocks += d.n_polys * d.n_limbs;
         }
+        if (int rc = launch_small(ctx, small.data(), small.size(), forward)) return rc;
         launch_pass(s, forward, true, l, blocks, 0, src);
     }
     if (total_two) {

@@ -165,3 +165,42 @@ def test_key_switch_batches_of_one_shape_share_launches(pkg, ctx):
     pkg.apply_galois_batch(ctx, entries)
     for i, (key, e, ct, out) in enumerate(entries):
         assert torch.equal(out, key.apply_galois(ct, e)), f"entry {i}"
+
+
+@pytest.mark.parametrize("mix", sorted(MIXES))
+@pytest.mark.parametrize("logn", [10, 11, 12, 13])
+def test_key_switches_match_separate_kernels(pkg, ctx, logn, mix):
+    """Digits read by the transforms, products formed between them: single-limb
+    and larger blocks, hybrid, gadget and bounded keys, conjugation, extremes."""
+    import torch
+
+    n, bits = 1 << logn, MIXES[mix]
+    q = _moduli(pkg, n, bits)
+    qp = q + pkg.find_ntt_primes(60, n, 1, skip=q)
+    L = len(q)
+    rng = np.random.default_rng(logn * 10 + L)
+    plan, q_plan = pkg.PreparedRnsNttPlan(ctx, qp, n), pkg.PreparedRnsNttPlan(ctx, q, n)
+    ct = rand_residues(rng, q, n, 6).reshape(3, 2, L, n)
+    ct[0, 1, :, : n // 2] = np.array(q, dtype=np.uint64)[:, None] - 1
+    ct[1, 1, :, n // 2:] = 0
+    ct = pkg.to_device(ct)
+
+    def material(mods, entries):
+        return rand_residues(rng, mods, n, entries), rand_residues(rng, mods, n, entries)
+
+    keys = [pkg.HybridKeySwitchKey(plan, L, [1] * L, *material(qp, L)),
+            pkg.HybridKeySwitchKey(plan, L, [L - L // 2, L // 2], *material(qp, 2)),
+            pkg.RnsKeySwitchKey(q_plan, [1] * L, *material(q, L))]
+    for base_log in (7, 31, 61):
+        d = pkg.bounded_digit_count(plan, L, base_log)
+        keys.append(pkg.BoundedKeySwitchKey(plan, L, base_log, *material(qp, d)))
+    for k, key in enumerate(keys):
+        for e in (5, 2 * n - 1, n + 1):
+            ctx.set_key_switch_fusion(ctx.KS_FUSION_OFF)
+            try:
+                want = key.apply_galois(ct, e)
+            finally:
+                ctx.set_key_switch_fusion(ctx.KS_FUSION_AUTO)
+            assert torch.equal(key.apply_galois(ct, e), want), f"key {k} exponent {e}"
+            one = ct[2:].contiguous()
+            assert torch.equal(key.apply_galois(one, e), want[2:]), f"key {k} exponent {e}, one ciphertext"

@@ -70,35 +70,33 @@ struct ColLaunch {
     u32 n, blocks;
 };
 
-template <int K1>
-__device__ __forceinline__ void col_read(u64 (&v)[16], const u64 *src, u32 n2, u32 tile, u32 tid, u32 kind) {
-    typedef ColTile<K1> C;
+template <class C>
+__device__ __forceinline__ void col_read(u64 (&v)[C::M], const u64 *src, u32 n2, u32 tile, u32 tid, u32 kind) {
     const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
     if (kind == kColInt8) {
         const int8_t *b = (const int8_t *)src;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = (u64)(int64_t)(b + C::template step<0>(n2, i))[o0 / 8];
+        for (int i = 0; i < C::M; ++i) v[i] = (u64)(int64_t)(b + C::template step<0>(n2, i))[o0 / 8];
     } else if (kind == kColPlain) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = load_once_at(src + C::template step<0>(n2, i), o0);
+        for (int i = 0; i < C::M; ++i) v[i] = load_once_at(src + C::template step<0>(n2, i), o0);
     } else {
         // read once per target limb: not streamed
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = load_at(src + C::template step<0>(n2, i), o0);
+        for (int i = 0; i < C::M; ++i) v[i] = load_at(src + C::template step<0>(n2, i), o0);
     }
 }
 
-template <int K1, class Ar>
-__device__ __forceinline__ void col_blocks(u64 (&v)[16], const u64 *src, u64 N, const CK_CONST_AS ColBlock &blk,
+template <class C, class Ar>
+__device__ __forceinline__ void col_blocks(u64 (&v)[C::M], const u64 *src, u64 N, const CK_CONST_AS ColBlock &blk,
                                            u32 limb, u32 n2, u32 tile, u32 tid, const CK_CONST_AS DevPrime &P) {
-    typedef ColTile<K1> C;
     typedef BlockSum<Ar::kFp> Sum;
     constexpr int W = 8;  // residues summed at a time: what their partial sums leave room for
     const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
     const CK_CONST_AS u64 *row0 = const_table(blk.rows) + (u64)limb * kColTerms * 2;
     const u32 first = blk.first, terms = blk.terms, split = blk.split;
 #pragma unroll
-    for (int g = 0; g < 16; g += W) {
+    for (int g = 0; g < C::M; g += W) {
         Sum s[W];
         u64 x[W];
         const CK_CONST_AS u64 *row = row0;
@@ -140,11 +138,10 @@ __device__ __forceinline__ void col_blocks(u64 (&v)[16], const u64 *src, u64 N, 
     }
 }
 
-template <int K1, bool BLOCK, class Ar>
+template <class C, bool BLOCK, class Ar>
 __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS DevPrime &P, const Ar &ar, u32 limb,
                                             u32 poly, u32 tile, u64 *lds) {
-    typedef ColTile<K1> C;
-    const u32 tid = threadIdx.x, n2 = e.logn - K1;
+    const u32 tid = threadIdx.x, n2 = e.logn - C::K;
     const u64 N = (u64)1 << e.logn;
     const u64 *src = nullptr;
     u64 limit = 0;
@@ -159,13 +156,13 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
         src = e.src + ct * e.stride + j * N;
         limit = e.kind == kColResidue ? const_table(e.primes)[j].q : e.limit;
     }
-    u64 v[16];
-    int b[16];
+    u64 v[C::M];
+    int b[C::M];
     if (BLOCK) {
         const u32 ct = poly / e.digits, j = poly % e.digits;
-        col_blocks<K1, Ar>(v, e.src + ct * e.stride, N, const_table(e.blocks)[j], limb, n2, tile, tid, P);
+        col_blocks<C, Ar>(v, e.src + ct * e.stride, N, const_table(e.blocks)[j], limb, n2, tile, tid, P);
     } else {
-        col_read<K1>(v, src, n2, tile, tid, e.kind);
+        col_read<C>(v, src, n2, tile, tid, e.kind);
         col_lift(v, e.kind, limit, ar, P);
     }
     C::set(b, Ar::kFp ? kColFpIn : kColIntIn);
@@ -174,19 +171,27 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
     // on to the row pass: times psi^((2u+1) t)
     u64 *dst = e.dst + ((u64)limb * e.n_polys + poly) * N;
     const typename Ar::Z *z = (const typename Ar::Z *)P.zf;
-    const u32 o1 = C::template offset<1>(tile, n2, tid, 0);
-    typename Ar::Z zv[16];
+    const u32 o1 = C::template offset<C::LAST>(tile, n2, tid, 0);
+    typename Ar::Z zv[C::M];
     if (Ar::kFp) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) zv[i] = load_z(z + C::template step<1>(n2, i), o1);
+        for (int i = 0; i < C::M; ++i) zv[i] = load_z(z + C::template step<C::LAST>(n2, i), o1);
     }
     __syncthreads();
     C::template get<1>(v, tid, lds);
     C::level(b);
     C::template fwd<1>(v, b, tid, P.fwd, ar);
+    if constexpr (C::LAST == 2) {
+        __syncthreads();
+        C::template put<1>(v, tid, lds);
+        __syncthreads();
+        C::template get<2>(v, tid, lds);
+        C::level(b);
+        C::template fwd<2>(v, b, tid, P.fwd, ar);
+    }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const u32 st = C::template step<1>(n2, i);
+    for (int i = 0; i < C::M; ++i) {
+        const u32 st = C::template step<C::LAST>(n2, i);
         // 16-byte row products: a few in flight at a time
         if (!Ar::kFp) zv[i] = load_z(z + st, o1);
         store_once_at(dst + st, o1 * 8, ar.times(v[i], zv[i]));
@@ -194,29 +199,36 @@ __device__ __forceinline__ void col_forward(const ColEntry &e, const CK_CONST_AS
     }
 }
 
-template <int K1, bool ADD, class Ar>
+template <class C, bool ADD, class Ar>
 __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS DevPrime &P, const Ar &ar, u32 limb,
                                             u32 poly, u32 tile, u64 *lds) {
-    typedef ColTile<K1> C;
-    const u32 tid = threadIdx.x, n2 = e.logn - K1;
+    const u32 tid = threadIdx.x, n2 = e.logn - C::K;
     const u64 N = (u64)1 << e.logn;
     const u64 *src = e.src + ((u64)limb * e.n_polys + poly) * N;
     u64 *dst = e.dst + poly * e.stride + limb * N;
-    u64 v[16];
-    int b[16];
+    u64 v[C::M];
+    int b[C::M];
     const typename Ar::Z *z = (const typename Ar::Z *)P.zi;
-    const u32 o1 = C::template offset<1>(tile, n2, tid, 0);
+    const u32 o1 = C::template offset<C::LAST>(tile, n2, tid, 0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const u32 st = C::template step<1>(n2, i);
+    for (int i = 0; i < C::M; ++i) {
+        const u32 st = C::template step<C::LAST>(n2, i);
         v[i] = load_once_at(src + st, o1 * 8);
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        v[i] = ar.times(v[i], load_z(z + C::template step<1>(n2, i), o1));
+    for (int i = 0; i < C::M; ++i) {
+        v[i] = ar.times(v[i], load_z(z + C::template step<C::LAST>(n2, i), o1));
         if (!Ar::kFp && (i & 3) == 3) sched_fence();
     }
     C::set(b, Ar::kZ);
+    if constexpr (C::LAST == 2) {
+        C::template inv<2>(v, b, tid, P.inv, ar);
+        C::template put<2>(v, tid, lds);
+        __syncthreads();
+        C::template get<1>(v, tid, lds);
+        C::level(b);
+        __syncthreads();
+    }
     C::template inv<1>(v, b, tid, P.inv, ar);
     C::template put<1>(v, tid, lds);
     __syncthreads();
@@ -225,7 +237,7 @@ __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS
     C::template inv<0>(v, b, tid, P.inv, ar);
     const u32 o0 = C::template offset<0>(tile, n2, tid, 0) * 8;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < C::M; ++i) {
         u64 r;
         if constexpr (Ar::kFp) {
             r = fp_residue(fp_mulmod(u64_as_f64(v[i]), P.ninv_d, P.ninv_p, ar.q), ar.q, ar.qinv);
@@ -259,8 +271,8 @@ __device__ __forceinline__ void col_inverse(const ColEntry &e, const CK_CONST_AS
 constexpr u32 kColGroup = 4;
 
 // OTHER: kColBlock digits (forward) or ColAdd (inverse), which take more registers
-template <bool FWD, bool OTHER>
-__global__ __launch_bounds__(256, OTHER ? 4 : 5) void k_columns(ColLaunch l) {
+template <bool FWD, bool OTHER, int B>
+__global__ __launch_bounds__(4096 >> B, B == 3 || OTHER ? 4 : 5) void k_columns(ColLaunch l) {
     __shared__ u64 lds[4096];
     u32 di = 0;
     while (di + 1 < l.n && blockIdx.x >= l.e[di + 1].block_start) ++di;
@@ -287,15 +299,17 @@ __global__ __launch_bounds__(256, OTHER ? 4 : 5) void k_columns(ColLaunch l) {
     const RowInt in{P.q};
     switch (e.logn - ntt_n2(e.logn)) {
 #define CK_COL(K1)                                                            \
-    case K1:                                                                  \
+    case K1: {                                                                \
+        typedef ColTile<K1, B> C;                                             \
         if (FWD) {                                                            \
-            if (P.fp) col_forward<K1, OTHER>(e, P, fp, limb, poly, tile, lds);      \
-            else col_forward<K1, OTHER>(e, P, in, limb, poly, tile, lds);           \
+            if (P.fp) col_forward<C, OTHER>(e, P, fp, limb, poly, tile, lds);      \
+            else col_forward<C, OTHER>(e, P, in, limb, poly, tile, lds);           \
         } else {                                                              \
-            if (P.fp) col_inverse<K1, OTHER>(e, P, fp, limb, poly, tile, lds);      \
-            else col_inverse<K1, OTHER>(e, P, in, limb, poly, tile, lds);           \
+            if (P.fp) col_inverse<C, OTHER>(e, P, fp, limb, poly, tile, lds);      \
+            else col_inverse<C, OTHER>(e, P, in, limb, poly, tile, lds);           \
         }                                                                     \
-        break;
+        break;                                                                \
+    }
         CK_COL(6)
         CK_COL(7)
         CK_COL(8)
@@ -303,6 +317,12 @@ __global__ __launch_bounds__(256, OTHER ? 4 : 5) void k_columns(ColLaunch l) {
     }
 }
 
+// Tiles up to which a launch takes the 512-thread form (ColTile B = 3), where a
+// CU has few waves to hide latencies in.  4 ciphertexts at N = 2^13 (208 and 208
+// tiles): mixed-radix digits 18.7 -> 12.4 us, inverse 10.1 -> 8.2 us.  Above, the
+// 16-residue form with its one exchange wins: inverse of 800 tiles 21.9 / 25.6 us,
+// of 65536 tiles 1250 / 1667 us.
+constexpr u32 kWideColumns = 512;
 int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool forward) {
     if (count > (size_t)kMaxColEntries) return fail(CKKS_ERR_INVALID, "NTT batch holds at most 16 entries");
     ColLaunch l{}, lo{};  // lo: OTHER entries of k_columns
@@ -338,13 +358,20 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
         (forward ? pc.ntt_forwards : pc.ntt_inverses) += c.n_polys;
         pc.ntt_limb_transforms += c.n_polys * c.n_limbs;
     }
-    const dim3 g(l.blocks), go(lo.blocks), t(256);
+    const auto launch = [&](auto fwd, auto other, const ColLaunch &c) {
+        constexpr bool F = decltype(fwd)::value, O = decltype(other)::value;
+        if (c.blocks == 0) return;
+        if (c.blocks <= kWideColumns)
+            hipLaunchKernelGGL((k_columns<F, O, 3>), dim3(c.blocks), dim3(512), 0, ctx->stream, c);
+        else
+            hipLaunchKernelGGL((k_columns<F, O, 4>), dim3(c.blocks), dim3(256), 0, ctx->stream, c);
+    };
     if (forward) {
-        if (l.blocks) hipLaunchKernelGGL((k_columns<true, false>), g, t, 0, ctx->stream, l);
-        if (lo.blocks) hipLaunchKernelGGL((k_columns<true, true>), go, t, 0, ctx->stream, lo);
+        launch(std::true_type(), std::false_type(), l);
+        launch(std::true_type(), std::true_type(), lo);
     } else {
-        if (l.blocks) hipLaunchKernelGGL((k_columns<false, false>), g, t, 0, ctx->stream, l);
-        if (lo.blocks) hipLaunchKernelGGL((k_columns<false, true>), go, t, 0, ctx->stream, lo);
+        launch(std::false_type(), std::false_type(), l);
+        launch(std::false_type(), std::true_type(), lo);
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
@@ -359,16 +386,23 @@ int launch_columns(ckks_context *ctx, const ColCall *calls, size_t count, bool f
 // share of heavy limbs.
 struct RowGrid {
     u32 n_cts, limbs, logn, groups;
+    u32 tb;   // a tile is 2^tb residues
     u32 xcd;  // 0: ciphertexts of a group on consecutive blocks
     unsigned char order[kMaxOrder];
 };
 
+// Tiles halve where whole ones would not give every CU more than one: a lone
+// tile's eight waves compete for issue slots that idle CUs have.  4 ciphertexts
+// at N = 2^13: tensor (72 whole tiles) 29.3 -> 23.0 us, key products of 2 digits
+// (104) 19.4 -> 15.4 us.  Above, whole tiles read keys in longer runs.
+constexpr size_t kHalfTiles = 256;
 static RowGrid row_grid(const ckks_rns_plan *plan, size_t limbs, size_t n_cts, bool xcd) {
     RowGrid g{};
     g.n_cts = (u32)n_cts;
     g.limbs = (u32)limbs;
     g.logn = plan->logn;
-    g.groups = (u32)(limbs << (plan->logn - 12));
+    g.tb = (limbs * n_cts) << (plan->logn - 12) <= kHalfTiles ? 11 : 12;
+    g.groups = (u32)(limbs << (plan->logn - g.tb));
     g.xcd = xcd ? 1u : 0u;
     limb_order(plan, limbs, g.order);
     return g;
@@ -393,7 +427,7 @@ __device__ __forceinline__ RowBlock row_block(const RowGrid &g, u32 b) {
         r.ct = b % g.n_cts;
     }
     r.idle = group >= g.groups;
-    const u32 lt = g.logn - 12, pos = group >> lt;
+    const u32 lt = g.logn - g.tb, pos = group >> lt;
     r.tile = group & ((1u << lt) - 1);
     r.limb = r.idle ? 0 : g.limbs <= kMaxOrder ? g.order[pos] : pos;
     return r;
@@ -411,14 +445,13 @@ struct RowMacArgs {
 // An exchange writes one of two LDS buffers and reads it after the barrier; the
 // buffer's previous readers passed the other exchange's barrier in between, so
 // one barrier per exchange is enough, also from one transform to the next.
-template <int L>
-using RowLds = u64[RowTile<L>::LDS];
+template <class R>
+using RowLds = u64[R::LDS];
 
 // geometry A (inter-pass) -> C (natural), bounds in b
-template <int L, class Ar>
-__device__ __forceinline__ void row_forward(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, RowLds<L> *lds,
+template <class R, class Ar>
+__device__ __forceinline__ void row_forward(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, RowLds<R> *lds,
                                             const Ar &ar) {
-    typedef RowTile<L> R;
     typename R::LowTw low;
     R::template fwd<0>(v, b, tid, tw, low, ar);
     R::template put<0>(v, tid, lds[0]);
@@ -435,10 +468,9 @@ __device__ __forceinline__ void row_forward(u64 (&v)[8], int (&b)[8], u32 tid, c
     for (int x = 0; x < (1 << R::EX); ++x) R::fwd_group(v, b, x, low, ar);
 }
 
-template <int L, class Ar>
+template <class R, class Ar>
 __device__ __forceinline__ void row_inverse(u64 (&v)[8], int (&b)[8], u32 tid, const Tw *tw, u64 *l0, u64 *l1,
                                             const Ar &ar) {
-    typedef RowTile<L> R;
     const typename R::LowTw low = R::low_twiddles(tw, tid);
     R::template inv<2>(v, b, tid, tw, low, ar);
     R::template put<2>(v, tid, l0);
@@ -457,7 +489,7 @@ __device__ __forceinline__ void row_inverse(u64 (&v)[8], int (&b)[8], u32 tid, c
 // thread's first, the 2^EX columns of a thread adjacent and 16-byte aligned.
 template <int L>
 __device__ __forceinline__ void natural_read(u64 (&w)[8], const u64 *k, u32 n1, u32 nat0) {
-    typedef RowTile<L> R;
+    typedef RowTile<L> R;  // the same for every tile size
 #pragma unroll
     for (int i = 0; i < 8; i += R::EX ? 2 : 1) {
         const u64 *at = k + (bitrev((u32)i >> R::EX, L) << n1) + (i & ((1 << R::EX) - 1));
@@ -471,14 +503,14 @@ __device__ __forceinline__ void natural_read(u64 (&w)[8], const u64 *k, u32 n1, 
     }
 }
 
-template <int L, class Ar, class Sum>
+template <int L, int TB, class Ar, class Sum>
 struct RowMacBody {
-    typedef RowTile<L> R;
+    typedef RowTile<L, TB> R;
     const RowMacArgs &a;
     const CK_CONST_AS DevPrime &P;
     const Ar ar;
     const Sum sum;
-    u64 (*lds)[RowTile<L>::LDS];
+    RowLds<R> *lds;
     u32 tid;
 
     __device__ __forceinline__ void run(const RowBlock &blk) {
@@ -560,23 +592,24 @@ struct RowMacBody {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = sum.total(c ? sa[i] : sb[i]);
             R::set(b, Sum::kIn);
-            row_inverse<L>(v, b, tid, P.inv, lds[0], lds[1], ar);
+            row_inverse<R>(v, b, tid, P.inv, lds[0], lds[1], ar);
 #pragma unroll
             for (int i = 0; i < 8; ++i) *(u64 *)((char *)(out + c * N + (i << (L - 3))) + off0) = v[i];
         }
     }
 };
 
-template <int L>
-__global__ __launch_bounds__(512, 4) void k_row_mac(RowMacArgs a) {
-    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+template <int L, int TB>
+__global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_mac(RowMacArgs a) {
+    typedef RowTile<L, TB> R;
+    __shared__ __align__(16) u64 lds[2][R::LDS];
     const RowBlock blk = row_block(a.grid, blockIdx.x);
     if (blk.idle) return;
     const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
     if (P.fp)
-        RowMacBody<L, RowFp, SumFp>{a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, threadIdx.x}.run(blk);
+        RowMacBody<L, TB, RowFp, SumFp>{a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, threadIdx.x}.run(blk);
     else
-        RowMacBody<L, RowInt, SumInt>{a, P, RowInt{P.q}, SumInt(P), lds, threadIdx.x}.run(blk);
+        RowMacBody<L, TB, RowInt, SumInt>{a, P, RowInt{P.q}, SumInt(P), lds, threadIdx.x}.run(blk);
 }
 
 int launch_row_mac(ckks_context *ctx, RowMac &m) {
@@ -595,11 +628,13 @@ int launch_row_mac(ckks_context *ctx, RowMac &m) {
     a.dnum = (u32)m.dnum;
     if ((u64)m.limbs * n_cts << (m.plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "key-switch batch too large for one launch");
-    const dim3 g(row_blocks(a.grid)), t(512);
-    switch (ntt_n2(m.plan->logn)) {
-        case 7: hipLaunchKernelGGL(k_row_mac<7>, g, t, 0, ctx->stream, a); break;
-        case 8: hipLaunchKernelGGL(k_row_mac<8>, g, t, 0, ctx->stream, a); break;
-        default: hipLaunchKernelGGL(k_row_mac<9>, g, t, 0, ctx->stream, a); break;
+    const dim3 g(row_blocks(a.grid)), t(1u << (a.grid.tb - 3));
+    switch (ntt_n2(m.plan->logn) * 2 + a.grid.tb - 11) {
+#define CK_ROW(L)                                                                                          \
+    case L * 2: hipLaunchKernelGGL((k_row_mac<L, 11>), g, t, 0, ctx->stream, a); break;                    \
+    case L * 2 + 1: hipLaunchKernelGGL((k_row_mac<L, 12>), g, t, 0, ctx->stream, a); break;
+        CK_ROW(7) CK_ROW(8) CK_ROW(9)
+#undef CK_ROW
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
@@ -639,10 +674,9 @@ struct RowMulArgs {
 // passes (memory-bound like this one: 16 bytes a residue) a plaintext product
 // of 16 ciphertexts and its rescale take 224 us at N = 2^15, 13 limbs (308 us
 // with separate passes), an encryption of 8 polynomials there 118 us (184 us).
-template <int L, bool INTER, class Ar, class Sum>
+template <int L, bool INTER, class R, class Ar, class Sum>
 __device__ __forceinline__ void row_mul_tile(const RowMulArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
-                                             const Sum &sum, RowLds<L> *lds, const RowBlock &blk) {
-    typedef RowTile<L> R;
+                                             const Sum &sum, RowLds<R> *lds, const RowBlock &blk) {
     const u32 tid = threadIdx.x, logn = a.grid.logn, n1 = logn - L;
     const u64 N = (u64)1 << logn;
     const u32 off0 = R::internal_off(blk.tile, n1, tid, 0) * 8;
@@ -656,14 +690,14 @@ __device__ __forceinline__ void row_mul_tile(const RowMulArgs &a, const CK_CONST
 #pragma unroll
         for (int i = 0; i < 8; ++i) w[i] = load_at(y + (i << (L - 3)), off0);
         R::set(b, Ar::kZ);
-        row_forward<L>(w, b, tid, P.fwd, lds, ar);
+        row_forward<R>(w, b, tid, P.fwd, lds, ar);
         row_factor(w, b, ar);
     } else {
         const u64 *k = a.w + blk.ct / a.share * a.w_stride + (u64)blk.limb * N;
         natural_read<L>(w, k, n1, R::natural_off(blk.tile, n1, tid, 0) * 8);
     }
     R::set(b, Ar::kZ);
-    row_forward<L>(v, b, tid, P.fwd, lds, ar);
+    row_forward<R>(v, b, tid, P.fwd, lds, ar);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         typename Sum::S s = 0;
@@ -672,21 +706,22 @@ __device__ __forceinline__ void row_mul_tile(const RowMulArgs &a, const CK_CONST
         v[i] = sum.total(s);
     }
     R::set(b, Sum::kIn);
-    row_inverse<L>(v, b, tid, P.inv, lds[0], lds[1], ar);
+    row_inverse<R>(v, b, tid, P.inv, lds[0], lds[1], ar);
 #pragma unroll
     for (int i = 0; i < 8; ++i) *(u64 *)((char *)(x + (i << (L - 3))) + off0) = v[i];
 }
 
-template <int L, bool INTER>
-__global__ __launch_bounds__(512, 4) void k_row_mul(RowMulArgs a) {
-    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+template <int L, int TB, bool INTER>
+__global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_mul(RowMulArgs a) {
+    typedef RowTile<L, TB> R;
+    __shared__ __align__(16) u64 lds[2][R::LDS];
     const RowBlock blk = row_block(a.grid, blockIdx.x);
     if (blk.idle) return;
     const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
     if (P.fp)
-        row_mul_tile<L, INTER>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
+        row_mul_tile<L, INTER, R>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
     else
-        row_mul_tile<L, INTER>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+        row_mul_tile<L, INTER, R>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
 }
 
 int launch_row_mul(ckks_context *ctx, const RowMul &m) {
@@ -701,13 +736,14 @@ int launch_row_mul(ckks_context *ctx, const RowMul &m) {
     a.grid = row_grid(m.plan, m.limbs, m.n_polys, true);
     if ((u64)m.limbs * m.n_polys << (m.plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
-    const dim3 g(row_blocks(a.grid)), t(512);
-    switch (ntt_n2(m.plan->logn) * 2 + (m.y ? 1 : 0)) {
-#define CK_RM(L)                                                                             \
-    case L * 2: hipLaunchKernelGGL((k_row_mul<L, false>), g, t, 0, ctx->stream, a); break;    \
-    case L * 2 + 1: hipLaunchKernelGGL((k_row_mul<L, true>), g, t, 0, ctx->stream, a); break;
-        CK_RM(7) CK_RM(8) CK_RM(9)
-#undef CK_RM
+    const dim3 g(row_blocks(a.grid)), t(1u << (a.grid.tb - 3));
+    switch ((ntt_n2(m.plan->logn) * 2 + a.grid.tb - 11) * 2 + (m.y ? 1 : 0)) {
+#define CK_ROW(L, TB, X)                                                                                       \
+    case (L * 2 + TB - 11) * 2 + X: hipLaunchKernelGGL((k_row_mul<L, TB, X>), g, t, 0, ctx->stream, a); break;
+#define CK_ROWS(L) CK_ROW(L, 11, 0) CK_ROW(L, 11, 1) CK_ROW(L, 12, 0) CK_ROW(L, 12, 1)
+        CK_ROWS(7) CK_ROWS(8) CK_ROWS(9)
+#undef CK_ROWS
+#undef CK_ROW
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
@@ -721,10 +757,9 @@ struct RowTensorArgs {
 
 // Four forward row passes, the products and three inverse passes of one tile;
 // b0 and a0 stay in registers as factors while b1 and a1 are transformed.
-template <int L, class Ar, class Sum>
+template <int L, class R, class Ar, class Sum>
 __device__ __forceinline__ void row_tensor_tile(const RowTensorArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
-                                                const Sum &sum, RowLds<L> *lds, const RowBlock &blk) {
-    typedef RowTile<L> R;
+                                                const Sum &sum, RowLds<R> *lds, const RowBlock &blk) {
     u32 tid = threadIdx.x;
     const u32 n1 = a.grid.logn - L;
     const u64 base = ((u64)blk.limb * a.grid.n_cts + blk.ct) << a.grid.logn;
@@ -738,7 +773,7 @@ __device__ __forceinline__ void row_tensor_tile(const RowTensorArgs &a, const CK
         for (int i = 0; i < 8; ++i) f[p][i] = load_at(a.x[p] + base + (i << (L - 3)), off0);
         R::set(b, Ar::kZ);
         tid = opaque(tid);
-        row_forward<L>(f[p], b, tid, P.fwd, lds, ar);
+        row_forward<R>(f[p], b, tid, P.fwd, lds, ar);
         row_factor(f[p], b, ar);
     }
 #pragma unroll
@@ -751,7 +786,7 @@ __device__ __forceinline__ void row_tensor_tile(const RowTensorArgs &a, const CK
         for (int i = 0; i < 8; ++i) v[i] = load_at(a.x[2 + p] + base + (i << (L - 3)), off0);
         R::set(b, Ar::kZ);
         tid = opaque(tid);
-        row_forward<L>(v, b, tid, P.fwd, lds, ar);
+        row_forward<R>(v, b, tid, P.fwd, lds, ar);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             row_mac(c[p][i], v[i], f[0][i], sum);
@@ -765,22 +800,23 @@ __device__ __forceinline__ void row_tensor_tile(const RowTensorArgs &a, const CK
         for (int i = 0; i < 8; ++i) v[i] = sum.total(c[k][i]);
         R::set(b, Sum::kIn);
         tid = opaque(tid);
-        row_inverse<L>(v, b, tid, P.inv, lds[0], lds[1], ar);
+        row_inverse<R>(v, b, tid, P.inv, lds[0], lds[1], ar);
 #pragma unroll
         for (int i = 0; i < 8; ++i) *(u64 *)((char *)(a.x[k] + base + (i << (L - 3))) + off0) = v[i];
     }
 }
 
-template <int L>
-__global__ __launch_bounds__(512, 4) void k_row_tensor(RowTensorArgs a) {
-    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+template <int L, int TB>
+__global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_tensor(RowTensorArgs a) {
+    typedef RowTile<L, TB> R;
+    __shared__ __align__(16) u64 lds[2][R::LDS];
     const RowBlock blk = row_block(a.grid, blockIdx.x);
     if (blk.idle) return;
     const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
     if (P.fp)
-        row_tensor_tile<L>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
+        row_tensor_tile<L, R>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
     else
-        row_tensor_tile<L>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+        row_tensor_tile<L, R>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
 }
 
 int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x[4], size_t n_cts, size_t limbs) {
@@ -791,11 +827,13 @@ int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x
     a.grid = row_grid(plan, limbs, n_cts, true);
     if ((u64)limbs * n_cts << (plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
-    const dim3 g(row_blocks(a.grid)), t(512);
-    switch (ntt_n2(plan->logn)) {
-        case 7: hipLaunchKernelGGL(k_row_tensor<7>, g, t, 0, ctx->stream, a); break;
-        case 8: hipLaunchKernelGGL(k_row_tensor<8>, g, t, 0, ctx->stream, a); break;
-        default: hipLaunchKernelGGL(k_row_tensor<9>, g, t, 0, ctx->stream, a); break;
+    const dim3 g(row_blocks(a.grid)), t(1u << (a.grid.tb - 3));
+    switch (ntt_n2(plan->logn) * 2 + a.grid.tb - 11) {
+#define CK_ROW(L)                                                                                          \
+    case L * 2: hipLaunchKernelGGL((k_row_tensor<L, 11>), g, t, 0, ctx->stream, a); break;                    \
+    case L * 2 + 1: hipLaunchKernelGGL((k_row_tensor<L, 12>), g, t, 0, ctx->stream, a); break;
+        CK_ROW(7) CK_ROW(8) CK_ROW(9)
+#undef CK_ROW
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
@@ -826,10 +864,9 @@ __device__ __forceinline__ u64 plus(u64 v, u64 x, const RowInt &) { return v + x
 // reads from L2 (keys alone: 1.18 ms without them); sharing them between two
 // ciphertexts of a workgroup took the registers that it saved in loads
 // (1.55 ms with spills), one workgroup per sum 1.83 ms.
-template <int L, class Ar, class Sum>
+template <int L, class R, class Ar, class Sum>
 __device__ __forceinline__ void row_rotate_tile(const RowRotateArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
-                                                const Sum &sum, RowLds<L> *lds, const RowBlock &blk) {
-    typedef RowTile<L> R;
+                                                const Sum &sum, RowLds<R> *lds, const RowBlock &blk) {
     constexpr int KC = R::KC, EX = R::EX, CL = R::CL;
     constexpr int kCanonical = Ar::kFp ? 2 : 1;
     u32 tid = threadIdx.x;
@@ -907,7 +944,7 @@ __device__ __forceinline__ void row_rotate_tile(const RowRotateArgs &a, const CK
         __syncthreads();
         R::template get<2>(v, tid, lds[c]);
         R::set(b, bound);
-        row_inverse<L>(v, b, tid, P.inv, lds[1 - c], lds[c], ar);
+        row_inverse<R>(v, b, tid, P.inv, lds[1 - c], lds[c], ar);
         const u32 u = (blk.tile << CL) + R::col_of(0, tid, 0);
         const u32 to = (((2 * u + 1) * e.kinv) & ((2u << n1) - 1)) >> 1;
         const u32 off = ((bitrev(to, n1) << L) + R::t_of(0, tid, 0)) * 8;
@@ -916,16 +953,17 @@ __device__ __forceinline__ void row_rotate_tile(const RowRotateArgs &a, const CK
     }
 }
 
-template <int L>
-__global__ __launch_bounds__(512, 4) void k_row_rotate(RowRotateArgs a) {
-    __shared__ __align__(16) u64 lds[2][RowTile<L>::LDS];
+template <int L, int TB>
+__global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_rotate(RowRotateArgs a) {
+    typedef RowTile<L, TB> R;
+    __shared__ __align__(16) u64 lds[2][R::LDS];
     const RowBlock blk = row_block(a.grid, blockIdx.x);
     if (blk.idle) return;
     const CK_CONST_AS DevPrime &P = const_table(a.primes)[blk.limb];
     if (P.fp)
-        row_rotate_tile<L>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
+        row_rotate_tile<L, R>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
     else
-        row_rotate_tile<L>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+        row_rotate_tile<L, R>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
 }
 
 int launch_row_rotate(ckks_context *ctx, const RowRotate &r) {
@@ -942,11 +980,13 @@ int launch_row_rotate(ckks_context *ctx, const RowRotate &r) {
     a.grid = row_grid(r.plan, r.limbs, r.n_cts * r.count, true);
     if ((u64)r.limbs * r.n_cts * r.count << (r.plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
-    const dim3 g(row_blocks(a.grid)), t(512);
-    switch (ntt_n2(r.plan->logn)) {
-        case 7: hipLaunchKernelGGL(k_row_rotate<7>, g, t, 0, ctx->stream, a); break;
-        case 8: hipLaunchKernelGGL(k_row_rotate<8>, g, t, 0, ctx->stream, a); break;
-        default: hipLaunchKernelGGL(k_row_rotate<9>, g, t, 0, ctx->stream, a); break;
+    const dim3 g(row_blocks(a.grid)), t(1u << (a.grid.tb - 3));
+    switch (ntt_n2(r.plan->logn) * 2 + a.grid.tb - 11) {
+#define CK_ROW(L)                                                                                          \
+    case L * 2: hipLaunchKernelGGL((k_row_rotate<L, 11>), g, t, 0, ctx->stream, a); break;                    \
+    case L * 2 + 1: hipLaunchKernelGGL((k_row_rotate<L, 12>), g, t, 0, ctx->stream, a); break;
+        CK_ROW(7) CK_ROW(8) CK_ROW(9)
+#undef CK_ROW
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;

@@ -923,13 +923,26 @@ struct DownArgs {
     u64 fp_targets;  // bit i: Q limb i takes the FP64 target path
     u32 limbs, q_limbs, logn, chunks;
     u32 split;  // every special prime below 2^60: FP64 targets by fp_split_target
+    u32 parts;  // workgroups that share a chunk's target limbs (down_parts)
 };
+
+// Target limbs of a chunk over several workgroups, each forming the P digits
+// for itself, while the launch would leave the chip idle: what a thread does
+// is then one serial chain over the limbs (without P limbs it is a stream and
+// gains nothing).  4 ciphertexts at N = 2^13, 9 + 4
+// limbs (256 workgroups undivided): 17.8 us in one part, 11.5 us in two.
+static u32 down_parts(size_t blocks, size_t q_limbs) {
+    u32 p = 1;
+    while (p < 4 && blocks * p < 1024 && q_limbs >= 4 * (size_t)p) p *= 2;
+    return p;
+}
 
 template <int K>
 __global__ __launch_bounds__(kKsThreads) void k_moddown(DownArgs a) {
     const u32 b = xcd_contiguous_block(blockIdx.x, gridDim.x);
-    const u32 chunk = b % a.chunks;
-    const u32 rest = b / a.chunks;
+    const u32 chunk = b / a.parts % a.chunks;
+    const u32 rest = b / a.parts / a.chunks;
+    const u32 part = b % a.parts, i0 = a.q_limbs * part / a.parts, i1 = a.q_limbs * (part + 1) / a.parts;
     const u32 comp = rest % 2;
     const DownJob &e = a.e[job_of(a, rest / 2)];
     const u32 ct = rest / 2 - (u32)e.first;
@@ -942,7 +955,7 @@ __global__ __launch_bounds__(kKsThreads) void k_moddown(DownArgs a) {
     if (add) add += ct * e.add_stride + ga.idx;
     u64 *o = e.out + ct * e.out_stride + (u64)comp * a.q_limbs * N + n;
     if (K == 0) {
-        for (u32 i = 0; i < a.q_limbs; ++i) {
+        for (u32 i = i0; i < i1; ++i) {
             u64 v = x[(u64)i * N];
             if (add) {
                 const u64 q = primes[i].q;
@@ -997,7 +1010,7 @@ __global__ __launch_bounds__(kKsThreads) void k_moddown(DownArgs a) {
     const CK_CONST_AS u64 *pinv = const_table(md->pinv);
     const CK_CONST_AS u64 *pinv_q = const_table(md->pinv_q);
     const u64 fpm = a.fp_targets;
-    for (u32 i = 0; i < a.q_limbs; ++i) {
+    for (u32 i = i0; i < i1; ++i) {
         if (i < 64 && ((fpm >> i) & 1)) {  // the mask is empty for bases over 64 limbs
             const CK_CONST_AS double *r = tf + (u64)i * kMdRow;
             const double q = r[0];
@@ -2104,7 +2117,8 @@ static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
     da.q_limbs = (u32)k->q_limbs;
     da.logn = k->plan->logn;
     da.chunks = chunks;
-    dim3 g((u32)(n_cts * 2 * chunks));
+    da.parts = jobs[0]->mfma || k->p_limbs == 0 ? 1 : down_parts(n_cts * 2 * chunks, k->q_limbs);
+    dim3 g((u32)(n_cts * 2 * chunks * da.parts));
     if (jobs[0]->mfma) {
         ModDownMfmaArgs dm{da, k->d_bc + D};
         dim3 gm((u32)(n_cts * 2 * (N / kBcRows)));
@@ -2681,7 +2695,8 @@ int ckks_mod_down(const ckks_rns_plan *qp_plan, size_t q_limbs, const uint64_t *
     da.q_limbs = (u32)q_limbs;
     da.logn = qp_plan->logn;
     da.chunks = (u32)(N / kKsThreads);
-    const dim3 g((u32)(n_polys * da.chunks));
+    da.parts = down_parts(n_polys * da.chunks, q_limbs);
+    const dim3 g((u32)(n_polys * da.chunks * da.parts));
     switch (K) {
 #define CK_MDS(KK) \
     case KK: hipLaunchKernelGGL(k_moddown<KK>, g, dim3(kKsThreads), 0, ctx->stream, da); break;

@@ -357,6 +357,7 @@ struct RescaleArgs {
     u64 in_stride, out_stride;
     u32 n_limbs, logn;
     u32 rescale;  // 0: mod switch (drop only)
+    u32 parts;    // workgroups that share a chunk's kept limbs
 };
 
 // One thread per coefficient of one ciphertext component; loops over the
@@ -364,20 +365,21 @@ struct RescaleArgs {
 __global__ __launch_bounds__(kEwThreads) void k_rescale(RescaleArgs a) {
     const u64 n = (u64)1 << a.logn;
     const u64 chunks = n / kEwThreads;
-    const u64 b = blockIdx.x;
+    const u64 b = blockIdx.x / a.parts;
     const u64 c = (b % chunks) * kEwThreads + threadIdx.x;
     const u64 comp = (b / chunks) % 2, ct = (b / chunks) / 2;
-    const u32 L = a.n_limbs, last = L - 1;
+    const u32 L = a.n_limbs, last = L - 1, part = blockIdx.x % a.parts;
+    const u32 i0 = last * part / a.parts, i1 = last * (part + 1) / a.parts;
     const u64 *src = a.in + ct * a.in_stride + comp * (u64)L * n;
     u64 *dst = a.out + ct * a.out_stride + comp * (u64)last * n;
     if (!a.rescale) {
-        for (u32 i = 0; i < last; ++i) dst[(u64)i * n + c] = src[(u64)i * n + c];
+        for (u32 i = i0; i < i1; ++i) dst[(u64)i * n + c] = src[(u64)i * n + c];
         return;
     }
     const u64 q_drop = a.primes[last].q;
     const u64 rem = src[(u64)last * n + c];
     const bool neg = rem > q_drop / 2;
-    for (u32 i = 0; i < last; ++i) {
+    for (u32 i = i0; i < i1; ++i) {
         const DevPrime &P = a.primes[i];
         const RescaleConst k = a.rc[i];
         u64 rq = rem >= P.q ? barrett_reduce128(0, rem, Barrett{P.q, P.br_hi, P.br_lo}) : rem;
@@ -409,7 +411,13 @@ static int rescale_like(bool rescale, const ckks_rns_plan *plan, const u64 *in, 
     a.n_limbs = (u32)n_limbs;
     a.logn = plan->logn;
     a.rescale = rescale ? 1u : 0u;
-    dim3 grid((u32)(n_cts * 2 * (n / kEwThreads)));
+    // while the launch would leave the chip idle, the serial loop over the kept
+    // limbs is divided: 4 ciphertexts at N = 2^13, 9 limbs:
+    // 10.5 -> 6.1 us
+    const size_t blocks = n_cts * 2 * (n / kEwThreads);
+    a.parts = 1;
+    while (a.parts < 8 && blocks * a.parts < 1024 && n_limbs > 2 * a.parts) a.parts *= 2;
+    dim3 grid((u32)(blocks * a.parts));
     hipLaunchKernelGGL(k_rescale, grid, dim3(kEwThreads), 0, plan->ctx->stream, a);
     CK_HIP(hipGetLastError());
     return CKKS_OK;

@@ -19,9 +19,10 @@
 // twiddles take 32 products plus one more per distinct twiddle.  The twiddles of the first six stages
 // are uniform over a wave (geometries below) and come through the scalar unit.
 //
-// A tile is 4096 residues: 2^L residues of 2^(12-L) rows, 8 per thread in 512
-// threads, three rounds of at most 3 stages with an LDS exchange between
-// rounds.  Eight residues a thread (not 16) leave the registers for two
+// A tile is 4096 residues (TB = 12): 2^L residues of 2^(12-L) rows, 8 per thread
+// in 512 threads, three rounds of at most 3 stages with an LDS exchange between
+// rounds.  TB = 11 halves rows and threads (round B's twiddles are then uniform
+// over half a wave only) for launches of few tiles.  Eight residues a thread (not 16) leave the registers for two
 // accumulators per residue.
 #pragma once
 #include "ntt_tile.hpp"
@@ -199,20 +200,20 @@ struct alignas(16) Pair {
     u64 x, y;
 };
 
-template <int L>
+template <int L, int TB = 12>
 struct RowTile {
-    static constexpr int CL = 12 - L, KC = L - 6, EX = 3 - KC;
-    static constexpr u32 THREADS = 512;
-    static_assert(L >= 7 && L <= 9, "rows of 128 .. 512 residues");
+    static constexpr int CL = TB - L, KC = L - 6, EX = 3 - KC;
+    static constexpr u32 THREADS = 1u << (TB - 3);
+    static_assert(L >= 7 && L <= 9 && CL >= 2 && CL >= EX, "rows of 128 .. 512 residues");
 
     CK_HD static u32 t_of(int geo, u32 tid, int i) {
         if (geo == 0) return (tid & ((1u << (L - 3)) - 1)) | ((u32)i << (L - 3));
-        if (geo == 1) return (tid & ((1u << KC) - 1)) | ((u32)i << KC) | ((tid >> 6) << (KC + 3));
+        if (geo == 1) return (tid & ((1u << KC) - 1)) | ((u32)i << KC) | ((tid >> (KC + CL)) << (KC + 3));
         return ((tid >> (CL - EX)) << KC) | ((u32)i >> EX);
     }
     CK_HD static u32 col_of(int geo, u32 tid, int i) {
         if (geo == 0) return tid >> (L - 3);
-        if (geo == 1) return (tid & 63u) >> KC;
+        if (geo == 1) return (tid & ((1u << (KC + CL)) - 1)) >> KC;
         return ((tid & ((1u << (CL - EX)) - 1)) << EX) | ((u32)i & ((1u << EX) - 1));
     }
     // LDS placement: slot a + 2 (a >> 4) of linear address a = (t << CL) | col.
@@ -220,7 +221,7 @@ struct RowTile {
     // a constant the instruction carries as its offset; 64 lanes of 8 bytes
     // touch an 8-byte slot two to four times (two is the least), geometry C's
     // 16-byte accesses each slot four times (the least).
-    static constexpr int LDS = 4096 + 2 * 256;
+    static constexpr int LDS = (1 << TB) + (1 << (TB - 3));
     CK_HD static u32 slot(u32 a) { return a + 2 * (a >> 4); }
     CK_HD static u32 lds_at(int geo, u32 tid, int i) {
         const u32 a = slot((t_of(geo, tid, 0) << CL) | col_of(geo, tid, 0)) +
@@ -294,7 +295,7 @@ struct RowTile {
         if (GEO == 2) return low.t[(1 << k) - 1 + ((i >> EX) >> (KC - k))];
         const u32 j = block_index<GEO>(tid, i, 3 * GEO + k);
         CK_BOUNDS(j, 1u << (L - 1));
-        return load_twiddle<true>(tw, j);
+        return load_twiddle<GEO == 0 || KC + CL >= 6>(tw, j);
     }
 
     // Stages of one geometry; b: bounds of the residues (uniform over threads).

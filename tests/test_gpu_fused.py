@@ -204,3 +204,32 @@ def test_key_switches_match_separate_kernels(pkg, ctx, logn, mix):
             assert torch.equal(key.apply_galois(ct, e), want), f"key {k} exponent {e}"
             one = ct[2:].contiguous()
             assert torch.equal(key.apply_galois(one, e), want[2:]), f"key {k} exponent {e}, one ciphertext"
+
+
+@pytest.mark.parametrize("bits", [[40, 41], [60, 55]])
+@pytest.mark.parametrize("logn", [13, 14, 15, 16, 17])
+def test_launches_of_few_tiles(pkg, ctx, logn, bits):
+    """One ciphertext over few limbs: halved row tiles, column tiles of 512
+    threads, divided ModDown and rescale loops, against larger launches of the
+    same ciphertext repeated (whole tiles) and against the separate kernels."""
+    import torch
+
+    n = 1 << logn
+    q = _moduli(pkg, n, bits)
+    qp = q + pkg.find_ntt_primes(59, n, 1, skip=q)
+    rng = np.random.default_rng(logn)
+    plan = pkg.PreparedRnsNttPlan(ctx, qp, n)
+    key = pkg.HybridKeySwitchKey(plan, 2, [2], rand_residues(rng, qp, n, 1), rand_residues(rng, qp, n, 1))
+    ct = pkg.to_device(_extremes(rng, q, n, 2).reshape(1, 2, 2, n))
+    many = ct.expand(64 if logn < 16 else 8, 2, 2, n).contiguous()
+    for e in (5, 2 * n - 1):
+        one = key.apply_galois(ct, e)
+        assert torch.equal(one[0], key.apply_galois(many, e)[-1]), "rotation"
+        assert torch.equal(key.rotate_hoisted(key.hoist(ct), ct, e), one), "hoisted rotation"
+        ctx.set_key_switch_fusion(ctx.KS_FUSION_OFF)
+        try:
+            assert torch.equal(key.apply_galois(ct, e), one), "separate kernels"
+        finally:
+            ctx.set_key_switch_fusion(ctx.KS_FUSION_AUTO)
+    assert torch.equal(plan.tensor(ct, ct, 2)[0], plan.tensor(many, many, 2)[-1]), "tensor"
+    assert torch.equal(key.multiply_relinearize_rescale(ct, ct)[0], key.multiply_relinearize_rescale(many, many)[-1])

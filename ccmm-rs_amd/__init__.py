@@ -99,6 +99,7 @@ _SIGNATURES = {
     "ckks_tensor": (C.c_int, [_p, _p, _p, _p, _sz, _sz, _sz, _sz]),
     "ckks_multiply_plain": (C.c_int, [_p, _p, _p, _p, _sz, _sz, _sz, _sz, _sz]),
     "ckks_multiply_plain_accumulate_ntt": (C.c_int, [_p, _p, _p, _sz, _p, _sz]),
+    "ckks_multiply_plain_accumulate_ntt_batch": (C.c_int, [_p, _p, _p, _sz, _p, _sz, _sz]),
     "ckks_graph_begin": (C.c_int, [_p]),
     "ckks_graph_end": (C.c_int, [_p, C.POINTER(_p)]),
     "ckks_graph_launch": (C.c_int, [_p]),

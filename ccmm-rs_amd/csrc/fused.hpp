@@ -133,4 +133,11 @@ struct SmallCall {
 };
 int launch_small(ckks_context *ctx, const SmallCall *calls, size_t count, bool forward);
 
+// out[e] = sum_t ct[t] pt[e][t] over NTT-domain ciphertexts [2][limbs][N] and
+// plaintexts [limbs][N]; plans of primes below 2^60.
+constexpr size_t kMacPointers = 384;
+bool mac_tiles_apply(const ckks_rns_plan *plan);
+int launch_mac_lists(const ckks_rns_plan *plan, const u64 *const *cts, const u64 *const *pts, size_t count,
+                     u64 *const *outs, size_t n_outs, size_t n_limbs);
+
 }  // namespace ck

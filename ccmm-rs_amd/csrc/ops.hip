@@ -180,6 +180,7 @@ struct MacListArgs {
     u32 count, n_limbs, logn, chunks;
 };
 
+// Plans with a prime from 2^60 up (others: mac_list.hip):
 // out = sum_t ct_t * pt_t, limb by limb and evaluation point by point
 // (NttPolynomial::pointwise_mul_add_assign, ring/ntt_polynomial.rs:222-235,
 // over the NTT-resident ciphertexts of ckks/rns_plain_multiply.rs:119-191).
@@ -954,26 +955,44 @@ int ckks_poly_neg(const ckks_rns_plan *plan, const uint64_t *x, uint64_t *out, s
 
 int ckks_multiply_plain_accumulate_ntt(const ckks_rns_plan *plan, const uint64_t *const *cts,
                                        const uint64_t *const *pts, size_t count, uint64_t *out, size_t n_limbs) {
+    return ckks_multiply_plain_accumulate_ntt_batch(plan, cts, pts, count, &out, 1, n_limbs);
+}
+
+int ckks_multiply_plain_accumulate_ntt_batch(const ckks_rns_plan *plan, const uint64_t *const *cts,
+                                             const uint64_t *const *pts, size_t count, uint64_t *const *outs,
+                                             size_t n_outs, size_t n_limbs) {
     int rc = check_plan_limbs(plan, n_limbs, "plaintext multiply-accumulate");
     if (rc) return rc;
-    if (!cts || !pts || !out || count == 0) return fail(CKKS_ERR_INVALID, "null argument");
+    if (!cts || !pts || !outs || count == 0) return fail(CKKS_ERR_INVALID, "null argument");
     if (count > kMaxMacTerms) return fail(CKKS_ERR_UNSUPPORTED, "plaintext multiply-accumulate of at most 64 terms");
-    MacListArgs a{};
-    for (size_t t = 0; t < count; ++t) {
-        if (!cts[t] || !pts[t]) return fail(CKKS_ERR_INVALID, "null buffer");
-        a.ct[t] = cts[t];
-        a.pt[t] = pts[t];
+    for (size_t e = 0; e < n_outs; ++e)
+        if (!outs[e]) return fail(CKKS_ERR_INVALID, "null argument");
+    for (size_t t = 0; t < count * (n_outs + 1); ++t)
+        if (!(t < count ? cts[t] : pts[t - count])) return fail(CKKS_ERR_INVALID, "null buffer");
+    const size_t most = mac_tiles_apply(plan) ? std::min<size_t>(16, kMacPointers / count - 1) : 1;
+    for (size_t e = 0; e < n_outs; e += most) {
+        const size_t m = std::min(most, n_outs - e);
+        if (mac_tiles_apply(plan)) {
+            if ((rc = launch_mac_lists(plan, cts, pts + e * count, count, outs + e, m, n_limbs))) return rc;
+        } else {
+            MacListArgs a{};
+            for (size_t t = 0; t < count; ++t) {
+                a.ct[t] = cts[t];
+                a.pt[t] = pts[e * count + t];
+            }
+            a.out = outs[e];
+            a.primes = plan->d_primes;
+            a.count = (u32)count;
+            a.n_limbs = (u32)n_limbs;
+            a.logn = plan->logn;
+            a.chunks = (u32)(plan->degree / kEwChunk);
+            hipLaunchKernelGGL(k_mac_list, dim3((u32)(2 * n_limbs * a.chunks)), dim3(kEwThreads), 0,
+                               plan->ctx->stream, a);
+            CK_HIP(hipGetLastError());
+        }
     }
-    a.out = out;
-    a.primes = plan->d_primes;
-    a.count = (u32)count;
-    a.n_limbs = (u32)n_limbs;
-    a.logn = plan->logn;
-    a.chunks = (u32)(plan->degree / kEwChunk);
-    hipLaunchKernelGGL(k_mac_list, dim3((u32)(2 * n_limbs * a.chunks)), dim3(kEwThreads), 0, plan->ctx->stream, a);
-    CK_HIP(hipGetLastError());
-    plan->ctx->counts().ciphertext_plaintext_multiplies += count;
-    plan->ctx->counts().additions += 2 * (count - 1);
+    plan->ctx->counts().ciphertext_plaintext_multiplies += count * n_outs;
+    plan->ctx->counts().additions += 2 * (count - 1) * n_outs;
     return CKKS_OK;
 }
 

@@ -463,19 +463,29 @@ class ProgramRunner:
                 fn = lib().ckks_ntt_forward_batch if code == OP_NTT else lib().ckks_ntt_inverse_batch
                 _check(fn(ctx.handle, ptr, len(arr)))
             return transform
+        if code == OP_MAC_PLAIN:
+            # sums of the same ciphertexts share a call
+            shared = {}
+            for out, ins, op in items:
+                if not ins or len(ins) != len(op[6]):
+                    raise ValueError("one plaintext per ciphertext, at least one term")
+                shared.setdefault(tuple(ins), []).append((_ptr(self._reg(out, la)),
+                                                          [_ptr(t, la * n, name="pt") for t in op[6]]))
+            sums = []
+            for ins, group in shared.items():
+                sums.append(((C.c_uint64 * len(ins))(*[_ptr(self._reg(i, la)) for i in ins]),
+                             (C.c_uint64 * (len(ins) * len(group)))(*[p for _, pts in group for p in pts]),
+                             (C.c_uint64 * len(group))(*[out for out, _ in group])))
+
+            def accumulate():
+                for ca, pa, oa in sums:
+                    _check(lib().ckks_multiply_plain_accumulate_ntt_batch(
+                        plan.handle, C.cast(ca, _p), C.cast(pa, _p), len(ca), C.cast(oa, _p), len(oa), la))
+            return accumulate
         steps = []
         for out, ins, op in items:
             _, _, _, _, key, _, pt = op
-            if code == OP_MAC_PLAIN:
-                if not ins or len(ins) != len(pt):
-                    raise ValueError("one plaintext per ciphertext, at least one term")
-                ca = (C.c_uint64 * len(ins))(*[_ptr(self._reg(i, la)) for i in ins])
-                pa = (C.c_uint64 * len(ins))(*[_ptr(t, la * n, name="pt") for t in pt])
-
-                def step(ca=ca, pa=pa, out=_ptr(self._reg(out, la))):
-                    _check(lib().ckks_multiply_plain_accumulate_ntt(plan.handle, C.cast(ca, _p), C.cast(pa, _p),
-                                                                    len(ca), out, la))
-            elif code == OP_MUL_PLAIN:
+            if code == OP_MUL_PLAIN:
                 def step(x=self._ct(ins[0], la), pt=pt, out=self._ct(out, la)):
                     plan.multiply_plain(x, pt, la, out=out)
             elif code in (OP_ADD, OP_SUB):

@@ -286,6 +286,12 @@ int ckks_multiply_plain(const ckks_rns_plan *plan, const uint64_t *in, const uin
  * 1..64; out may be one of the cts. */
 int ckks_multiply_plain_accumulate_ntt(const ckks_rns_plan *plan, const uint64_t *const *cts,
                                        const uint64_t *const *pts, size_t count, uint64_t *out, size_t n_limbs);
+/* n_outs such sums of the same ciphertexts in as few launches as their
+ * operands fit: outs[e] = sum_{t < count} cts[t] * pts[e * count + t].  No out
+ * may be one of the cts unless n_outs is 1. */
+int ckks_multiply_plain_accumulate_ntt_batch(const ckks_rns_plan *plan, const uint64_t *const *cts,
+                                             const uint64_t *const *pts, size_t count, uint64_t *const *outs,
+                                             size_t n_outs, size_t n_limbs);
 
 /* encrypt_rns_raw_with_distribution_ntt_rng (grafting/rns_key_switch.rs:
  * 245-383) after its sampling, which stays on the host (ChaCha20, Gaussian

@@ -233,3 +233,36 @@ def test_launches_of_few_tiles(pkg, ctx, logn, bits):
             ctx.set_key_switch_fusion(ctx.KS_FUSION_AUTO)
     assert torch.equal(plan.tensor(ct, ct, 2)[0], plan.tensor(many, many, 2)[-1]), "tensor"
     assert torch.equal(key.multiply_relinearize_rescale(ct, ct)[0], key.multiply_relinearize_rescale(many, many)[-1])
+
+
+@pytest.mark.parametrize("mix", ["both", "wide"])
+@pytest.mark.parametrize("logn,count,n_outs", [(10, 1, 1), (10, 64, 6), (12, 5, 3), (13, 16, 16), (13, 9, 17), (14, 8, 4)])
+def test_shared_inner_sums(pkg, ctx, mix, logn, count, n_outs):
+    """Several sums of the same ciphertexts in one call, edges of the groups of
+    eight and of a launch's operands, against products and additions."""
+    import ctypes as C
+    import torch
+
+    n = 1 << logn
+    q = _moduli(pkg, n, MIXES[mix])
+    L = len(q)
+    rng = np.random.default_rng(count * 100 + n_outs)
+    plan = pkg.PreparedRnsNttPlan(ctx, q, n)
+    cts = [pkg.to_device(_extremes(rng, q, n, 2)) for _ in range(count)]
+    pts = [[pkg.to_device(_extremes(rng, q, n, 1)) for _ in range(count)] for _ in range(n_outs)]
+    outs = [pkg.empty((2, L, n)) for _ in range(n_outs)]
+
+    def array(ts):
+        return (C.c_uint64 * len(ts))(*[t.data_ptr() for t in ts])
+
+    ca, pa, oa = array(cts), array([p for row in pts for p in row]), array(outs)
+    rc = pkg.lib().ckks_multiply_plain_accumulate_ntt_batch(plan.handle, C.cast(ca, C.c_void_p), C.cast(pa, C.c_void_p),
+                                                            count, C.cast(oa, C.c_void_p), n_outs, L)
+    assert rc == 0
+    for e in range(n_outs):
+        want = torch.zeros((2, L, n), dtype=torch.int64, device="cuda")
+        for ct, pt in zip(cts, pts[e]):
+            prod = pkg.empty((2, L, n))
+            plan.pointwise_mul(ct, pt.expand(2, L, n).contiguous(), prod)
+            plan.add(want, prod, want)
+        assert torch.equal(outs[e], want), f"sum {e}"

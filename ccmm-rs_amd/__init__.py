@@ -111,6 +111,9 @@ _SIGNATURES = {
     "ckks_encrypt_raw": (C.c_int, [_p, _p, _p, _p, _p, _p, _sz, _sz, _sz]),
     "ckks_encode_coefficients": (C.c_int, [_p, _p, C.c_double, _p, _sz, _sz]),
     "ckks_mod_down": (C.c_int, [_p, _sz, _p, _p, _sz]),
+    "ckks_embed_slots": (C.c_int, [_p, _p, _p, _p, _sz]),
+    "ckks_encode_spectrum": (C.c_int, [_p, _p, _p, C.c_double, _p, _sz, _sz]),
+    "ckks_decode_twisted": (C.c_int, [_p, _p, C.c_double, _p, _p, _sz, _sz]),
     "ckks_decode_coefficients": (C.c_int, [_p, _p, C.c_double, _p, _sz, _sz]),
     "ckks_server_create": (C.c_int, [_p, _sz, _sz, C.POINTER(_p)]),
     "ckks_server_submit": (C.c_int, [_p, _p, C.POINTER(C.c_uint64)]),

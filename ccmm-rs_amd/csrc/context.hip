@@ -94,6 +94,7 @@ int ckks_context_destroy(ckks_context *ctx) {
     for (void *p : ctx->owned) hipFree(p);
     for (int i = 0; i < 2 * ckks_context::kSlots; ++i)
         if (ctx->ws[i]) hipFree(ctx->ws[i]);
+    if (ctx->h_flag) hipHostFree(ctx->h_flag);
     if (ctx->ev_fork) hipEventDestroy(ctx->ev_fork);
     if (ctx->ev_join) hipEventDestroy(ctx->ev_join);
     if (ctx->aux) hipStreamDestroy(ctx->aux);

@@ -120,6 +120,7 @@ struct ckks_context {
     ckks_execution_profile profile = {}, captured = {};
     ckks_execution_profile &counts() { return capturing ? captured : profile; }
     std::vector<void *> owned;  // misc device allocations freed at destroy
+    int *h_flag = nullptr;  // pinned: a kernel's verdict on its input (encode), read after a wait
     uint64_t *ntt_scratch = nullptr;  // this device's no-allocation NTT scratch
 
     int workspace(int slot, size_t bytes, void **out);

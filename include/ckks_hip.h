@@ -327,6 +327,17 @@ int ckks_mod_down(const ckks_rns_plan *qp_plan, size_t q_limbs, const uint64_t *
 int ckks_encode_coefficients(const ckks_rns_plan *plan, const double *coeffs, double scale,
                              uint64_t *out, size_t n_polys, size_t n_limbs);
 
+/* The same from slots, with the FFT in between left to the caller:
+ * ckks_embed_slots writes the evaluations ev [p][N] (complex doubles) of slots
+ * [p][N/2], slot j at root index roots[j] (device, distinct, with N - 1 -
+ * roots[j] covering every index) and its conjugate at N - 1 - roots[j];
+ * ckks_encode_spectrum takes their forward DFT freq [p][N] and encodes
+ * coefficients Re(freq[k] / N * conj(twist[k])), twist [N] complex doubles. */
+int ckks_embed_slots(const ckks_rns_plan *plan, const double *slots, const int64_t *roots, double *ev,
+                     size_t n_polys);
+int ckks_encode_spectrum(const ckks_rns_plan *plan, const double *freq, const double *twist, double scale,
+                         uint64_t *out, size_t n_polys, size_t n_limbs);
+
 /* Decode (bin/r30_13b_ckks_primitives.rs:55-80), integer half: exact CRT of
  * [p][limb][N] residues over the first n_limbs limbs to the centered integer
  * (value > floor(Q/2) -> negative, ring/wide_crt.rs), converted to FP64 and
@@ -334,6 +345,10 @@ int ckks_encode_coefficients(const ckks_rns_plan *plan, const double *coeffs, do
  * first call per limb count (not capturable) and kept by the plan. */
 int ckks_decode_coefficients(const ckks_rns_plan *plan, const uint64_t *in, double scale,
                              double *out, size_t n_polys, size_t n_limbs);
+/* The same times twist [N] (complex doubles): out [p][N] complex, the input of
+ * the inverse DFT that gives the evaluations. */
+int ckks_decode_twisted(const ckks_rns_plan *plan, const uint64_t *in, double scale, const double *twist,
+                        double *out, size_t n_polys, size_t n_limbs);
 
 /* rns_tensor_with_prepared_ntt (grafting/rns_key_switch.rs:1724-1777):
  * (b0,a0) x (b1,a1) -> (c0,c1,c2) coefficient domain, out laid out as

@@ -266,3 +266,30 @@ def test_shared_inner_sums(pkg, ctx, mix, logn, count, n_outs):
             plan.pointwise_mul(ct, pt.expand(2, L, n).contiguous(), prod)
             plan.add(want, prod, want)
         assert torch.equal(outs[e], want), f"sum {e}"
+
+
+@pytest.mark.parametrize("logn,polys,scale", [(10, 1, 2.0 ** 40), (12, 3, 2.0 ** 55), (13, 2, 1.0), (15, 8, 2.0 ** 40),
+                                              (16, 2, 3.7e11)])
+def test_embedding_passes_match_torch(pkg, ctx, logn, polys, scale):
+    """The scatter, twist and rounding inside the library's kernels give the
+    values of the same passes as torch operations, bit for bit."""
+    import torch
+
+    n = 1 << logn
+    q = _moduli(pkg, n, [60, 40, 41])
+    plan, emb = pkg.PreparedRnsNttPlan(ctx, q, n), pkg.encoding.CanonicalEmbedding(n)
+    gen = torch.Generator(device="cuda").manual_seed(logn)
+    z = torch.randn((polys, n // 2), dtype=torch.complex128, device="cuda", generator=gen)
+    for slots in (z, z.conj(), z.real, z[0], torch.zeros_like(z), z.to(torch.complex64).cpu()):
+        got = pkg.encoding.encode(plan, emb, slots, scale)
+        c = emb.slots_to_coefficients(torch.as_tensor(slots).cuda()).reshape(-1, n)
+        want = pkg.empty((c.shape[0], 3, n))
+        pkg._check(pkg.lib().ckks_encode_coefficients(plan.handle, pkg._ptr(c, dtype="float64"), scale, pkg._ptr(want),
+                                                      c.shape[0], 3))
+        assert torch.equal(got.reshape(want.shape), want)
+    with pytest.raises(pkg.CkksError):
+        pkg.encoding.encode(plan, emb, z, 2.0 ** 70)
+    assert torch.equal(pkg.encoding.encode(plan, emb, z, scale).reshape(-1), pkg.encoding.encode(plan, emb, z, scale).reshape(-1))
+    x = pkg.to_device(_extremes(np.random.default_rng(logn), q, n, polys))
+    want = emb.coefficients_to_slots(pkg.encoding.decode_coefficients(plan, x, scale))
+    assert torch.equal(pkg.encoding.decode(plan, emb, x, scale), want)

@@ -867,7 +867,7 @@ __device__ __forceinline__ u64 plus(u64 v, u64 x, const RowInt &) { return v + x
 template <int L, class R, class Ar, class Sum>
 __device__ __forceinline__ void row_rotate_tile(const RowRotateArgs &a, const CK_CONST_AS DevPrime &P, const Ar &ar,
                                                 const Sum &sum, RowLds<R> *lds, const RowBlock &blk) {
-    constexpr int KC = R::KC, EX = R::EX, CL = R::CL;
+    constexpr int EX = R::EX, CL = R::CL;
     constexpr int kCanonical = Ar::kFp ? 2 : 1;
     u32 tid = threadIdx.x;
     const u32 logn = a.grid.logn, n1 = logn - L;

@@ -2171,8 +2171,8 @@ static bool hoisted_mac_fused(const ckks_context *ctx, u32 logn, size_t dnum) {
 // CKKS_KS_FUSION_XCD / LINEAR (XCD for an untuned key): the digits' forward
 // row pass, the key MAC and the inverse row pass of both sums run in one
 // kernel per tile (launch_row_mac), between the two column passes; neither
-// the NTT-domain digits nor the sums reach HBM.  Other degrees and primes
-// from 2^60 up take the separate kernels.
+// the NTT-domain digits nor the sums reach HBM.  Degrees up to 2^12: ks_small;
+// primes from 2^60 up take the separate kernels.
 static int ks_fusion(const ckks_ksk *k) {
     const ckks_context *ctx = k->ctx;
     return ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;

@@ -13,7 +13,7 @@ namespace ck {
 struct BlockExec {
     u32 threads;
     // thread id handed to the phases; a caller that runs several passes in a
-    // loop can make it opaque per iteration (see k_ntt_row_mac) so the
+    // loop can make it opaque per iteration so the
     // compiler recomputes the index math instead of keeping it live
     u32 tid = threadIdx.x;
     template <class F>

@@ -89,7 +89,10 @@ int ckks_get_ntt_variant(const ckks_context *ctx, uint32_t logn, int *variant);
  * the MAC and the inverse row pass run as one kernel (neither the NTT-domain
  * digits nor the sums reach HBM), with the blocks sharing a key tile placed
  * on one XCD or in plain order; degrees 2^13 .. 2^17 with every prime below
- * 2^60, separate kernels otherwise.
+ * 2^60 (hoisted rotations too: products, Galois permutation and inverse row
+ * pass in one kernel).  Degrees up to 2^12 with such primes: the transforms
+ * read single-limb digits and form the products themselves.  Separate kernels
+ * otherwise.
  * CKKS_KS_FUSION_INVERSE: the MAC is computed inside the first inverse NTT
  * pass (the NTT-domain accumulators never reach HBM; dnum <= 8); set on the
  * context, it also fuses the MAC of hoisted rotations of degrees above

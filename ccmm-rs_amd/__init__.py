@@ -87,6 +87,7 @@ _SIGNATURES = {
     "ckks_poly_mul": (C.c_int, [_p, _p, _p, _p, _sz, _sz, _sz]),
     "ckks_poly_mac": (C.c_int, [_p, _p, _p, _p, _sz, _sz, _sz]),
     "ckks_poly_add": (C.c_int, [_p, _p, _p, _p, _sz, _sz, _sz]),
+    "ckks_poly_sum": (C.c_int, [_p, _p, _sz, _p, _sz, _sz, _sz]),
     "ckks_poly_sub": (C.c_int, [_p, _p, _p, _p, _sz, _sz, _sz]),
     "ckks_poly_neg": (C.c_int, [_p, _p, _p, _sz, _sz, _sz]),
     "ckks_automorphism": (C.c_int, [_p, _p, _p, _sz, _sz, _sz, _u64]),

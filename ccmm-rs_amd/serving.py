@@ -389,6 +389,25 @@ def schedule(prog: Program, n_limbs: int, spare: int):
     return groups, used
 
 
+def merge_sums(groups):
+    """Chains of in-place additions that follow each other directly (an
+    accumulator and what is added to it) as one addition of up to 64 operands:
+    nothing runs between them, and sums of canonical residues do not depend on
+    their order."""
+    out = []
+    for g in groups:
+        code, la, items = g
+        if code == OP_ADD and len(items) == 1 and out and out[-1][0] == OP_ADD and out[-1][1] == la \
+                and len(out[-1][2]) == 1:
+            row, ins, op = items[0]
+            acc, terms, first = out[-1][2][0]
+            if row == acc and ins[0] == acc and ins[1] != acc and len(terms) < 64:
+                out[-1] = (code, la, [(acc, terms + [ins[1]], first)])
+                continue
+        out.append(g)
+    return out
+
+
 class ProgramRunner:
     """Runs one Program directly on registers it owns, outside the serving
     loop, so that a whole rotation schedule can be captured once as a hipGraph
@@ -423,7 +442,8 @@ class ProgramRunner:
         self.graph = None
 
     def _plan_ops(self):
-        self.groups, self.rows = schedule(self.prog, self.L, self.spare)
+        groups, self.rows = schedule(self.prog, self.L, self.spare)
+        self.groups = merge_sums(groups)
         self.planned = len(self.prog.ops)
         self.calls = None
 
@@ -488,6 +508,11 @@ class ProgramRunner:
             if code == OP_MUL_PLAIN:
                 def step(x=self._ct(ins[0], la), pt=pt, out=self._ct(out, la)):
                     plan.multiply_plain(x, pt, la, out=out)
+            elif code == OP_ADD and len(ins) > 2:
+                xs = (C.c_uint64 * len(ins))(*[_ptr(self._reg(i, la)) for i in ins])
+
+                def step(xs=xs, out=_ptr(self._reg(out, la))):
+                    _check(lib().ckks_poly_sum(plan.handle, C.cast(xs, _p), len(xs), out, 2, la, la * n))
             elif code in (OP_ADD, OP_SUB):
                 def step(fn=plan.add if code == OP_ADD else plan.sub, x=self._reg(ins[0], la),
                          y=self._reg(ins[1], la), out=self._reg(out, la)):

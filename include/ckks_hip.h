@@ -225,6 +225,10 @@ int ckks_poly_mac(const ckks_rns_plan *plan, uint64_t *acc, const uint64_t *x, c
                   size_t n_polys, size_t n_limbs, size_t poly_stride);
 int ckks_poly_add(const ckks_rns_plan *plan, const uint64_t *x, const uint64_t *y,
                   uint64_t *out, size_t n_polys, size_t n_limbs, size_t poly_stride);
+/* out = xs[0] + .. + xs[count - 1] in one pass, count in 1..64 (a host array of
+ * device pointers); out may be one of them. */
+int ckks_poly_sum(const ckks_rns_plan *plan, const uint64_t *const *xs, size_t count, uint64_t *out,
+                  size_t n_polys, size_t n_limbs, size_t poly_stride);
 int ckks_poly_sub(const ckks_rns_plan *plan, const uint64_t *x, const uint64_t *y,
                   uint64_t *out, size_t n_polys, size_t n_limbs, size_t poly_stride);
 int ckks_poly_neg(const ckks_rns_plan *plan, const uint64_t *x, uint64_t *out,

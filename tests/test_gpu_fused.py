@@ -293,3 +293,23 @@ def test_embedding_passes_match_torch(pkg, ctx, logn, polys, scale):
     x = pkg.to_device(_extremes(np.random.default_rng(logn), q, n, polys))
     want = emb.coefficients_to_slots(pkg.encoding.decode_coefficients(plan, x, scale))
     assert torch.equal(pkg.encoding.decode(plan, emb, x, scale), want)
+
+
+@pytest.mark.parametrize("logn,count,polys", [(10, 1, 1), (12, 2, 3), (13, 16, 2), (11, 64, 1)])
+def test_sums_of_many_match_additions(pkg, ctx, logn, count, polys):
+    import ctypes as C
+    import torch
+
+    n = 1 << logn
+    q = _moduli(pkg, n, MIXES["wide"])
+    rng = np.random.default_rng(count)
+    plan = pkg.PreparedRnsNttPlan(ctx, q, n)
+    xs = [pkg.to_device(_extremes(rng, q, n, polys)) for _ in range(count)]
+    want = xs[0].clone()
+    for x in xs[1:]:
+        plan.add(want, x, want)
+    arr = (C.c_uint64 * count)(*[x.data_ptr() for x in xs])
+    for out in (pkg.empty(tuple(want.shape)), xs[-1]):
+        assert pkg.lib().ckks_poly_sum(plan.handle, C.cast(arr, C.c_void_p), count, C.c_void_p(out.data_ptr()), polys,
+                                       len(q), len(q) * n) == 0
+        assert torch.equal(out, want)

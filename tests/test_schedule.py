@@ -91,3 +91,24 @@ def test_baby_and_giant_steps_go_out_together():
     assert [c for c in sizes if c[0] == S.OP_ROTATE] == [(S.OP_ROTATE, 15)] * 2
     assert [c for c in sizes if c[0] in (S.OP_NTT, S.OP_INTT)] == [(S.OP_NTT, 16), (S.OP_INTT, 16)]
     assert not [c for c in sizes if c[0] == S.OP_COPY]
+
+
+def test_merged_additions_give_the_same_sums():
+    for seed in range(200):
+        rng = random.Random(seed)
+        rows = 6
+        groups = []
+        for i in range(rng.randint(1, 80)):
+            a, b = rng.randrange(rows), rng.randrange(rows)
+            out = a if rng.random() < 0.8 else rng.randrange(rows)
+            code = S.OP_ADD if rng.random() < 0.9 else S.OP_SUB
+            groups.append((code, 9 - (rng.random() < 0.05), [(out, [a, b], (code, out, a, b, None, 0, None))]))
+        merged = S.merge_sums(groups)
+        plain, fused = [1 << (8 * i) for i in range(rows)], [1 << (8 * i) for i in range(rows)]
+        for regs, gs in ((plain, groups), (fused, merged)):
+            for code, _, [(out, ins, _)] in gs:
+                assert len(ins) <= 64
+                regs[out] = sum(regs[i] for i in ins) if code == S.OP_ADD else regs[ins[0]] - regs[ins[1]]
+        assert plain == fused
+    chain = [(S.OP_ADD, 8, [(1, [1, r], None)]) for r in range(2, 17)]
+    assert S.merge_sums(chain) == [(S.OP_ADD, 8, [(1, [1] + list(range(2, 17)), None)])]

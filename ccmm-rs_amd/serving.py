@@ -10,6 +10,7 @@ budget, and batches the same op of different jobs into one launch.
 from __future__ import annotations
 
 import ctypes as C
+import operator
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -420,7 +421,8 @@ class ProgramRunner:
     keys must belong to the plan's context; each run switches that context
     to the runner's own (non-null, default-priority) stream and back, which
     waits for the run.  The first run() sizes every library workspace, so
-    run() must precede capture(); nothing is allocated while capturing."""
+    run() must precede capture(); nothing is allocated while capturing.  A
+    program changed after a run is planned anew by the next one."""
 
     # rows of results that wait for others of their kind, and the library's
     # workspaces per group grow with them: bounded at large degrees, where a
@@ -436,16 +438,26 @@ class ProgramRunner:
         n = plan.degree
         self.per = 2 * self.L * n
         self.spare = max(0, min(2 * _TOGETHER, self._SPARE_BYTES // (8 * self.per) - 1))
-        self.limbs = program.register_limbs(self.L)
         self._plan_ops()
         self.regs = torch.empty((max(self.rows, program.n_regs + 2), self.per), dtype=torch.int64, device="cuda")
         self.graph = None
 
     def _plan_ops(self):
-        groups, self.rows = schedule(self.prog, self.L, self.spare)
+        prog = self.prog
+        self.planned = list(prog.ops), (prog.n_regs, prog.n_inputs, prog.out_reg)
+        self.limbs = prog.register_limbs(self.L)
+        groups, self.rows = schedule(prog, self.L, self.spare)
         self.groups = merge_sums(groups)
-        self.planned = len(self.prog.ops)
         self.calls = None
+
+    def _stale(self):
+        """Whether the program differs from the planned one.  An op is a tuple,
+        the same as long as it is the same object; one that could change in
+        place is not taken for the same.  What an op refers to (a key's handle,
+        a plaintext's address, the list of a mac_plain) is read on every run."""
+        prog, (ops, shape) = self.prog, self.planned
+        return (len(ops) != len(prog.ops) or shape != (prog.n_regs, prog.n_inputs, prog.out_reg)
+                or not all(map(operator.is_, prog.ops, ops)) or any(type(op) is not tuple for op in ops))
 
     def _reg(self, i, limbs):
         return self.regs[i, : 2 * limbs * self.plan.degree]
@@ -487,20 +499,19 @@ class ProgramRunner:
             # sums of the same ciphertexts share a call
             shared = {}
             for out, ins, op in items:
-                if not ins or len(ins) != len(op[6]):
-                    raise ValueError("one plaintext per ciphertext, at least one term")
-                shared.setdefault(tuple(ins), []).append((_ptr(self._reg(out, la)),
-                                                          [_ptr(t, la * n, name="pt") for t in op[6]]))
-            sums = []
-            for ins, group in shared.items():
-                sums.append(((C.c_uint64 * len(ins))(*[_ptr(self._reg(i, la)) for i in ins]),
-                             (C.c_uint64 * (len(ins) * len(group)))(*[p for _, pts in group for p in pts]),
-                             (C.c_uint64 * len(group))(*[out for out, _ in group])))
+                shared.setdefault(tuple(ins), []).append((_ptr(self._reg(out, la)), op[6]))
+            sums = [([_ptr(self._reg(i, la)) for i in ins], [pts for _, pts in group],
+                     (C.c_uint64 * len(group))(*[out for out, _ in group])) for ins, group in shared.items()]
 
             def accumulate():
-                for ca, pa, oa in sums:
+                for ins, lists, outs in sums:
+                    if not ins or any(len(pts) != len(ins) for pts in lists):
+                        raise ValueError("one plaintext per ciphertext, at least one term")
+                    cts = (C.c_uint64 * len(ins))(*ins)
+                    pts = (C.c_uint64 * (len(ins) * len(lists)))(*[_ptr(t, la * n, name="pt")
+                                                                    for pts in lists for t in pts])
                     _check(lib().ckks_multiply_plain_accumulate_ntt_batch(
-                        plan.handle, C.cast(ca, _p), C.cast(pa, _p), len(ca), C.cast(oa, _p), len(oa), la))
+                        plan.handle, C.cast(cts, _p), C.cast(pts, _p), len(ins), C.cast(outs, _p), len(outs), la))
             return accumulate
         steps = []
         for out, ins, op in items:
@@ -537,9 +548,13 @@ class ProgramRunner:
         return each
 
     def _run_ops(self):
-        if self.planned != len(self.prog.ops):
-            self.spare = self.regs.shape[0] - self.prog.n_regs - 2
+        if self._stale():
+            # the rows there are stay: a captured graph and the caller's views hold them
+            self.spare = max(0, self.regs.shape[0] - self.prog.n_regs - 2)
             self._plan_ops()
+            if max(self.rows, self.prog.n_regs) > self.regs.shape[0]:
+                self.planned = [], ()
+                raise ValueError("the program outgrew the runner's registers")
         if self.calls is None:
             self.calls = [self._call(*g) for g in self.groups]
         for call in self.calls:

@@ -369,22 +369,23 @@ def schedule(prog: Program, n_limbs: int, spare: int):
             oldest += 1
         if oldest < len(todo):
             early = {r: i for r, i in early.items() if i >= todo[oldest][0]}
-    # the registers that outlive the run move to their own rows
+    # the registers that outlive the run move to their own rows: first those
+    # whose row holds nothing another move still reads.  Where none is left, the
+    # moves' rows are the registers' own (as many of them as values to move), so
+    # row n is free: one value steps aside there and its row takes what it awaits
     moves = []
-    at = {r: v.row for r, v in final}
-    for r, _ in final:
-        if at[r] == r:
-            continue
-        for q in at:
-            if q != r and at[q] == r:  # another one sits there: aside first
-                aside = next(x for x in range(n + 2 + spare) if x not in at.values() and x not in at)
-                moves.append((aside, [r], (OP_COPY, q, r, 0, None, 0, None)))
-                used = max(used, aside + 1)
-                for z in at:
-                    if at[z] == r:
-                        at[z] = aside
-        moves.append((r, [at[r]], (OP_COPY, r, at[r], 0, None, 0, None)))
-        at[r] = r
+    pending = {r: v.row for r, v in final if v.row != r}
+    while pending:
+        read = set(pending.values())
+        r = next((r for r in pending if r not in read), None)
+        if r is None:
+            q, row = next(iter(pending.items()))
+            moves.append((n, [row], (OP_COPY, q, row, 0, None, 0, None)))
+            used = max(used, n + 1)
+            pending = {z: n if x == row else x for z, x in pending.items()}
+        else:
+            row = pending.pop(r)
+            moves.append((r, [row], (OP_COPY, r, row, 0, None, 0, None)))
     for m in moves:
         groups.append((OP_COPY, n_limbs, [m]))
     return groups, used

@@ -112,3 +112,49 @@ def test_merged_additions_give_the_same_sums():
         assert plain == fused
     chain = [(S.OP_ADD, 8, [(1, [1, r], None)]) for r in range(2, 17)]
     assert S.merge_sums(chain) == [(S.OP_ADD, 8, [(1, [1] + list(range(2, 17)), None)])]
+
+
+def _outlive(prog, groups, rows):
+    """Runs both orders twice; the registers that outlive a run hold the same."""
+    n = prog.n_regs
+    written, carried = set(), {prog.out_reg}
+    for op in prog.ops:
+        carried.update(r for r in _reads(op) if r not in written)
+        written.add(op[1])
+    regs = [("in", r) for r in range(n)]
+    phys = regs + [None] * (rows - n)
+    for _ in range(2):
+        for op in prog.ops:
+            ins = [regs[r] for r in _reads(op)]
+            regs[op[1]] = ins[0] if op[0] == S.OP_COPY else _apply(op[0], ins, op)
+        for code, _, items in groups:
+            new = [phys[ins[0]] if code == S.OP_COPY else _apply(code, [phys[i] for i in ins], op)
+                   for _, ins, op in items]
+            for (o, _, _), v in zip(items, new):
+                phys[o] = v
+        assert [phys[r] for r in sorted(carried)] == [regs[r] for r in sorted(carried)]
+
+
+@pytest.mark.parametrize("n_regs,n_inputs,out_reg,ops", [
+    # values left in each other's rows and in both rows past the registers
+    (3, 2, 2, [(S.OP_COPY, 2, 0, 0, None, 0, None), (S.OP_ROTATE, 1, 1, 0, None, 1, None),
+               (S.OP_NTT, 0, 2, 0, None, 2, None)]),
+    (4, 4, 1, [(S.OP_MAC_PLAIN, 3, 3, 1, None, 0, None), (S.OP_MUL_PLAIN, 0, 0, 0, None, 1, None),
+               (S.OP_NTT, 1, 0, 0, None, 2, None), (S.OP_ROTATE, 0, 1, 0, None, 3, None),
+               (S.OP_RESCALE, 0, 2, 0, None, 4, None)]),
+])
+def test_final_moves_without_a_spare_row(n_regs, n_inputs, out_reg, ops):
+    prog = S.Program(n_regs=n_regs, out_reg=out_reg, n_inputs=n_inputs, ops=list(ops))
+    groups, rows = S.schedule(prog, 9, 0)
+    assert rows <= n_regs + 2
+    _outlive(prog, groups, rows)
+
+
+def test_every_register_that_outlives_a_run_is_in_its_row():
+    for seed in range(4000):
+        rng = random.Random(seed)
+        n_regs, spare = rng.choice([1, 2, 3, 4, 5, 8]), rng.choice([0, 0, 0, 1, 2, 16])
+        prog = _program(rng, n_regs, rng.randint(0, 40))
+        groups, rows = S.schedule(prog, 9, spare)
+        assert rows <= n_regs + 2 + spare
+        _outlive(prog, groups, rows)

@@ -473,9 +473,9 @@ class ProgramRunner:
             keys = [op[4] for _, _, op in items]
             arr = (GaloisBatchEntry * len(items))()
             for e, (out, (a,), op) in zip(arr, items):
-                key = op[4]
-                p_ct, p_out = key._ct_ptrs(1, [("ct", self._ct(a, la), 2)], self._ct(out, la))
-                e.exponent, e.input, e.output, e.n_cts = op[5], p_ct, p_out, 1
+                key, ct = op[4], self._ct(a, la)
+                e.exponent, e.n_cts = op[5], key._n_cts(ct, 2)
+                e.input, e.output = key._ct_ptrs(e.n_cts, [("ct", ct, 2)], self._ct(out, la))
             ptr = C.cast(arr, _p)
 
             def rotate():

@@ -35,19 +35,6 @@ class _Calls:
         self.log.append(("mac", read(cts, count), read(pts, count * n_outs), read(outs, n_outs)))
 
 
-class _Key:
-    q_limbs = L
-
-    def __init__(self, handle):
-        self.handle = handle
-
-    def _n_cts(self, t, polys):
-        return t.numel() // (polys * self.q_limbs * N)
-
-    def _ct_ptrs(self, n, ins, out):
-        return [t.data_ptr() for _, t, _ in ins] + [out.data_ptr()]
-
-
 class _Plan:
     class ctx:
         handle = 1
@@ -55,6 +42,15 @@ class _Plan:
 
     def multiply_plain(self, x, pt, la, out=None):
         pkg.lib().log.append(("mul", pt.data_ptr()))
+
+
+class _Key(pkg._KeySwitchKey):
+    def __init__(self, handle, q_limbs=L):
+        self._finish_init(_Plan, handle)
+        self.q_limbs = q_limbs
+
+    def close(self):
+        pass
 
 
 @pytest.fixture
@@ -168,3 +164,11 @@ def test_appended_and_removed_ops_run(calls):
     assert _made(runner, calls)[-1][:3] == ("rotate", 13, 125)
     prog.ops.pop()
     assert len(_made(runner, calls)) == n
+
+
+def test_a_rotation_by_a_key_of_other_limbs_is_refused(calls):
+    """As by the key's apply_galois: the register is no batch of its ciphertexts."""
+    prog = S.Program(n_regs=2, out_reg=1)
+    prog.rotate(1, 0, _Key(11, L - 1), 5)
+    with pytest.raises(ValueError):
+        _runner(prog)._run_ops()

@@ -2749,7 +2749,15 @@ int ckks_autotune_key_switch(ckks_ksk *k, size_t n_cts, int *best_engine, int *b
     const int saved_mode = ctx->base_conversion, saved_fusion = ctx->ks_fusion;
     int best_e = CKKS_BASECONV_VALU, best_f = CKKS_KS_FUSION_OFF;
     float best_ms = 0.f;
-    const bool can_fuse = k->plan->logn > 12 && k->plan->logn <= 17;
+    // the modes that run other kernels than CKKS_KS_FUSION_OFF for this key
+    auto applies = [&](int fusion) {
+        switch (fusion) {
+            case CKKS_KS_FUSION_XCD: return fused_rows_apply(k->plan) || small_tiles_apply(k->plan);
+            case CKKS_KS_FUSION_LINEAR: return fused_rows_apply(k->plan);
+            case CKKS_KS_FUSION_INVERSE: return k->plan->logn > 12 && k->plan->logn <= 17 && k->dnum <= 8;
+            default: return true;
+        }
+    };
     auto body = [&]() -> int {
         CK_HIP(hipMemsetAsync(buf, 0, 2 * n_cts * per * sizeof(u64), ctx->stream));
         CK_HIP(hipEventCreate(&e0));
@@ -2758,8 +2766,7 @@ int ckks_autotune_key_switch(ckks_ksk *k, size_t n_cts, int *best_engine, int *b
         for (int engine = CKKS_BASECONV_VALU; engine <= CKKS_BASECONV_MFMA; ++engine) {
             if (engine == CKKS_BASECONV_MFMA && !k->mfma) continue;
             for (int fusion = CKKS_KS_FUSION_OFF; fusion <= CKKS_KS_FUSION_INVERSE; ++fusion) {
-                if (fusion != CKKS_KS_FUSION_OFF && !can_fuse) continue;
-                if (fusion == CKKS_KS_FUSION_INVERSE && k->dnum > 8) continue;
+                if (!applies(fusion)) continue;
                 ctx->base_conversion = engine;
                 ctx->ks_fusion = fusion;
                 int r = key_switch_core(k, in + poly, per, in, nullptr, per, out, per, n_cts);

@@ -170,3 +170,24 @@ def test_split_key_switch_matches_single_stream(pkg, ctx, n_cts):
     finally:
         ctx.set_key_switch_split(ctx.KS_SPLIT_AUTO)
     assert (got[0] == want[0]).all() and (got[1] == want[1]).all()
+
+
+@pytest.mark.parametrize("logn,bits,modes", [
+    (12, 60, {0, 1}),        # single pass: LINEAR is XCD, INVERSE has no first pass
+    (13, 60, {0, 1, 2, 3}),
+    (13, 61, {0, 3}),        # from 2^60 up XCD and LINEAR are OFF
+    (12, 61, {0}),
+])
+def test_autotuner_times_the_modes_that_differ(pkg, ctx, logn, bits, modes):
+    n, L = 1 << logn, 3
+    q = pkg.find_ntt_primes(bits, n, 1) + pkg.find_ntt_primes(40, n, L - 1)
+    qp = q + pkg.find_ntt_primes(bits, n, 1, skip=q)
+    rng = np.random.default_rng(logn + bits)
+    plan = pkg.PreparedRnsNttPlan(ctx, qp, n)
+    key = pkg.HybridKeySwitchKey(plan, L, [1] * L, rand_residues(rng, qp, n, L), rand_residues(rng, qp, n, L))
+    ct = pkg.to_device(rand_residues(rng, q, n, polys=4).reshape(2, 2, L, n))
+    want = pkg.to_host(key.apply_galois(ct, 5))
+    engine, fusion, times = key.autotune(2)
+    assert {f for _, f in times} == modes
+    assert times[(engine, fusion)] == min(times.values())
+    assert (pkg.to_host(key.apply_galois(ct, 5)) == want).all()

@@ -6,6 +6,7 @@
 #include "fused.hpp"
 #include "fused_dev.hpp"
 #include "ntt_pass.hpp"
+#include "routes.hpp"
 #include "col_tile.hpp"
 
 namespace ck {
@@ -391,17 +392,13 @@ struct RowGrid {
     unsigned char order[kMaxOrder];
 };
 
-// Tiles halve where whole ones would not give every CU more than one: a lone
-// tile's eight waves compete for issue slots that idle CUs have.  4 ciphertexts
-// at N = 2^13: tensor (72 whole tiles) 29.3 -> 23.0 us, key products of 2 digits
-// (104) 19.4 -> 15.4 us.  Above, whole tiles read keys in longer runs.
-constexpr size_t kHalfTiles = 256;
-static RowGrid row_grid(const ckks_rns_plan *plan, size_t limbs, size_t n_cts, bool xcd) {
+// half: tiles up to which they halve (routes.hpp)
+static RowGrid row_grid(const ckks_rns_plan *plan, size_t limbs, size_t n_cts, bool xcd, size_t half = kHalfTiles) {
     RowGrid g{};
     g.n_cts = (u32)n_cts;
     g.limbs = (u32)limbs;
     g.logn = plan->logn;
-    g.tb = (limbs * n_cts) << (plan->logn - 12) <= kHalfTiles ? 11 : 12;
+    g.tb = limb_tiles(limbs, n_cts, plan->logn) <= half ? 11 : 12;
     g.groups = (u32)(limbs << (plan->logn - g.tb));
     g.xcd = xcd ? 1u : 0u;
     limb_order(plan, limbs, g.order);
@@ -624,7 +621,7 @@ int launch_row_mac(ckks_context *ctx, RowMac &m) {
     }
     a.count = (u32)m.count;
     a.primes = m.plan->d_primes;
-    a.grid = row_grid(m.plan, m.limbs, n_cts, m.xcd_order);
+    a.grid = row_grid(m.plan, m.limbs, n_cts, m.xcd_order, row_mac_half_tiles(ntt_n2(m.plan->logn)));
     a.dnum = (u32)m.dnum;
     if ((u64)m.limbs * n_cts << (m.plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "key-switch batch too large for one launch");
@@ -977,7 +974,7 @@ int launch_row_rotate(ckks_context *ctx, const RowRotate &r) {
     a.count = (u32)r.count;
     a.dnum = (u32)r.dnum;
     a.q_limbs = (u32)r.q_limbs;
-    a.grid = row_grid(r.plan, r.limbs, r.n_cts * r.count, true);
+    a.grid = row_grid(r.plan, r.limbs, r.n_cts * r.count, true, row_rotate_half_tiles(r.dnum, ntt_n2(r.plan->logn)));
     if ((u64)r.limbs * r.n_cts * r.count << (r.plan->logn - 12) >= (1ull << 30))
         return fail(CKKS_ERR_INVALID, "NTT batch too large for one launch");
     const dim3 g(row_blocks(a.grid)), t(1u << (a.grid.tb - 3));

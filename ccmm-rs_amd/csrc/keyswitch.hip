@@ -26,6 +26,7 @@
 #include "fused_dev.hpp"
 #include "host_math.hpp"
 #include "internal.hpp"
+#include "routes.hpp"
 
 namespace ck {
 
@@ -102,7 +103,7 @@ struct ckks_ksk {
     unsigned base_log = 0, bounded_words = 0;
     ck::u64 *d_bounded = nullptr;  // table blob (BoundedTable points into it)
     int tuned_engine = CKKS_BASECONV_VALU;  // engine of CKKS_BASECONV_AUTO for this key
-    int tuned_fusion = CKKS_KS_FUSION_XCD;  // mode of CKKS_KS_FUSION_AUTO for this key (see ks_fused)
+    int tuned_fusion = CKKS_KS_FUSION_AUTO;  // mode of CKKS_KS_FUSION_AUTO for this key; AUTO: by shape (ks_fused)
     int tuned_split = CKKS_KS_SPLIT_OFF;    // mode of CKKS_KS_SPLIT_AUTO for this key
     // hoisted rotations: key entries [2][D][B][N] permuted by k^-1, per k,
     // at most kHoistKeyCacheMax of them; hoist_lru lists the exponents most
@@ -2168,25 +2169,39 @@ static bool hoisted_mac_fused(const ckks_context *ctx, u32 logn, size_t dnum) {
     return logn > 12 && logn <= 17 && dnum <= 8 && ctx->ks_fusion == CKKS_KS_FUSION_INVERSE;
 }
 
-// CKKS_KS_FUSION_XCD / LINEAR (XCD for an untuned key): the digits' forward
-// row pass, the key MAC and the inverse row pass of both sums run in one
-// kernel per tile (launch_row_mac), between the two column passes; neither
-// the NTT-domain digits nor the sums reach HBM.  Degrees up to 2^12: ks_small;
-// primes from 2^60 up take the separate kernels.
+// CKKS_KS_FUSION_XCD / LINEAR: the digits' forward row pass, the key MAC and the
+// inverse row pass of both sums run in one kernel per tile (launch_row_mac),
+// between the two column passes; neither the NTT-domain digits nor the sums
+// reach HBM.  Degrees up to 2^12: ks_small; primes from 2^60 up take the
+// separate kernels.  Untuned keys (AUTO) in XCD order where that pays for the
+// n_cts ciphertexts of the launch.
 static int ks_fusion(const ckks_ksk *k) {
     const ckks_context *ctx = k->ctx;
     return ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;
 }
-static bool ks_fused(const ckks_ksk *k) {
+static bool ks_fused(const ckks_ksk *k, size_t n_cts) {
+    if (!fused_rows_apply(k->plan)) return false;
     const int f = ks_fusion(k);
-    return (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && fused_rows_apply(k->plan);
+    if (f == CKKS_KS_FUSION_AUTO) return row_mac_pays(k->dnum, limb_tiles(k->limbs, n_cts, k->plan->logn));
+    return f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR;
+}
+
+// Hoisted rotations of n_cts ciphertexts by several exponents through
+// launch_row_rotate.  The autotuner times single key switches: its choice says
+// nothing here.
+static bool ks_rotates(const ckks_ksk *k, size_t n_cts, size_t exponents) {
+    if (!fused_rows_apply(k->plan)) return false;
+    const int f = k->ctx->ks_fusion;
+    if (f == CKKS_KS_FUSION_AUTO)
+        return row_rotate_pays(k->dnum, k->limbs, n_cts * exponents, exponents, k->plan->logn);
+    return f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR;
 }
 
 // The same switch at single-pass degrees: the digits' transforms read
 // single-limb blocks themselves, the inverse transforms form the products.
 static bool ks_small(const ckks_ksk *k) {
     const int f = ks_fusion(k);
-    return (f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR) && small_tiles_apply(k->plan);
+    return f != CKKS_KS_FUSION_OFF && f != CKKS_KS_FUSION_INVERSE && small_tiles_apply(k->plan);
 }
 
 // What a fused key switch of n_cts ciphertexts hands its forward column pass:
@@ -2246,9 +2261,9 @@ static int launch_garner(const KsJob *const *jobs, size_t count, hipStream_t s) 
 
 // Residues of the digit buffer per ciphertext.  Fused: the column pass's input
 // (see ks_lift), reused for the two sums the row passes write.
-static size_t ks_digit_residues(const ckks_ksk *k, size_t n_cts) {
+static size_t ks_digit_residues(const ckks_ksk *k, size_t n_cts, bool fused) {
     const size_t full = k->dnum * k->limbs;
-    if (!ks_fused(k)) return full * k->degree;
+    if (!fused) return full * k->degree;
     const ColKind lift = ks_lift(k, n_cts);
     const size_t in = lift == kColPlain ? full : lift == kColBlock ? k->q_limbs : k->dnum;
     return std::max(in, 2 * k->limbs) * k->degree;
@@ -2306,7 +2321,7 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
     if (!rc)
         rc = ks_by_shape(jobs, count, [&](const std::vector<size_t> &grp) {
             const ckks_ksk *k = jobs[grp[0]]->k;
-            RowMac m{k->plan, k->dnum, k->limbs, ks_fusion(k) == CKKS_KS_FUSION_XCD, grp.size()};
+            RowMac m{k->plan, k->dnum, k->limbs, ks_fusion(k) != CKKS_KS_FUSION_LINEAR, grp.size()};
             for (size_t g = 0; g < grp.size(); ++g) {
                 const KsJob &j = *jobs[grp[g]];
                 m.e[g] = RowMacJob{fwd[grp[g]].out, j.k->d_kb, j.k->d_ka, j.digits, (u32)j.n_cts, 0};
@@ -2349,7 +2364,7 @@ static u64 galois_inverse(u64 k, u64 two_n) {
     return inv & (two_n - 1);
 }
 
-// Steps 2 to 4 of hoisted jobs whose keys are fused (ks_fused) and which share
+// Steps 2 to 4 of hoisted jobs that are fused (ks_rotates) and which share
 // their digits, key shape and plan: sums into each job's mac_out, inverse
 // column pass into its accumulators.
 static int ks_rotate_middle(ckks_context *ctx, const KsJob *const *jobs, size_t count) {
@@ -2386,7 +2401,8 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
     const bool two_pass = logn > 12 && logn <= 17;
     const bool hoist_fused = hm && !hm->bhat && hoisted_mac_fused(ctx, logn, D);
     // hoisted: slot 4 holds the unpermuted MAC output instead of the digits
-    const size_t slot4 = hm ? n_cts * 2 * B * N : n_cts * ks_digit_residues(k, n_cts);
+    const bool fused = hm ? ks_rotates(k, n_cts, 1) : ks_fused(k, n_cts);
+    const size_t slot4 = hm ? n_cts * 2 * B * N : n_cts * ks_digit_residues(k, n_cts, fused);
     if (!hoist_fused && (rc = ctx->workspace(4, slot4 * sizeof(u64), &wd))) return rc;
     if ((rc = ctx->workspace(5, n_cts * 2 * B * N * sizeof(u64), &wa))) return rc;
     KsJob j{k, x, x_stride, add0, add1, add_stride, out, out_stride, n_cts, galois_kinv, hoisted, hm};
@@ -2394,8 +2410,8 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
     j.acc = (u64 *)wa;
     j.mac_out = hm ? (u64 *)wd : j.acc;
     j.mfma = ks_uses_mfma(k);
-    j.raw = !hm && ks_fused(k);
-    if (!hm && ks_fused(k)) {
+    j.raw = !hm && fused;
+    if (!hm && fused) {
         void *wc;
         if ((rc = ctx->workspace(0, n_cts * D * B * N * sizeof(u64), &wc))) return rc;
         const KsJob *jp = &j;
@@ -2407,7 +2423,7 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
         if ((rc = ks_small_middle(ctx, &jp, 1))) return rc;
         return ks_moddown(j, s);
     }
-    if (hm && ks_fused(k)) {
+    if (hm && fused) {
         const KsJob *jp = &j;
         if ((rc = ks_rotate_middle(ctx, &jp, 1))) return rc;
         return ks_moddown(j, s);
@@ -2453,8 +2469,14 @@ struct KsMultiEntry {
 static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t count) {
     if (count > 16) return fail(CKKS_ERR_INVALID, "a key-switch batch holds at most 16 entries");
     size_t dig = 0, acc = 0;
+    // by the ciphertexts of every entry that shares its launches
+    std::vector<char> rows(count);
     for (size_t i = 0; i < count; ++i) {
-        dig += e[i].n_cts * ks_digit_residues(e[i].k, e[i].n_cts);
+        size_t together = 0;
+        for (size_t m = 0; m < count; ++m)
+            if (e[m].k->plan == e[i].k->plan && e[m].k->dnum == e[i].k->dnum) together += e[m].n_cts;
+        rows[i] = ks_fused(e[i].k, together);
+        dig += e[i].n_cts * ks_digit_residues(e[i].k, e[i].n_cts, rows[i]);
         acc += e[i].n_cts * 2 * e[i].k->limbs * e[i].k->degree;
         ckks_execution_profile &pc = ctx->counts();
         pc.key_switches += e[i].n_cts;
@@ -2478,12 +2500,12 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
         j.digits = pd;
         j.acc = j.mac_out = pa;
         j.mfma = ks_uses_mfma(k);
-        j.raw = ks_fused(k);
-        pd += e[i].n_cts * ks_digit_residues(k, e[i].n_cts);
+        j.raw = rows[i];
+        pd += e[i].n_cts * ks_digit_residues(k, e[i].n_cts, rows[i]);
         pa += e[i].n_cts * 2 * B * N;
         fwd[i] = NttCall{k->plan, j.digits, j.digits, e[i].n_cts * k->dnum, B, B * N, B * N};
         inv[i] = NttCall{k->plan, j.acc, j.acc, e[i].n_cts * 2, B, B * N, B * N};
-        if (!ks_fused(k) && !ks_small(k) && (rc = ks_decompose(j, s))) return rc;
+        if (!rows[i] && !ks_small(k) && (rc = ks_decompose(j, s))) return rc;
     }
     // fused entries (ks_fused) share one launch per column pass, the others
     // one launch per pass of the whole transforms
@@ -2493,7 +2515,7 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
     for (size_t i = 0; i < count; ++i) {
         if (ks_small(e[i].k)) {
             small.push_back(&jobs[i]);
-        } else if (ks_fused(e[i].k)) {
+        } else if (rows[i]) {
             fused.push_back(&jobs[i]);
             cols += e[i].n_cts * e[i].k->dnum * e[i].k->limbs * e[i].k->degree;
         } else {
@@ -2509,7 +2531,7 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
     if ((rc = ks_small_middle(ctx, small.data(), small.size()))) return rc;
     if ((rc = launch_ntt(ctx, plain.data(), plain.size(), true))) return rc;
     for (size_t i = 0; i < count; ++i)
-        if (!ks_fused(e[i].k) && !ks_small(e[i].k) && (rc = ks_mac(jobs[i], s))) return rc;
+        if (!rows[i] && !ks_small(e[i].k) && (rc = ks_mac(jobs[i], s))) return rc;
     if ((rc = launch_ntt(ctx, back.data(), back.size(), false))) return rc;
     std::vector<const KsJob *> all(count);
     for (size_t i = 0; i < count; ++i) all[i] = &jobs[i];
@@ -3351,7 +3373,7 @@ int ckks_rotate_hoisted_batch(ckks_context *ctx, const ckks_hoisted_rotation *e,
     // every entry's MAC in the first inverse pass (CKKS_KS_FUSION_INVERSE), or none
     bool fused = true;
     for (const Fast &f : fast)
-        fused = fused && !ks_fused(f.key) && !f.h->d_bhat && hoisted_mac_fused(ctx, f.key->plan->logn, f.key->dnum);
+        fused = fused && !f.h->d_bhat && hoisted_mac_fused(ctx, f.key->plan->logn, f.key->dnum);
     // the MAC outputs (slot 4, unfused only) and the accumulators (slot 5)
     size_t total = 0;
     for (const Fast &f : fast) total += f.h->n_cts * 2 * f.key->limbs * f.key->degree;
@@ -3391,31 +3413,33 @@ int ckks_rotate_hoisted_batch(ckks_context *ctx, const ckks_hoisted_rotation *e,
     }
     // entries of one hoisted batch share their digit reads: the fused ones in
     // one launch, the others in MACs of up to kMacMaxExp exponents
-    std::vector<bool> done(fast.size(), false);
+    std::vector<bool> done(fast.size(), fused);
+    std::vector<NttCall> rest;
+    if (fused) rest = inv;
     for (size_t i = 0; i < fast.size(); ++i) {
-        const bool rows = ks_fused(fast[i].key);
-        if (done[i] || (fused && !rows)) continue;
-        std::vector<size_t> grp{i};
-        for (size_t m = i + 1; m < fast.size() && (rows || grp.size() < (size_t)kMacMaxExp); ++m)
+        if (done[i]) continue;
+        std::vector<size_t> grp;
+        for (size_t m = i; m < fast.size(); ++m)
             if (!done[m] && fast[m].h == fast[i].h && fast[m].key->dnum == fast[i].key->dnum &&
-                fast[m].key->limbs == fast[i].key->limbs && ks_fused(fast[m].key) == rows) {
+                fast[m].key->limbs == fast[i].key->limbs) {
                 grp.push_back(m);
+                done[m] = true;
             }
-        for (size_t m : grp) done[m] = true;
-        if (rows) {
+        if (ks_rotates(fast[i].key, fast[i].h->n_cts, grp.size())) {
             std::vector<const KsJob *> jp;
             for (size_t m : grp) jp.push_back(&jobs[m]);
             if ((rc = ks_rotate_middle(ctx, jp.data(), jp.size()))) return rc;
-        } else if ((rc = ks_mac_group(jobs, grp, s))) {
-            return rc;
+            continue;
         }
+        for (size_t b = 0; b < grp.size(); b += kMacMaxExp) {
+            const std::vector<size_t> part(grp.begin() + b, grp.begin() + std::min(grp.size(), b + kMacMaxExp));
+            if ((rc = ks_mac_group(jobs, part, s))) return rc;
+        }
+        for (size_t m : grp) rest.push_back(inv[m]);
     }
     // one inverse NTT launch per pass for the entries left, each reading its
     // MAC (computed in the first pass when fused) through its own Galois
     // permutation
-    std::vector<NttCall> rest;
-    for (size_t i = 0; i < fast.size(); ++i)
-        if (!ks_fused(fast[i].key)) rest.push_back(inv[i]);
     if (!rest.empty() && (rc = launch_ntt(ctx, rest.data(), rest.size(), false))) return rc;
     std::vector<const KsJob *> all;
     for (const KsJob &j : jobs) all.push_back(&j);

@@ -99,7 +99,9 @@ int ckks_get_ntt_variant(const ckks_context *ctx, uint32_t logn, int *variant);
  * 2^12 into their Galois-read first inverse pass (off otherwise: slower
  * than the separate MAC, which reads each key entry once per batch).
  * CKKS_KS_FUSION_AUTO (default): the choice ckks_autotune_key_switch made
- * for the key, XCD for an untuned key.  Identical residues in every mode.
+ * for the key; for an untuned key, and for hoisted rotations by any key, XCD or
+ * the separate kernels, by what was faster at such shapes (many digits over few
+ * ciphertexts: separate).  Identical residues in every mode.
  * No reference counterpart. */
 enum {
     CKKS_KS_FUSION_AUTO = -1,

@@ -1,0 +1,97 @@
+"""Key switches and hoisted rotations on both sides of the route rules: the
+same residues by the separate kernels, the fused ones in either order and the
+ones an untuned key takes."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import rand_residues
+
+pytestmark = pytest.mark.gpu
+
+
+def _by_mode(ctx, call):
+    """{mode: residues}, the context left as it was."""
+    out = {}
+    try:
+        for mode in (ctx.KS_FUSION_OFF, ctx.KS_FUSION_XCD, ctx.KS_FUSION_LINEAR, ctx.KS_FUSION_AUTO):
+            ctx.set_key_switch_fusion(mode)
+            out[mode] = call()
+    finally:
+        ctx.set_key_switch_fusion(ctx.KS_FUSION_AUTO)
+    return out
+
+
+@pytest.mark.parametrize("logn,kind,limbs,base_log,cts", [
+    (13, "bounded", 2, 10, 1),   # 11 digits, few tiles: separate
+    (13, "bounded", 2, 10, 4),   # fused
+    (15, "bounded", 2, 8, 2),    # 14 digits
+    (14, "gadget", 6, 0, 1),
+    (16, "gadget", 5, 0, 1),
+    (17, "gadget", 5, 0, 1),     # rotations of a row of 512
+    (17, "gadget", 2, 0, 1),     # whole tiles where half ones were taken
+])
+def test_routes_agree(pkg, ctx, logn, kind, limbs, base_log, cts):
+    import torch
+
+    n = 1 << logn
+    rng = np.random.default_rng(logn * 100 + limbs)
+    if kind == "bounded":
+        m = pkg.find_ntt_primes(55, n, limbs + 1)
+        q = m[:limbs]
+        plan = pkg.PreparedRnsNttPlan(ctx, m, n)
+        d = pkg.bounded_digit_count(plan, limbs, base_log)
+        make = lambda: pkg.BoundedKeySwitchKey(plan, limbs, base_log, rand_residues(rng, m, n, d),
+                                               rand_residues(rng, m, n, d))
+    else:
+        q = pkg.find_ntt_primes(60, n, 1) + pkg.find_ntt_primes(40, n, limbs - 1)
+        plan = pkg.PreparedRnsNttPlan(ctx, q, n)
+        make = lambda: pkg.RnsKeySwitchKey(plan, [1] * limbs, rand_residues(rng, q, n, limbs),
+                                           rand_residues(rng, q, n, limbs))
+    keys = [make() for _ in range(2)]
+    exps = [pow(5, i + 1, 2 * n) for i in range(5)]
+    batches = [pkg.to_device(rand_residues(rng, q, n, 2 * cts).reshape(cts, 2, limbs, n)) for _ in range(2)]
+    digits = [keys[0].hoist(ct) for ct in batches]
+
+    def rotations():
+        outs = [torch.empty_like(batches[0]) for _ in range(7)]
+        # five exponents of one batch, two of another
+        entries = [(digits[i // 5], keys[i % 2], exps[i % 5], batches[i // 5], o) for i, o in enumerate(outs)]
+        pkg.rotate_hoisted_batch(ctx, entries)
+        single = keys[0].rotate_hoisted(digits[0], batches[0], exps[0])
+        return torch.stack(outs + [single])
+
+    def switches():
+        return torch.stack([keys[i % 2].apply_galois(batches[i // 5], exps[i % 5]) for i in range(7)]
+                           + [keys[0].apply_galois(batches[0], exps[0])])
+
+    want = switches()
+    for call in (switches, rotations):
+        for mode, got in _by_mode(ctx, call).items():
+            assert torch.equal(got, want), (call.__name__, mode)
+
+
+def test_entries_of_one_batch_on_both_routes(pkg, ctx):
+    """Entries counted together where they share launches: one alone of its kind
+    on the separate kernels beside fused ones."""
+    import torch
+
+    n, m = 1 << 13, pkg.find_ntt_primes(55, 1 << 13, 3)
+    rng = np.random.default_rng(4)
+    plan = pkg.PreparedRnsNttPlan(ctx, m, n)
+    keys = []
+    for base_log in (10, 10, 10, 8, 30):
+        d = pkg.bounded_digit_count(plan, 2, base_log)
+        keys.append(pkg.BoundedKeySwitchKey(plan, 2, base_log, rand_residues(rng, m, n, d), rand_residues(rng, m, n, d)))
+    cts = [pkg.to_device(rand_residues(rng, m[:2], n, 2 * c).reshape(c, 2, 2, n)) for c in (1, 1, 2, 1, 1)]
+    exps = [5, 25, 125, 625, 3125]
+    want = [k.apply_galois(ct, e) for k, ct, e in zip(keys, cts, exps)]
+
+    def batch():
+        outs = [torch.empty_like(ct) for ct in cts]
+        pkg.apply_galois_batch(ctx, [(k, e, ct, o) for k, e, ct, o in zip(keys, exps, cts, outs)])
+        return outs
+
+    for mode, got in _by_mode(ctx, batch).items():
+        assert all(torch.equal(g, w) for g, w in zip(got, want)), mode

@@ -2096,7 +2096,9 @@ static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
     const ckks_ksk *k = jobs[0]->k;
     const u64 N = k->degree, B = k->limbs, D = k->dnum;
     const u32 chunks = (u32)(N / kKsThreads);
-    if (jobs[0]->mfma && count > 1) {
+    size_t least = jobs[0]->n_cts;
+    for (size_t i = 1; i < count; ++i) least = std::min(least, jobs[i]->n_cts);
+    if (count > 1 && (jobs[0]->mfma || !moddown_together(count, least * 2 * chunks))) {
         for (size_t i = 0; i < count; ++i)
             if (int rc = ks_moddown(jobs + i, 1, s)) return rc;
         return CKKS_OK;

@@ -95,3 +95,22 @@ def test_entries_of_one_batch_on_both_routes(pkg, ctx):
 
     for mode, got in _by_mode(ctx, batch).items():
         assert all(torch.equal(g, w) for g, w in zip(got, want)), mode
+
+
+def test_moddown_of_large_jobs_in_launches_of_their_own(pkg, ctx):
+    import torch
+
+    n, L = 1 << 16, 2
+    q, p = pkg.chain_moduli(L - 1, 1)
+    rng = np.random.default_rng(9)
+    plan = pkg.PreparedRnsNttPlan(ctx, q + p, n)
+    key = pkg.HybridKeySwitchKey(plan, L, [1, 1], rand_residues(rng, q + p, n, 2), rand_residues(rng, q + p, n, 2))
+    ct = pkg.to_device(rand_residues(rng, q, n, 32).reshape(16, 2, L, n))
+    exps = [5, 25, 125]
+    want = [key.apply_galois(ct, e) for e in exps]
+    h = key.hoist(ct)
+    for batch in (lambda outs: pkg.rotate_hoisted_batch(ctx, [(h, key, e, ct, o) for e, o in zip(exps, outs)]),
+                  lambda outs: pkg.apply_galois_batch(ctx, [(key, e, ct, o) for e, o in zip(exps, outs)])):
+        outs = [torch.empty_like(ct) for _ in exps]
+        batch(outs)
+        assert all(torch.equal(o, w) for o, w in zip(outs, want))

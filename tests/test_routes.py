@@ -21,6 +21,7 @@ def emu():
     lib.emu_limb_tiles.restype = C.c_size_t
     lib.emu_half_tiles.argtypes = [C.c_int, C.c_size_t, C.c_uint]
     lib.emu_half_tiles.restype = C.c_size_t
+    lib.emu_moddown_together.argtypes = [C.c_size_t, C.c_size_t]
     return lib
 
 
@@ -60,3 +61,12 @@ def test_hoisted_rotations(emu, dnum, limbs, cts, exps, logn, separate, fused):
 ])
 def test_tile_sizes(emu, rotate, dnum, tiles, logn, whole, half):
     assert (tiles <= emu.emu_half_tiles(rotate, dnum, (logn + 1) // 2)) == (half < whole)
+
+
+# exponents, ciphertexts, log2 N, us in one launch, us in one launch each
+@pytest.mark.parametrize("jobs,cts,logn,together,apart", [
+    (4, 4, 16, 1071.4, 1186.0), (4, 16, 16, 3979.4, 3870.6), (3, 16, 16, 1236.4, 1178.4), (2, 8, 17, 889.8, 895.6),
+    (4, 4, 17, 2272.1, 2395.3), (3, 16, 17, 2599.8, 2478.8), (3, 8, 17, 1375.0, 1317.2),
+])
+def test_moddown_launches(emu, jobs, cts, logn, together, apart):
+    assert emu.emu_moddown_together(jobs, cts * 2 << (logn - 8)) == (together < apart)

@@ -93,8 +93,9 @@ struct ckks_context {
     std::set<ckks_server *> servers;  // destroyed before the keys and plans they use
     // (q, logn) -> device twiddle tables, shared by plans of this context
     std::map<std::pair<uint64_t, uint32_t>, ck::TwiddleTables> tables;
-    // grow-only scratch slots: slot 0 is the NTT's inter-pass buffer, the
-    // others belong to the composite operations (tensor, key switch).
+    // grow-only scratch slots: slot 0 is the inter-pass buffer of the NTT and
+    // of the fused key switch's digits, the others belong to the composite
+    // operations (tensor, products, key switch).
     // two lanes of slots: lane 1 belongs to the auxiliary stream of a key
     // switch whose batch is split in two (see key_switch_core)
     static constexpr int kSlots = 8;
@@ -109,11 +110,12 @@ struct ckks_context {
     // 512 MiB chunks run a lone forward transform 7 % faster than one chunk
     // and the inverse equally fast, but the 64 + 16 ciphertext rotation call
     // gained nothing; 32-128 MiB chunks are slower (each chunk's launches
-    // drain the GPU).
+    // drain the GPU).  Fused key switches cut their batch by ciphertexts to fit
+    // it (ks_fused_chunks).
     size_t ntt_chunk_bytes = 0;
     int base_conversion = CKKS_BASECONV_AUTO;
     uint8_t ntt_variant[32] = {};  // two-pass NTT kernel variant per log2 N
-    int ks_fusion = CKKS_KS_FUSION_AUTO;  // digits' row pass fused with the key MAC
+    int ks_fusion = CKKS_KS_FUSION_AUTO;  // kernels of a key switch between its column passes (ks_fused, ks_rotates)
     bool capturing = false;  // a hipGraph capture of `stream` is open
     // operations run so far (ckks_profile_get); during a capture the counts
     // go to `captured` and are added on each launch of the graph

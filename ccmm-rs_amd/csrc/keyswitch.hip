@@ -2181,8 +2181,14 @@ static int ks_fusion(const ckks_ksk *k) {
     const ckks_context *ctx = k->ctx;
     return ctx->ks_fusion == CKKS_KS_FUSION_AUTO ? k->tuned_fusion : ctx->ks_fusion;
 }
+// Inter-pass residues of one ciphertext's digits (workspace slot 0).
+static size_t ks_column_residues(const ckks_ksk *k) { return k->dnum * k->limbs * k->degree; }
+// A chunk (ckks_set_ntt_chunk_bytes) that holds less than one ciphertext's
+// digits takes the separate kernels, whose transforms it cuts limb by limb.
 static bool ks_fused(const ckks_ksk *k, size_t n_cts) {
     if (!fused_rows_apply(k->plan)) return false;
+    const size_t chunk = k->ctx->ntt_chunk_bytes / sizeof(u64);
+    if (k->ctx->ntt_chunk_bytes && chunk < ks_column_residues(k)) return false;
     const int f = ks_fusion(k);
     if (f == CKKS_KS_FUSION_AUTO) return row_mac_pays(k->dnum, limb_tiles(k->limbs, n_cts, k->plan->logn));
     return f == CKKS_KS_FUSION_XCD || f == CKKS_KS_FUSION_LINEAR;
@@ -2333,6 +2339,50 @@ static int ks_fused_middle(ckks_context *ctx, const KsJob *const *jobs, size_t c
     return rc ? rc : launch_columns(ctx, inv.data(), count, false);
 }
 
+// The same with the inter-pass data in workspace slot 0, within the context's
+// chunk: the ciphertexts of the jobs in turn, as many at a time as fit.
+static int ks_fused_chunks(ckks_context *ctx, const KsJob *const *jobs, size_t count) {
+    size_t total = 0;
+    for (size_t i = 0; i < count; ++i) total += jobs[i]->n_cts * ks_column_residues(jobs[i]->k);
+    size_t cap = ctx->ntt_chunk_bytes / sizeof(u64);
+    if (ctx->ntt_chunk_bytes == 0 || cap > total) cap = total;
+    void *w;
+    if (int rc = ctx->workspace(0, cap * sizeof(u64), &w)) return rc;
+    if (cap == total) return ks_fused_middle(ctx, jobs, count, (u64 *)w);
+    std::vector<KsJob> pieces;
+    size_t used = 0;
+    auto run = [&]() -> int {
+        std::vector<const KsJob *> jp;
+        for (const KsJob &p : pieces) jp.push_back(&p);
+        const int rc = ks_fused_middle(ctx, jp.data(), jp.size(), (u64 *)w);
+        pieces.clear();
+        used = 0;
+        return rc;
+    };
+    for (size_t i = 0; i < count; ++i) {
+        const KsJob &j = *jobs[i];
+        const ckks_ksk *k = j.k;
+        const size_t per = ks_column_residues(k), digits = ks_digit_residues(k, j.n_cts, true);
+        for (size_t c = 0; c < j.n_cts;) {
+            const size_t take = std::min(j.n_cts - c, (cap - used) / per);
+            if (take == 0) {
+                if (int rc = run()) return rc;
+                continue;
+            }
+            KsJob p = j;
+            p.n_cts = take;
+            p.x += c * j.x_stride;
+            p.digits += c * digits;
+            p.acc += c * 2 * k->limbs * k->degree;
+            if (p.hoisted) p.hoisted += c * k->dnum * k->degree;
+            pieces.push_back(p);
+            used += take * per;
+            c += take;
+        }
+    }
+    return run();
+}
+
 // Steps 1 to 4 of ks_small jobs.
 static int ks_small_middle(ckks_context *ctx, const KsJob *const *jobs, size_t count) {
     std::vector<SmallCall> fwd(count), inv(count);
@@ -2414,10 +2464,8 @@ static int key_switch_lane(const ckks_ksk *k, const u64 *x, u64 x_stride, const 
     j.mfma = ks_uses_mfma(k);
     j.raw = !hm && fused;
     if (!hm && fused) {
-        void *wc;
-        if ((rc = ctx->workspace(0, n_cts * D * B * N * sizeof(u64), &wc))) return rc;
         const KsJob *jp = &j;
-        if ((rc = ks_fused_middle(ctx, &jp, 1, (u64 *)wc))) return rc;
+        if ((rc = ks_fused_chunks(ctx, &jp, 1))) return rc;
         return ks_moddown(j, s);
     }
     if (!hm && ks_small(k)) {
@@ -2513,23 +2561,17 @@ static int key_switch_multi(ckks_context *ctx, const KsMultiEntry *e, size_t cou
     // one launch per pass of the whole transforms
     std::vector<const KsJob *> fused, small;
     std::vector<NttCall> plain, back;
-    size_t cols = 0;
     for (size_t i = 0; i < count; ++i) {
         if (ks_small(e[i].k)) {
             small.push_back(&jobs[i]);
         } else if (rows[i]) {
             fused.push_back(&jobs[i]);
-            cols += e[i].n_cts * e[i].k->dnum * e[i].k->limbs * e[i].k->degree;
         } else {
             plain.push_back(fwd[i]);
             back.push_back(inv[i]);
         }
     }
-    if (!fused.empty()) {
-        void *wc;
-        if ((rc = ctx->workspace(0, cols * sizeof(u64), &wc))) return rc;
-        if ((rc = ks_fused_middle(ctx, fused.data(), fused.size(), (u64 *)wc))) return rc;
-    }
+    if (!fused.empty() && (rc = ks_fused_chunks(ctx, fused.data(), fused.size()))) return rc;
     if ((rc = ks_small_middle(ctx, small.data(), small.size()))) return rc;
     if ((rc = launch_ntt(ctx, plain.data(), plain.size(), true))) return rc;
     for (size_t i = 0; i < count; ++i)

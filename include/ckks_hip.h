@@ -65,7 +65,9 @@ int ckks_context_set_stream(ckks_context *ctx, void *stream);
 int ckks_sync(ckks_context *ctx);
 
 /* Tuning: bytes of the NTT inter-pass buffer per chunk of a batched
- * transform (default 0 = the whole batch in one chunk).  Results do not
+ * transform (default 0 = the whole batch in one chunk).  The fused key switch
+ * keeps its digits' inter-pass data within it too, by ciphertexts; a chunk
+ * below one ciphertext's digits takes the separate kernels.  Results do not
  * depend on it.  No reference counterpart. */
 int ckks_set_ntt_chunk_bytes(ckks_context *ctx, size_t bytes);
 

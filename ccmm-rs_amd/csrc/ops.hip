@@ -503,8 +503,7 @@ static int tensor(const ckks_rns_plan *plan, const u64 *ct0, const u64 *ct1, u64
     ckks_context *ctx = plan->ctx;
     void *w1, *w2;
     if ((rc = ctx->workspace(1, n_cts * 4 * poly * sizeof(u64), &w1))) return rc;
-    if ((rc = ctx->workspace(2, n_cts * 3 * poly * sizeof(u64), &w2))) return rc;
-    u64 *x = (u64 *)w1, *y = (u64 *)w2;
+    u64 *x = (u64 *)w1;
     if (fused_rows_apply(plan)) {
         const size_t each = n_cts * poly;
         u64 *const p[4] = {x, x + each, x + 2 * each, x + 3 * each};
@@ -515,6 +514,8 @@ static int tensor(const ckks_rns_plan *plan, const u64 *ct0, const u64 *ct1, u64
         if ((rc = launch_columns(ctx, f, 4, true)) || (rc = launch_row_tensor(ctx, plan, p, n_cts, n_limbs))) return rc;
         return launch_columns(ctx, iv, 3, false);
     }
+    if ((rc = ctx->workspace(2, n_cts * 3 * poly * sizeof(u64), &w2))) return rc;
+    u64 *y = (u64 *)w2;
     // x = [ct][b0, a0, b1, a1][limb][N] in the NTT domain
     NttCall fwd[4] = {
         {plan, ct0, x, n_cts, n_limbs, in_stride, 4 * poly},

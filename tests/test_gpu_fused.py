@@ -313,3 +313,24 @@ def test_sums_of_many_match_additions(pkg, ctx, logn, count, polys):
         assert pkg.lib().ckks_poly_sum(plan.handle, C.cast(arr, C.c_void_p), count, C.c_void_p(out.data_ptr()), polys,
                                        len(q), len(q) * n) == 0
         assert torch.equal(out, want)
+
+
+def test_a_tensor_keeps_only_its_factors(pkg):
+    """The products take the place of the factors: four polynomials a pair in
+    workspaces, no second buffer."""
+    import torch
+
+    n, cts = 1 << 14, 64
+    c = pkg.Context(0)
+    q, _ = pkg.chain_moduli(7, 0)
+    plan = pkg.PreparedRnsNttPlan(c, q, n)
+    poly = len(q) * n * 8
+    ct = torch.zeros((cts, 2, len(q), n), dtype=torch.int64, device="cuda")
+    out = torch.empty((cts, 3, len(q), n), dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    plan.tensor(ct, ct, len(q), out=out)
+    torch.cuda.synchronize()
+    grown = before - torch.cuda.mem_get_info()[0]
+    c.close()
+    assert grown < 5 * cts * poly, grown

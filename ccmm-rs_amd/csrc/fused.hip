@@ -606,7 +606,7 @@ __global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_mac(Row
     if (P.fp)
         RowMacBody<L, TB, RowFp, SumFp>{a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, threadIdx.x}.run(blk);
     else
-        RowMacBody<L, TB, RowInt, SumInt>{a, P, RowInt{P.q}, SumInt(P), lds, threadIdx.x}.run(blk);
+        RowMacBody<L, TB, RowInt, SumInt>{a, P, RowInt{P.q}, SumInt(P.q, P.br_hi, P.br_lo), lds, threadIdx.x}.run(blk);
 }
 
 int launch_row_mac(ckks_context *ctx, RowMac &m) {
@@ -718,7 +718,7 @@ __global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_mul(Row
     if (P.fp)
         row_mul_tile<L, INTER, R>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
     else
-        row_mul_tile<L, INTER, R>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+        row_mul_tile<L, INTER, R>(a, P, RowInt{P.q}, SumInt(P.q, P.br_hi, P.br_lo), lds, blk);
 }
 
 int launch_row_mul(ckks_context *ctx, const RowMul &m) {
@@ -813,7 +813,7 @@ __global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_tensor(
     if (P.fp)
         row_tensor_tile<L, R>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
     else
-        row_tensor_tile<L, R>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+        row_tensor_tile<L, R>(a, P, RowInt{P.q}, SumInt(P.q, P.br_hi, P.br_lo), lds, blk);
 }
 
 int launch_row_tensor(ckks_context *ctx, const ckks_rns_plan *plan, u64 *const x[4], size_t n_cts, size_t limbs) {
@@ -960,7 +960,7 @@ __global__ __launch_bounds__(1 << (TB - 3), TB == 11 ? 2 : 4) void k_row_rotate(
     if (P.fp)
         row_rotate_tile<L, R>(a, P, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, lds, blk);
     else
-        row_rotate_tile<L, R>(a, P, RowInt{P.q}, SumInt(P), lds, blk);
+        row_rotate_tile<L, R>(a, P, RowInt{P.q}, SumInt(P.q, P.br_hi, P.br_lo), lds, blk);
 }
 
 int launch_row_rotate(ckks_context *ctx, const RowRotate &r) {

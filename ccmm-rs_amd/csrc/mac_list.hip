@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_mac_lists(MacLists a) {
     if (P.fp)
         mac_thread<E>(a, RowFp{P.qd, P.qinv}, SumFp{P.qd, P.qinv}, limb, n, e0);
     else
-        mac_thread<E>(a, RowInt{P.q}, SumInt(P), limb, n, e0);
+        mac_thread<E>(a, RowInt{P.q}, SumInt(P.q, P.br_hi, P.br_lo), limb, n, e0);
 }
 
 int launch_mac_lists(const ckks_rns_plan *plan, const u64 *const *cts, const u64 *const *pts, size_t count,

@@ -210,7 +210,7 @@ __global__ __launch_bounds__(512, 4) void k_small(SmallLaunch l) {
         else small_forward<L, EXTRA>(e, P, in, limb, poly, lds);
     } else {
         if (P.fp) small_inverse<L, EXTRA>(e, P, fp, SumFp{P.qd, P.qinv}, limb, poly, lds);
-        else small_inverse<L, EXTRA>(e, P, in, SumInt(P), limb, poly, lds);
+        else small_inverse<L, EXTRA>(e, P, in, SumInt(P.q, P.br_hi, P.br_lo), limb, poly, lds);
     }
 }
 

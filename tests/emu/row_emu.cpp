@@ -8,6 +8,8 @@
 #include "../../ccmm-rs_amd/csrc/host_math.hpp"
 #include "../../ccmm-rs_amd/csrc/ntt_pass.hpp"
 #include "../../ccmm-rs_amd/csrc/col_tile.hpp"
+#include "../../ccmm-rs_amd/csrc/row_sums.hpp"
+#include "../../ccmm-rs_amd/csrc/small_tile.hpp"
 
 using namespace ck;
 
@@ -50,19 +52,19 @@ u64 lazy(u64 x, const RowFp &) { return f64_as_u64((double)x); }
 u64 lazy(u64 x, const RowInt &) { return x; }
 
 // forward: inter-pass data -> natural-order values; inverse the other way.
-template <int L, class Ar>
+template <int L, int TB, class Ar>
 void row_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward) {
-    typedef RowTile<L> R;
+    typedef RowTile<L, TB> R;
     const u32 n1 = p.logn - L;
-    static u64 v[512][8];
-    alignas(16) static u64 lds[RowTile<L>::LDS];
-    for (u32 tile = 0; tile < (1u << (p.logn - 12)); ++tile) {
+    static u64 v[R::THREADS][8];
+    alignas(16) static u64 lds[R::LDS];
+    for (u32 tile = 0; tile < (1u << (p.logn - TB)); ++tile) {
         int b[8], bx[8];
         auto each = [&](auto &&f) {
-            for (u32 tid = 0; tid < 512; ++tid) f(tid);
+            for (u32 tid = 0; tid < R::THREADS; ++tid) f(tid);
         };
         auto rounds = [&](auto &&f) {
-            for (u32 tid = 0; tid < 512; ++tid) {
+            for (u32 tid = 0; tid < R::THREADS; ++tid) {
                 std::memcpy(bx, b, sizeof b);
                 f(tid);
             }
@@ -130,20 +132,20 @@ void row_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward
 
 // forward: coefficients -> inter-pass residues (canonical here), without the
 // row products; inverse the other way, times N^-1.
-template <int K1, class Ar>
+template <int K1, int B, class Ar>
 void col_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward, int bound) {
-    typedef ColTile<K1> C;
+    typedef ColTile<K1, B> C;
     const u32 n2 = p.logn - K1;
     const u64 q = p.q, ninv = host::invmod((1ull << p.logn) % q, q), ninv_q = host::shoup_quotient(ninv, q);
-    static u64 v[256][16];
+    static u64 v[C::THREADS][C::M];
     static u64 lds[4096];
     for (u32 tile = 0; tile < (1u << (p.logn - 12)); ++tile) {
-        int b[16], bx[16];
+        int b[C::M], bx[C::M];
         auto each = [&](auto &&f) {
-            for (u32 tid = 0; tid < 256; ++tid) f(tid);
+            for (u32 tid = 0; tid < C::THREADS; ++tid) f(tid);
         };
         auto rounds = [&](auto &&f) {
-            for (u32 tid = 0; tid < 256; ++tid) {
+            for (u32 tid = 0; tid < C::THREADS; ++tid) {
                 std::memcpy(bx, b, sizeof b);
                 f(tid);
             }
@@ -154,7 +156,7 @@ void col_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward
         C::set(b, bound);
         if (forward) {
             each([&](u32 t) {
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < C::M; ++i) {
                     const u32 o = C::template offset<0>(tile, n2, t, i);
                     CK_BOUNDS(o, 1u << p.logn);
                     v[t][i] = lazy(in[o], ar);
@@ -165,24 +167,36 @@ void col_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward
             each([&](u32 t) { C::template get<1>(v[t], t, lds); });
             C::level(b);
             rounds([&](u32 t) { C::template fwd<1>(v[t], bx, t, tw, ar); });
+            if constexpr (C::LAST == 2) {
+                each([&](u32 t) { C::template put<1>(v[t], t, lds); });
+                each([&](u32 t) { C::template get<2>(v[t], t, lds); });
+                C::level(b);
+                rounds([&](u32 t) { C::template fwd<2>(v[t], bx, t, tw, ar); });
+            }
             each([&](u32 t) {
-                for (int i = 0; i < 16; ++i) {
-                    const u32 o = C::template offset<1>(tile, n2, t, i);
+                for (int i = 0; i < C::M; ++i) {
+                    const u32 o = C::template offset<C::LAST>(tile, n2, t, i);
                     CK_BOUNDS(o, 1u << p.logn);
                     out[o] = canonical(v[t][i], ar);
                 }
             });
         } else {
             each([&](u32 t) {
-                for (int i = 0; i < 16; ++i) v[t][i] = lazy(in[C::template offset<1>(tile, n2, t, i)], ar);
+                for (int i = 0; i < C::M; ++i) v[t][i] = lazy(in[C::template offset<C::LAST>(tile, n2, t, i)], ar);
             });
+            if constexpr (C::LAST == 2) {
+                rounds([&](u32 t) { C::template inv<2>(v[t], bx, t, tw, ar); });
+                each([&](u32 t) { C::template put<2>(v[t], t, lds); });
+                each([&](u32 t) { C::template get<1>(v[t], t, lds); });
+                C::level(b);
+            }
             rounds([&](u32 t) { C::template inv<1>(v[t], bx, t, tw, ar); });
             each([&](u32 t) { C::template put<1>(v[t], t, lds); });
             each([&](u32 t) { C::template get<0>(v[t], t, lds); });
             C::level(b);
             rounds([&](u32 t) { C::template inv<0>(v[t], bx, t, tw, ar); });
             each([&](u32 t) {
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < C::M; ++i) {
                     const u32 o = C::template offset<0>(tile, n2, t, i);
                     CK_BOUNDS(o, 1u << p.logn);
                     out[o] = shoup(canonical(v[t][i], ar), ninv, ninv_q, q);
@@ -192,14 +206,84 @@ void col_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward
     }
 }
 
-template <class Ar>
+// TB: 12, or 11 for the halved tiles of small launches
+template <int TB = 12, class Ar>
 int run(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward) {
     switch (ntt_n2(p.logn)) {
-        case 7: row_pass<7>(p, ar, in, out, forward); return 0;
-        case 8: row_pass<8>(p, ar, in, out, forward); return 0;
-        case 9: row_pass<9>(p, ar, in, out, forward); return 0;
+        case 7: row_pass<7, TB>(p, ar, in, out, forward); return 0;
+        case 8: row_pass<8, TB>(p, ar, in, out, forward); return 0;
+        case 9: row_pass<9, TB>(p, ar, in, out, forward); return 0;
         default: return -1;
     }
+}
+
+// A whole transform of a single-pass degree, natural order both ways.
+template <int L, class Ar>
+void small_pass(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward, int bound) {
+    typedef SmallTile<L> S;
+    const u64 q = p.q, ninv = host::invmod((1ull << L) % q, q), ninv_q = host::shoup_quotient(ninv, q);
+    static u64 v[S::THREADS][8];
+    static u64 lds[2][S::LDS];
+    int b[8], bx[8];
+    auto each = [&](auto &&f) {
+        for (u32 tid = 0; tid < S::THREADS; ++tid) f(tid);
+    };
+    auto rounds = [&](auto &&f) {
+        for (u32 tid = 0; tid < S::THREADS; ++tid) {
+            std::memcpy(bx, b, sizeof b);
+            f(tid);
+        }
+        std::memcpy(b, bx, sizeof b);
+    };
+    const Tw *tw = p.tw(forward);
+    std::memset(lds, 0xA5, sizeof lds);
+    each([&](u32 t) {
+        for (int i = 0; i < 8; ++i) v[t][i] = lazy(in[t + i * S::THREADS], ar);
+    });
+    S::set(b, bound);
+    // the kernels' exchanges: the buffers take turns
+    if (forward) {
+        rounds([&](u32 t) { S::template fwd<0>(v[t], bx, S::template twiddles<0>(tw, t), ar); });
+        each([&](u32 t) { S::template put<0>(v[t], t, lds[0]); });
+        each([&](u32 t) { S::template get<1>(v[t], t, lds[0]); });
+        S::level(b);
+        rounds([&](u32 t) { S::template fwd<1>(v[t], bx, S::template twiddles<1>(tw, t), ar); });
+        each([&](u32 t) { S::template put<1>(v[t], t, lds[1]); });
+        each([&](u32 t) { S::template get<2>(v[t], t, lds[1]); });
+        S::level(b);
+        rounds([&](u32 t) { S::template fwd<2>(v[t], bx, S::template twiddles<2>(tw, t), ar); });
+        each([&](u32 t) { S::template put<2>(v[t], t, lds[0]); });
+        each([&](u32 t) { S::template get<3>(v[t], t, lds[0]); });
+        S::level(b);
+        rounds([&](u32 t) { S::template fwd<3>(v[t], bx, S::template twiddles<3>(tw, t), ar); });
+        each([&](u32 t) {
+            for (int i = 0; i < 8; ++i) v[t][i] = canonical(v[t][i], ar);
+            S::template put<3>(v[t], t, lds[1]);
+        });
+        each([&](u32 t) { S::get_natural(v[t], t, lds[1]); });
+    } else {
+        each([&](u32 t) { S::put_natural(v[t], t, lds[0]); });
+        each([&](u32 t) { S::template get<3>(v[t], t, lds[0]); });
+        rounds([&](u32 t) { S::template inv<3>(v[t], bx, S::template twiddles<3>(tw, t), ar); });
+        each([&](u32 t) { S::template put<3>(v[t], t, lds[1]); });
+        each([&](u32 t) { S::template get<2>(v[t], t, lds[1]); });
+        S::level(b);
+        rounds([&](u32 t) { S::template inv<2>(v[t], bx, S::template twiddles<2>(tw, t), ar); });
+        each([&](u32 t) { S::template put<2>(v[t], t, lds[0]); });
+        each([&](u32 t) { S::template get<1>(v[t], t, lds[0]); });
+        S::level(b);
+        rounds([&](u32 t) { S::template inv<1>(v[t], bx, S::template twiddles<1>(tw, t), ar); });
+        each([&](u32 t) { S::template put<1>(v[t], t, lds[1]); });
+        each([&](u32 t) { S::template get<0>(v[t], t, lds[1]); });
+        S::level(b);
+        rounds([&](u32 t) { S::template inv<0>(v[t], bx, S::template twiddles<0>(tw, t), ar); });
+        each([&](u32 t) {
+            for (int i = 0; i < 8; ++i) v[t][i] = shoup(canonical(v[t][i], ar), ninv, ninv_q, q);
+        });
+    }
+    each([&](u32 t) {
+        for (int i = 0; i < 8; ++i) out[t + i * S::THREADS] = v[t][i];
+    });
 }
 
 }  // namespace
@@ -216,31 +300,94 @@ extern "C" int emu_row_pass(const uint64_t *in, uint64_t *out, uint64_t q, uint3
 }
 
 // Column passes: the kernels' input bounds (kColFpIn, kColIntIn, row products)
-template <class Ar>
+template <int B = 4, class Ar>
 static int col_run(const Limb &p, const Ar &ar, const u64 *in, u64 *out, bool forward) {
     // canonical residues enter an inverse as 2 units of 0.52 q (FP64)
     const int bound = forward ? (Ar::kFp ? 16 : 4) : (Ar::kFp ? 2 : 3);
     switch (ntt_n1(p.logn)) {
-        case 6: col_pass<6>(p, ar, in, out, forward, bound); return 0;
-        case 7: col_pass<7>(p, ar, in, out, forward, bound); return 0;
-        case 8: col_pass<8>(p, ar, in, out, forward, bound); return 0;
+        case 6: col_pass<6, B>(p, ar, in, out, forward, bound); return 0;
+        case 7: col_pass<7, B>(p, ar, in, out, forward, bound); return 0;
+        case 8: col_pass<8, B>(p, ar, in, out, forward, bound); return 0;
         default: return -1;
     }
 }
 
-// A whole transform by column and row tiles: forward canonical coefficients to
-// natural-order values, inverse back.
-extern "C" int emu_fused_ntt(const uint64_t *in, uint64_t *out, uint64_t q, uint32_t logn, int forward) {
+template <int TB, int B>
+static int fused_ntt(const uint64_t *in, uint64_t *out, uint64_t q, uint32_t logn, int forward) {
     if (logn < 13 || logn > 17 || q >= kLazyModulusBound) return -1;
     if (!host::negacyclic_root(q, 1ull << logn)) return -2;
     const Limb p(q, logn);
     std::vector<uint64_t> mid(1ull << logn);
     auto go = [&](const auto &ar) {
-        int rc = forward ? col_run(p, ar, in, mid.data(), true) : run(p, ar, in, mid.data(), false);
+        int rc = forward ? col_run<B>(p, ar, in, mid.data(), true) : run<TB>(p, ar, in, mid.data(), false);
         if (rc) return rc;
-        return forward ? run(p, ar, mid.data(), out, true) : col_run(p, ar, mid.data(), out, false);
+        return forward ? run<TB>(p, ar, mid.data(), out, true) : col_run<B>(p, ar, mid.data(), out, false);
     };
     return p.fp ? go(RowFp{(double)q, 1.0 / (double)q}) : go(RowInt{q});
+}
+
+// A whole transform by column and row tiles: forward canonical coefficients to
+// natural-order values, inverse back.
+extern "C" int emu_fused_ntt(const uint64_t *in, uint64_t *out, uint64_t q, uint32_t logn, int forward) {
+    return fused_ntt<12, 4>(in, out, q, logn, forward);
+}
+// The same by the tiles of small launches.
+extern "C" int emu_fused_ntt_halved(const uint64_t *in, uint64_t *out, uint64_t q, uint32_t logn, int forward) {
+    return fused_ntt<11, 3>(in, out, q, logn, forward);
+}
+
+// A transform of a single-pass degree at the kernels' largest input bounds.
+extern "C" int emu_small_ntt(const uint64_t *in, uint64_t *out, uint64_t q, uint32_t logn, int forward) {
+    if (logn < 10 || logn > 12 || q >= kLazyModulusBound) return -1;
+    if (!host::negacyclic_root(q, 1ull << logn)) return -2;
+    const Limb p(q, logn);
+    auto go = [&](const auto &ar, int bound) {
+        switch (logn) {
+            case 10: small_pass<10>(p, ar, in, out, forward, bound); break;
+            case 11: small_pass<11>(p, ar, in, out, forward, bound); break;
+            default: small_pass<12>(p, ar, in, out, forward, bound); break;
+        }
+        return 0;
+    };
+    return p.fp ? go(RowFp{(double)q, 1.0 / (double)q}, forward ? 16 : 2) : go(RowInt{q}, forward ? 4 : 3);
+}
+
+// sum_t c_t w_t mod q of a gadget block as the column pass and ModUp form it:
+// the FP64 remainder as an integer, or the integer one shifted by q.
+extern "C" int64_t emu_block_sum(int fp, const uint64_t *c, const uint64_t *w, int n, uint64_t q) {
+    auto go = [&](auto s) {
+        for (int t = 0; t < n; ++t) s.add(c[t] | kDigitBias, w[t], (double)w[t] / (double)q);
+        return s.value(q);
+    };
+    if (!fp) return (int64_t)go(BlockSum<false>{});
+    return (int64_t)u64_as_f64(go(BlockSum<true>{}));
+}
+
+// sum_j y_j w_j of a key product as the row kernels form it; *peak: the
+// largest sum met (FP64: its magnitude), before any reduction.
+extern "C" int64_t emu_key_sum(int fp, const int64_t *y, const uint64_t *w, int n, uint64_t q, uint64_t *peak) {
+    *peak = 0;
+    if (fp) {
+        const SumFp sum{(double)q, 1.0 / (double)q};
+        double s = 0;
+        for (int j = 0; j < n; ++j) {
+            sum.mac(s, f64_as_u64((double)y[j]), w[j]);
+            const uint64_t m = (uint64_t)__builtin_fabs(s);
+            *peak = m > *peak ? m : *peak;
+            if (SumFp::full(j) && j + 1 < n) s = sum.reduced(s);
+        }
+        return (int64_t)u64_as_f64(sum.total(s));
+    }
+    uint64_t br_hi, br_lo;
+    host::barrett(q, br_hi, br_lo);
+    const SumInt sum(q, br_hi, br_lo);
+    uint64_t s = 0;
+    for (int j = 0; j < n; ++j) {
+        sum.mac(s, (uint64_t)y[j], w[j]);
+        *peak = s > *peak ? s : *peak;
+        if (SumInt::full(j) && j + 1 < n) s = sum.reduced(s);
+    }
+    return (int64_t)sum.total(s);
 }
 
 // shoup_lazy3 at y w mod q: the residue it returns (before any reduction)

@@ -6,7 +6,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from conftest import rand_residues
+from conftest import O, P60, Q0, rand_residues
 
 pytestmark = pytest.mark.gpu
 
@@ -114,3 +114,25 @@ def test_moddown_of_large_jobs_in_launches_of_their_own(pkg, ctx):
         outs = [torch.empty_like(ct) for _ in exps]
         batch(outs)
         assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+
+@pytest.mark.parametrize("case", ["blocks_of_12", "basis_over_64"])
+def test_large_blocks_and_bases_match_oracle(pkg, ctx, case):
+    """Blocks of 10 to 12 limbs (13 terms where the first prime is split) and a
+    basis past the limb order's 64, by the fused passes."""
+    n = 1 << 13
+    blocks = [12, 11, 10] if case == "blocks_of_12" else [12] * 5 + [6]
+    L, K = sum(blocks), 8 if case == "blocks_of_12" else 4
+    q = Q0 + O.ntt_primes(40, n, L - 1)
+    qp = q + P60[:K] if K <= len(P60) else q + P60 + O.ntt_primes(59, 65536, K - len(P60))
+    assert len(qp) == L + K == len(set(qp))
+    rng = np.random.default_rng(L)
+    kb, ka = rand_residues(rng, qp, n, len(blocks)), rand_residues(rng, qp, n, len(blocks))
+    key = pkg.HybridKeySwitchKey(pkg.PreparedRnsNttPlan(ctx, qp, n), L, blocks, kb, ka)
+    ct = rand_residues(rng, q, n, 2).reshape(1, 2, L, n)
+    ct[0, 1, :, :64] = np.array(q, dtype=np.uint64)[:, None] - 1
+    ct[0, 1, :, 64:128] = np.array(q, dtype=np.uint64)[:, None] // 2
+    want = np.stack(O.hybrid_key_switch(O.RnsPlan(qp, n), L, blocks, ct[0, 0], ct[0, 1], kb, ka))
+    x = pkg.to_device(ct)
+    for mode, got in _by_mode(ctx, lambda: pkg.to_host(key.switch(x))).items():
+        assert (got[0] == want).all(), mode

@@ -12,20 +12,15 @@ namespace ck {
 #if defined(__HIP_DEVICE_COMPILE__)
 struct BlockExec {
     u32 threads;
-    // thread id handed to the phases; a caller that runs several passes in a
-    // loop can make it opaque per iteration so the
-    // compiler recomputes the index math instead of keeping it live
-    u32 tid = threadIdx.x;
     template <class F>
     __device__ __forceinline__ void run(F &&phase) {
-        phase(tid);
+        phase(threadIdx.x);
     }
     __device__ __forceinline__ void barrier() { __syncthreads(); }
 };
 #else
 struct BlockExec {
     u32 threads;
-    u32 tid = 0;  // unused on the host: run() walks every thread
     template <class F>
     void run(F &&phase) {
         for (u32 t = 0; t < threads; ++t) phase(t);

@@ -218,6 +218,15 @@ def _ptr(t, numel: int | None = None, dtype: str = "int64", name: str = "tensor"
     return t.data_ptr()
 
 
+def _ptrs(ts, numel: int, name: str) -> list:
+    """_ptr of each int64 tensor, for lists where the call itself counts (256
+    plaintexts: 100 us with _ptr, 59 us)."""
+    torch = _torch()
+    kind, dt = torch.Tensor, torch.int64
+    return [t.data_ptr() if isinstance(t, kind) and t.dtype is dt and t.is_cuda and t.is_contiguous()
+            and t.numel() >= numel else _ptr(t, numel, name=name) for t in ts]
+
+
 # --------------------------------------------------------------- parameters
 def find_ntt_primes(bits: int, degree: int, count: int, skip=()) -> list[int]:
     """find_ntt_prime_below_bits (ring/ntt_prime.rs:67) continued downward."""

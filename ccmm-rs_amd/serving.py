@@ -14,7 +14,7 @@ import operator
 from dataclasses import dataclass, field
 from typing import Optional
 
-from . import GaloisBatchEntry, NttBatchEntry, PreparedRnsNttPlan, _check, _p, _ptr, _sz, lib
+from . import GaloisBatchEntry, NttBatchEntry, PreparedRnsNttPlan, _check, _p, _ptr, _ptrs, _sz, lib
 
 OP_ROTATE, OP_MUL_PLAIN, OP_ADD, OP_RESCALE, OP_MUL_RELIN_RESCALE, OP_COPY, OP_MOD_SWITCH, OP_SUB = 1, 2, 3, 4, 5, 6, 7, 8
 OP_NTT, OP_INTT, OP_MAC_PLAIN = 9, 10, 11
@@ -446,6 +446,7 @@ class ProgramRunner:
     def _plan_ops(self):
         prog = self.prog
         self.planned = list(prog.ops), (prog.n_regs, prog.n_inputs, prog.out_reg)
+        self.mutable = any(type(op) is not tuple for op in prog.ops)
         self.limbs = prog.register_limbs(self.L)
         groups, self.rows = schedule(prog, self.L, self.spare)
         self.groups = merge_sums(groups)
@@ -457,8 +458,8 @@ class ProgramRunner:
         place is not taken for the same.  What an op refers to (a key's handle,
         a plaintext's address, the list of a mac_plain) is read on every run."""
         prog, (ops, shape) = self.prog, self.planned
-        return (len(ops) != len(prog.ops) or shape != (prog.n_regs, prog.n_inputs, prog.out_reg)
-                or not all(map(operator.is_, prog.ops, ops)) or any(type(op) is not tuple for op in ops))
+        return (self.mutable or len(ops) != len(prog.ops) or shape != (prog.n_regs, prog.n_inputs, prog.out_reg)
+                or not all(map(operator.is_, prog.ops, ops)))
 
     def _reg(self, i, limbs):
         return self.regs[i, : 2 * limbs * self.plan.degree]
@@ -509,8 +510,7 @@ class ProgramRunner:
                     if not ins or any(len(pts) != len(ins) for pts in lists):
                         raise ValueError("one plaintext per ciphertext, at least one term")
                     cts = (C.c_uint64 * len(ins))(*ins)
-                    pts = (C.c_uint64 * (len(ins) * len(lists)))(*[_ptr(t, la * n, name="pt")
-                                                                    for pts in lists for t in pts])
+                    pts = (C.c_uint64 * (len(ins) * len(lists)))(*[p for pts in lists for p in _ptrs(pts, la * n, "pt")])
                     _check(lib().ckks_multiply_plain_accumulate_ntt_batch(
                         plan.handle, C.cast(cts, _p), C.cast(pts, _p), len(ins), C.cast(outs, _p), len(outs), la))
             return accumulate

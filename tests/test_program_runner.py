@@ -61,6 +61,7 @@ def calls(monkeypatch):
     for module in (pkg, S):
         monkeypatch.setattr(module, "lib", lambda: c)
         monkeypatch.setattr(module, "_ptr", lambda t, numel=None, **kw: t.data_ptr())
+        monkeypatch.setattr(module, "_ptrs", lambda ts, numel, name: [t.data_ptr() for t in ts])
         monkeypatch.setattr(module, "_check", lambda rc: None)
     monkeypatch.setattr(torch, "empty", lambda shape, dtype, device: empty(shape, dtype=dtype))
     return c

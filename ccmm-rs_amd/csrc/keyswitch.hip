@@ -916,8 +916,11 @@ struct DownJob {
     u64 first;
 };
 
+// J: 1, or kKsJobs.  A lone job's launch carries an eighth of the arguments and
+// no search for its job.
+template <size_t J>
 struct DownArgs {
-    DownJob e[kKsJobs];
+    DownJob e[J];
     u32 count;
     const ModDownTable *md;  // null: no special primes
     const DevPrime *primes;  // key basis
@@ -938,14 +941,15 @@ static u32 down_parts(size_t blocks, size_t q_limbs) {
     return p;
 }
 
-template <int K>
-__global__ __launch_bounds__(kKsThreads) void k_moddown(DownArgs a) {
+template <int K, size_t J>
+__global__ __launch_bounds__(kKsThreads) void k_moddown(DownArgs<J> a) {
     const u32 b = xcd_contiguous_block(blockIdx.x, gridDim.x);
-    const u32 chunk = b / a.parts % a.chunks;
-    const u32 rest = b / a.parts / a.chunks;
-    const u32 part = b % a.parts, i0 = a.q_limbs * part / a.parts, i1 = a.q_limbs * (part + 1) / a.parts;
+    const u32 parts = K == 0 ? 1 : a.parts;
+    const u32 chunk = b / parts % a.chunks;
+    const u32 rest = b / parts / a.chunks;
+    const u32 part = b % parts, i0 = a.q_limbs * part / parts, i1 = a.q_limbs * (part + 1) / parts;
     const u32 comp = rest % 2;
-    const DownJob &e = a.e[job_of(a, rest / 2)];
+    const DownJob &e = a.e[J == 1 ? 0 : job_of(a, rest / 2)];
     const u32 ct = rest / 2 - (u32)e.first;
     const u64 N = (u64)1 << a.logn;
     const u64 n = (u64)chunk * kKsThreads + threadIdx.x;
@@ -1205,7 +1209,7 @@ __global__ __launch_bounds__(256) void k_modup_mfma(ModUpMfmaArgs args) {
 }
 
 struct ModDownMfmaArgs {
-    DownArgs base;
+    DownArgs<1> base;
     const BcPlan *plan;  // P digits -> Q limbs
 };
 
@@ -1215,7 +1219,7 @@ __global__ __launch_bounds__(256) void k_moddown_mfma(ModDownMfmaArgs args) {
     __shared__ __align__(16) signed char lds_a[kBcRows * KR];
     __shared__ int lds_e[4][64 * 33];
     __shared__ unsigned char lds_neg[kBcRows];
-    const DownArgs &a = args.base;
+    const DownArgs<1> &a = args.base;
     const DownJob &job = a.e[0];
     const BcPlan &bp = *args.plan;
     const ModDownTable &md = *a.md;
@@ -2090,20 +2094,12 @@ static int ks_by_shape(const KsJob *const *in, size_t count, const Launch &launc
     return CKKS_OK;
 }
 
-// 5. ModDown (or plain finalize) of the coefficient-domain accumulators of
-// jobs of one shape, with the pass-through adds
-static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
+template <size_t J>
+static int ks_moddown_launch(const KsJob *const *jobs, size_t count, hipStream_t s) {
     const ckks_ksk *k = jobs[0]->k;
     const u64 N = k->degree, B = k->limbs, D = k->dnum;
     const u32 chunks = (u32)(N / kKsThreads);
-    size_t least = jobs[0]->n_cts;
-    for (size_t i = 1; i < count; ++i) least = std::min(least, jobs[i]->n_cts);
-    if (count > 1 && (jobs[0]->mfma || !moddown_together(count, least * 2 * chunks))) {
-        for (size_t i = 0; i < count; ++i)
-            if (int rc = ks_moddown(jobs + i, 1, s)) return rc;
-        return CKKS_OK;
-    }
-    DownArgs da{};
+    DownArgs<J> da{};
     size_t n_cts = 0;
     for (size_t i = 0; i < count; ++i) {
         const KsJob &j = *jobs[i];
@@ -2122,28 +2118,45 @@ static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
     da.chunks = chunks;
     da.parts = jobs[0]->mfma || k->p_limbs == 0 ? 1 : down_parts(n_cts * 2 * chunks, k->q_limbs);
     dim3 g((u32)(n_cts * 2 * chunks * da.parts));
-    if (jobs[0]->mfma) {
-        ModDownMfmaArgs dm{da, k->d_bc + D};
-        dim3 gm((u32)(n_cts * 2 * (N / kBcRows)));
-        switch (k->p_limbs) {
+    if constexpr (J == 1) {
+        if (jobs[0]->mfma) {
+            ModDownMfmaArgs dm{da, k->d_bc + D};
+            dim3 gm((u32)(n_cts * 2 * (N / kBcRows)));
+            switch (k->p_limbs) {
 #define CK_MDM(KK) \
     case KK: hipLaunchKernelGGL(k_moddown_mfma<KK>, gm, dim3(256), 0, s, dm); break;
-            CK_MDM(1) CK_MDM(2) CK_MDM(3) CK_MDM(4) CK_MDM(5) CK_MDM(6) CK_MDM(7) CK_MDM(8)
+                CK_MDM(1) CK_MDM(2) CK_MDM(3) CK_MDM(4) CK_MDM(5) CK_MDM(6) CK_MDM(7) CK_MDM(8)
 #undef CK_MDM
-            default: return fail(CKKS_ERR_UNSUPPORTED, "too many special primes");
+                default: return fail(CKKS_ERR_UNSUPPORTED, "too many special primes");
+            }
+            CK_HIP(hipGetLastError());
+            return CKKS_OK;
         }
-        CK_HIP(hipGetLastError());
-        return CKKS_OK;
     }
     switch (k->p_limbs) {
 #define CK_MD(KK) \
-    case KK: hipLaunchKernelGGL(k_moddown<KK>, g, dim3(kKsThreads), 0, s, da); break;
+    case KK: hipLaunchKernelGGL((k_moddown<KK, J>), g, dim3(kKsThreads), 0, s, da); break;
         CK_MD(0) CK_MD(1) CK_MD(2) CK_MD(3) CK_MD(4) CK_MD(5) CK_MD(6) CK_MD(7) CK_MD(8)
 #undef CK_MD
         default: return fail(CKKS_ERR_UNSUPPORTED, "too many special primes");
     }
     CK_HIP(hipGetLastError());
     return CKKS_OK;
+}
+
+// 5. ModDown (or plain finalize) of the coefficient-domain accumulators of
+// jobs of one shape, with the pass-through adds
+static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
+    const u32 chunks = (u32)(jobs[0]->k->degree / kKsThreads);
+    size_t least = jobs[0]->n_cts;
+    for (size_t i = 1; i < count; ++i) least = std::min(least, jobs[i]->n_cts);
+    if (count > 1 && (jobs[0]->mfma || !moddown_together(count, least * 2 * chunks))) {
+        for (size_t i = 0; i < count; ++i)
+            if (int rc = ks_moddown(jobs + i, 1, s)) return rc;
+        return CKKS_OK;
+    }
+    if (count == 1) return ks_moddown_launch<1>(jobs, count, s);
+    return ks_moddown_launch<kKsJobs>(jobs, count, s);
 }
 
 static int ks_moddown(const KsJob &j, hipStream_t s) {
@@ -2748,7 +2761,7 @@ int ckks_mod_down(const ckks_rns_plan *qp_plan, size_t q_limbs, const uint64_t *
         it = mp->moddown.emplace(q_limbs, std::make_pair(dc, dm)).first;
     }
     const size_t N = qp_plan->degree;
-    DownArgs da{};
+    DownArgs<1> da{};
     da.count = 1;
     da.e[0].acc = in;
     da.e[0].out = out;
@@ -2765,7 +2778,7 @@ int ckks_mod_down(const ckks_rns_plan *qp_plan, size_t q_limbs, const uint64_t *
     const dim3 g((u32)(n_polys * da.chunks * da.parts));
     switch (K) {
 #define CK_MDS(KK) \
-    case KK: hipLaunchKernelGGL(k_moddown<KK>, g, dim3(kKsThreads), 0, ctx->stream, da); break;
+    case KK: hipLaunchKernelGGL((k_moddown<KK, 1>), g, dim3(kKsThreads), 0, ctx->stream, da); break;
         CK_MDS(1) CK_MDS(2) CK_MDS(3) CK_MDS(4) CK_MDS(5) CK_MDS(6) CK_MDS(7) CK_MDS(8)
 #undef CK_MDS
     }

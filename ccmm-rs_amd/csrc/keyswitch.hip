@@ -2149,8 +2149,12 @@ static int ks_moddown_launch(const KsJob *const *jobs, size_t count, hipStream_t
 static int ks_moddown(const KsJob *const *jobs, size_t count, hipStream_t s) {
     const u32 chunks = (u32)(jobs[0]->k->degree / kKsThreads);
     size_t least = jobs[0]->n_cts;
-    for (size_t i = 1; i < count; ++i) least = std::min(least, jobs[i]->n_cts);
-    if (count > 1 && (jobs[0]->mfma || !moddown_together(count, least * 2 * chunks))) {
+    bool permuted = true;
+    for (size_t i = 0; i < count; ++i) {
+        least = std::min(least, jobs[i]->n_cts);
+        permuted = permuted && jobs[i]->galois_kinv && !ks_mac_takes_b(*jobs[i]);
+    }
+    if (count > 1 && (jobs[0]->mfma || !moddown_together(count, least * 2 * chunks, permuted))) {
         for (size_t i = 0; i < count; ++i)
             if (int rc = ks_moddown(jobs + i, 1, s)) return rc;
         return CKKS_OK;

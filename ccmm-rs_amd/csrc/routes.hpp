@@ -63,11 +63,14 @@ inline size_t row_rotate_half_tiles(size_t dnum, unsigned n2) {
 }
 
 // ModDown of several jobs of one shape in one launch, or each in its own
-// (workgroups of the smallest job).  One launch saves the tails of small ones,
-// but spreads the XCDs over every job's accumulators.  In one / each its own, us:
-// four exponents at N = 2^16, 32 limbs, 4 ciphertexts (2048 workgroups) 1070 / 1185,
-// 16 ciphertexts (8192) 3980 / 3870; three at 12 limbs, 16 ciphertexts 1236 / 1178;
-// two at N = 2^17, 12 limbs, 8 ciphertexts (8192) 890 / 896.
-inline bool moddown_together(size_t jobs, size_t workgroups) { return jobs < 3 || workgroups < 8192; }
+// (workgroups of the smallest job).  One launch saves the tails of small ones.
+// Where the jobs add their permuted b components it spreads the XCDs over every
+// job's gathers, which large jobs feel.  In one / each its own, us: four exponents
+// at N = 2^16, 32 limbs, 4 ciphertexts (2048 workgroups) 1070 / 1185, 16 ciphertexts
+// (8192) 3980 / 3870, without b components 3617 / 3707; three at 12 limbs, 16
+// ciphertexts 1236 / 1178; two at N = 2^17, 12 limbs, 8 ciphertexts (8192) 890 / 896.
+inline bool moddown_together(size_t jobs, size_t workgroups, bool permuted) {
+    return jobs < 3 || workgroups < 8192 || !permuted;
+}
 
 }  // namespace ck

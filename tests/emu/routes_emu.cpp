@@ -10,5 +10,7 @@ size_t emu_limb_tiles(size_t limbs, size_t n_cts, unsigned logn) { return ck::li
 size_t emu_half_tiles(int rotate, size_t dnum, unsigned n2) {
     return rotate ? ck::row_rotate_half_tiles(dnum, n2) : ck::row_mac_half_tiles(n2);
 }
-int emu_moddown_together(size_t jobs, size_t workgroups) { return ck::moddown_together(jobs, workgroups); }
+int emu_moddown_together(size_t jobs, size_t workgroups, int permuted) {
+    return ck::moddown_together(jobs, workgroups, permuted != 0);
+}
 }

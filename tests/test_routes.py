@@ -21,7 +21,7 @@ def emu():
     lib.emu_limb_tiles.restype = C.c_size_t
     lib.emu_half_tiles.argtypes = [C.c_int, C.c_size_t, C.c_uint]
     lib.emu_half_tiles.restype = C.c_size_t
-    lib.emu_moddown_together.argtypes = [C.c_size_t, C.c_size_t]
+    lib.emu_moddown_together.argtypes = [C.c_size_t, C.c_size_t, C.c_int]
     return lib
 
 
@@ -63,10 +63,11 @@ def test_tile_sizes(emu, rotate, dnum, tiles, logn, whole, half):
     assert (tiles <= emu.emu_half_tiles(rotate, dnum, (logn + 1) // 2)) == (half < whole)
 
 
-# exponents, ciphertexts, log2 N, us in one launch, us in one launch each
-@pytest.mark.parametrize("jobs,cts,logn,together,apart", [
-    (4, 4, 16, 1071.4, 1186.0), (4, 16, 16, 3979.4, 3870.6), (3, 16, 16, 1236.4, 1178.4), (2, 8, 17, 889.8, 895.6),
-    (4, 4, 17, 2272.1, 2395.3), (3, 16, 17, 2599.8, 2478.8), (3, 8, 17, 1375.0, 1317.2),
+# exponents, ciphertexts, log2 N, whether b is added permuted, us in one launch, us in one launch each
+@pytest.mark.parametrize("jobs,cts,logn,permuted,together,apart", [
+    (4, 4, 16, 1, 1071.4, 1186.0), (4, 16, 16, 1, 3979.4, 3870.6), (3, 16, 16, 1, 1236.4, 1178.4),
+    (2, 8, 17, 1, 889.8, 895.6), (4, 4, 17, 1, 2272.1, 2395.3), (3, 16, 17, 1, 2599.8, 2478.8),
+    (3, 8, 17, 1, 1375.0, 1317.2), (4, 16, 16, 0, 3616.7, 3707.1), (3, 24, 16, 0, 1124.1, 1133.1),
 ])
-def test_moddown_launches(emu, jobs, cts, logn, together, apart):
-    assert emu.emu_moddown_together(jobs, cts * 2 << (logn - 8)) == (together < apart)
+def test_moddown_launches(emu, jobs, cts, logn, permuted, together, apart):
+    assert emu.emu_moddown_together(jobs, cts * 2 << (logn - 8), permuted) == (together < apart)

@@ -417,11 +417,14 @@ class ProgramRunner:
     rotations and transforms go out together, one library call for up to 16
     of them (schedule): a baby-step / giant-step request at N = 2^14 is 30
     rotations of one ciphertext, whose kernels each fill a third of the chip
-    one at a time (256 x 256, 8 limbs: 3.06 ms one by one, 0.75 ms).  Registers hold compact [2][limbs][N]
-    ciphertexts at their current level (as the server's).  The program's
+    one at a time (256 x 256, 8 limbs: 3.06 ms one by one, 0.53 ms).  Registers hold compact [2][limbs][N]
+    ciphertexts at their current level (as the server's); after a run the
+    output register and those the program reads before it writes them hold
+    their program-order values, the others whatever was last put there.  The program's
     keys must belong to the plan's context; each run switches that context
     to the runner's own (non-null, default-priority) stream and back, which
-    waits for the run.  The first run() sizes every library workspace, so
+    waits for the run.  The first run() sizes every library workspace and
+    builds the calls (1.7 ms where later runs take 0.53), so
     run() must precede capture(); nothing is allocated while capturing.  A
     program changed after a run is planned anew by the next one."""
 

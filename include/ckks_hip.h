@@ -334,7 +334,8 @@ int ckks_mod_down(const ckks_rns_plan *qp_plan, size_t q_limbs, const uint64_t *
  * coefficients [p][N] (device doubles, from the canonical embedding) times
  * scale, rounded half away from zero (f64::round), rem_euclid every limb ->
  * out [p][limb][N].  CKKS_ERR_INVALID if a rounded value reaches 2^63.
- * Synchronises the context stream (overflow check). */
+ * Synchronises the context stream (overflow check).  The first encode of a
+ * context allocates its pinned flag (about 45 us). */
 int ckks_encode_coefficients(const ckks_rns_plan *plan, const double *coeffs, double scale,
                              uint64_t *out, size_t n_polys, size_t n_limbs);
 
